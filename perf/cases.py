@@ -231,3 +231,57 @@ def tolerance(case):
     if case["net"] == "conv":
         return {"rel": 5e-5, "max": 4e-3}
     return {"rel": 6e-3, "max": 0.04} if case["net"] == "oidn_unet" else {"rel": 2e-4, "max": 8e-3}
+
+
+def exact(case, seed):
+    """The layers one after the other in binary64 with torch; every output value in the order `run` returns it."""
+    if case["entry"] == "stream":
+        return [_exact_frame(case, seed * STREAM_FRAMES + f) for f in range(STREAM_FRAMES)]
+    return _exact_frame(case, seed)
+
+
+def _exact_frame(case, seed):
+    model = _network(case)
+    t = {"input": _frame(case, seed).permute(2, 0, 1).double()}
+    ops = model.to_ops({"H": case["H"], "W": case["W"]})
+    last = {s: i for i, op in enumerate(ops) for s in ([op["src"]] if isinstance(op["src"], str) else op["src"])}
+    for i, op in enumerate(ops):
+        names = [op["src"]] if isinstance(op["src"], str) else op["src"]
+        x, kind = t[names[0]], op["op"]
+        if kind == "conv2d":
+            w = torch.from_numpy(np.asarray(op["weight"])).cuda().double()
+            b = torch.from_numpy(np.asarray(op["bias"])).cuda().double()
+            (sy, sx), (py, px) = op["stride"], op["padding"]
+            K, C, R, S = w.shape
+            xp = torch.nn.functional.pad(x, (px, px, py, py))
+            h, wd = (x.shape[1] + 2 * py - R) // sy + 1, (x.shape[2] + 2 * px - S) // sx + 1
+            y = b[:, None].expand(K, h * wd).contiguous()
+            for r in range(R):
+                for s in range(S):
+                    y.addmm_(w[:, :, r, s].contiguous(), xp[:, r:r + (h - 1) * sy + 1:sy, s:s + (wd - 1) * sx + 1:sx].reshape(C, h * wd))
+            y = y.view(K, h, wd)
+        elif kind == "activation":
+            # the slope is a binary16 number, and these networks apply it to binary16 values
+            y = x.clamp_min(0.0) if op["func"] == "relu" else torch.where(x > 0, x, x * float(np.float16(op["alpha"])))
+        elif kind == "pool":
+            n = x.reshape(x.shape[0], x.shape[1] // 2, 2, x.shape[2] // 2, 2)
+            y = n.amax(dim=(2, 4)) if op["func"] == "max" else n.mean(dim=(2, 4))
+        elif kind == "upsample":
+            y = x.repeat_interleave(op["factor"], 1).repeat_interleave(op["factor"], 2)
+        elif kind == "concat":
+            y = torch.cat([x, t[names[1]]])
+        elif kind == "pad":
+            y = torch.nn.functional.pad(x[None], (op["left"], op["right"], op["top"], op["bottom"]), mode="replicate")[0]
+        elif kind == "slice":
+            y = x[:, op["top"]:op["top"] + op["out_h"], op["left"]:op["left"] + op["out_w"]]
+        for s in set(names):
+            if last[s] == i:
+                del t[s]
+        t[op["dst"]] = y
+    y = t[model.outputs[0].name]
+    if case["layout"] == "HWC":
+        y = y.permute(1, 2, 0)
+    elif case["layout"] == "CHWC8":
+        y = y.reshape(-1, 8, *y.shape[1:]).permute(0, 2, 3, 1)
+    y = y.contiguous()
+    return y.reshape(-1) if case["entry"] == "device" else y.cpu().numpy()
