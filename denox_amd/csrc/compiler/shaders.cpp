@@ -1025,14 +1025,33 @@ public:
     k.define("CH", in.channels); k.define("KX", op.kernelX); k.define("KY", op.kernelY); k.define("VEC", vec);
     if (avg) k.define("AVG", 1);
     defineOutput(k, place);
-    const std::string entry = std::string(avg ? "pool_avg_c" : "pool_max_c") + std::to_string(in.channels) + "v" + std::to_string(vec) + place.suffix;
+    const std::string entry = std::string(avg ? "pool_avg_c" : "pool_max_c") + std::to_string(in.channels) + "v" + std::to_string(vec) + (padded ? "e" : "") + place.suffix;
     k.define("KERNEL_NAME", entry);
     auto d = impl.registerDispatch(k, entry, rowGrid(sym, out.width, chunksPerPixel(kernelChannels(place, in.channels), vec)), out.height, gridZ(place), WG_BANDWIDTH);
     d.addBinding(dnx::Access::ReadOnly, m.inputs[0]);
     bindOutput(d, sym, model, m, place);
     d.addPushConstant(in.width); d.addPushConstant(in.height);
-    d.setName(std::string(avg ? "avgpool" : "maxpool") + (place.view.valid ? "+concat" : "")); d.setOperation(avg ? "avgpool" : "maxpool"); d.setConfig("vec" + std::to_string(vec) + (place.planes ? "/chwc8" : ""));
+    if (padded) {
+      const Op &pad = model.ops()[m.ops[0]];
+      d.addPushConstant(pad.left); d.addPushConstant(pad.right); d.addPushConstant(pad.top); d.addPushConstant(pad.bottom);
+    }
+    d.setName(std::string(padded ? "pad+" : "") + (avg ? "avgpool" : "maxpool") + (place.view.valid ? "+concat" : "")); d.setOperation(std::string(padded ? "pad+" : "") + (avg ? "avgpool" : "maxpool")); d.setConfig("vec" + std::to_string(vec) + (place.planes ? "/chwc8" : ""));
     if (place.planes) impl.edge().config = "chwc8";
+  // a replicate pad in front of the pool is read through (clamped window coordinates), pixel-major tensors only
+  std::vector<Match> matchAll(const Model &model, const CompileOptions &opt) const override {
+    std::vector<Match> out = SingleOpShader::matchAll(model, opt);
+    if (!opt.features.enablePadFusion) return out;
+    for (size_t i = 0, n = out.size(); i < n; ++i) {
+      const int prod = model.tensors()[out[i].inputs[0]].producer;
+      if (!out[i].inputFormats.empty() || prod < 0 || model.ops()[prod].kind != OpKind::Pad || model.ops()[prod].padMode != PaddingMode::Replicate) continue;
+      Match v = out[i];
+      v.pattern = PAT_PADA;
+      v.ops.insert(v.ops.begin(), prod);
+      v.inputs = model.ops()[prod].inputs;
+      out.push_back(std::move(v));
+    }
+    return out;
+  }
     d.setMemoryReads(bytesOf(sym, in)); d.setMemoryWrites(bytesOf(sym, out)); d.setFlops(Sym::Const(0));
   }
 };
@@ -1042,8 +1061,10 @@ public:
   explicit BasicUpsampleShader(const hip::HipCompiler *c) : SingleOpShader(c, OpKind::Upsample) {}
   std::string name() const override { return "basic_upsample"; }
   void implement(OpImpl &impl, const Model &model, const Match &m, unsigned, SymGraph &sym, const CompileOptions &) const override {
-    const Op &op = model.ops()[m.ops[0]];
-    const TensorNode &in = model.tensors()[m.inputs[0]], &out = model.tensors()[m.output];
+    const Op &op = model.ops()[m.ops.back()];
+    if (padded) k.define("PAD", 1);
+    const bool padded = (m.pattern & PAT_PADA) != 0;
+    const TensorNode &src = model.tensors()[m.inputs[0]], &in = model.tensors()[op.inputs[0]], &out = model.tensors()[m.output];
     const Placement place = placementOf(model, m, in.channels);
     const unsigned vec = place.vec;
     auto k = m_compiler->read("upsample.hip");
@@ -1060,7 +1081,7 @@ public:
     d.addPushConstant(in.width); d.addPushConstant(in.height);
     d.setName(std::string("upsample") + (place.view.valid ? "+concat" : "")); d.setOperation("upsample"); d.setConfig("vec" + std::to_string(vec) + (flat ? "/rows" : "") + (place.planes ? "/chwc8" : ""));
     if (place.planes) impl.edge().config = "chwc8";
-    d.setMemoryReads(bytesOf(sym, in)); d.setMemoryWrites(bytesOf(sym, out)); d.setFlops(Sym::Const(0));
+    d.setMemoryReads(bytesOf(sym, src)); d.setMemoryWrites(bytesOf(sym, out)); d.setFlops(Sym::Const(0));
   }
 };
 
