@@ -1287,6 +1287,151 @@ std::vector<std::unique_ptr<IShader>> get_all_shaders(const hip::HipCompiler *c)
   s.push_back(std::make_unique<MemoryPadShader>(c));
   s.push_back(std::make_unique<MemorySliceShader>(c));
   return s;
+// A chain of at least two data-movement layers in one pass (kernels/gather.hip): a source seen through a 2x or larger nearest
+// upsample or a replicate pad, or a concat of two such sources, then an activation and a crop.  Each part obeys the feature
+// switch of the same fusion into a convolution; layers that a convolution can absorb are still offered there.  Pixel-major only.
+class GatherShader final : public IShader {
+public:
+  explicit GatherShader(const hip::HipCompiler *c) : m_compiler(c) {}
+  std::string name() const override { return "gather"; }
+
+  struct Source { std::vector<int> ops; int tensor; };
+  static std::vector<Source> sourcesOf(const Model &model, TensorHandle t, const CompileOptions &opt) {
+    std::vector<Source> out{{{}, t}};
+    const int prod = model.tensors()[t].producer;
+    if (prod < 0) return out;
+    const Op &p = model.ops()[prod];
+    if ((p.kind == OpKind::Upsample && opt.features.enableUpsampleFusion) || (p.kind == OpKind::Pad && p.padMode == PaddingMode::Replicate && opt.features.enablePadFusion))
+      out.push_back({{prod}, p.inputs[0]});
+    return out;
+  }
+
+  std::vector<Match> matchAll(const Model &model, const CompileOptions &opt) const override {
+    std::vector<Match> out;
+    const auto &ops = model.ops();
+    struct Front { std::vector<int> ops, inputs; };
+    for (size_t t = 0; t < model.tensors().size(); ++t) {
+      // everything that can produce tensor t without an intermediate tensor
+      std::vector<Front> fronts;
+      for (const Source &a : sourcesOf(model, static_cast<int>(t), opt)) fronts.push_back({a.ops, {a.tensor}});
+      const int prod = model.tensors()[t].producer;
+      if (prod >= 0 && ops[prod].kind == OpKind::Concat && opt.features.enableConcatConvFusion)
+        for (const Source &a : sourcesOf(model, ops[prod].inputs[0], opt))
+          for (const Source &b : sourcesOf(model, ops[prod].inputs[1], opt)) {
+            Front f{a.ops, {a.tensor, b.tensor}};
+            for (int o : b.ops) if (std::find(f.ops.begin(), f.ops.end(), o) == f.ops.end()) f.ops.push_back(o); // (one padded tensor may be both sources)
+            f.ops.push_back(prod);
+            fronts.push_back(std::move(f));
+          }
+      // ... and what may follow it: nothing, an activation, a crop, both
+      struct Tail { std::vector<int> ops; int output; };
+      std::vector<Tail> tails{{{}, static_cast<int>(t)}};
+      for (size_t i = 0; i < tails.size(); ++i) {
+        const Tail cur = tails[i];
+        if (!singleUse(model, cur.output)) continue;
+        const int c = model.tensors()[cur.output].consumers[0];
+        const bool act = ops[c].kind == OpKind::Activation && opt.features.enableConvReluFusion && cur.ops.empty();
+        const bool crop = ops[c].kind == OpKind::Slice && opt.features.enableSliceFusion && (cur.ops.empty() || ops[cur.ops.back()].kind == OpKind::Activation);
+        if (!act && !crop) continue;
+        Tail next = cur;
+        next.ops.push_back(c);
+        next.output = ops[c].output;
+        tails.push_back(std::move(next));
+      }
+      for (const Front &f : fronts)
+        for (const Tail &tl : tails) {
+          if (f.ops.size() + tl.ops.size() < 2) continue; // a single layer has a kernel of its own
+          // A concat that ends the chain is left to its producers: they store each source into its channel range (ConcatView)
+          // and nothing is copied, where this pass would read back a source that a dispatch has just written.
+          if (f.inputs.size() == 2 && tl.ops.empty()) continue;
+          Match m;
+          m.ops = f.ops;
+          m.ops.insert(m.ops.end(), tl.ops.begin(), tl.ops.end());
+          m.inputs = f.inputs;
+          m.output = tl.output;
+          out.push_back(std::move(m));
+        }
+    }
+    return out;
+  }
+
+  // Pixels per workgroup of the LDS form: at most one per thread and 16 KB of staged halves (copy_transform.hip's
+  // measurement), a multiple of 8; wider pixels than that leaves 8 of are not offered.
+  static unsigned pixelsPerGroup(unsigned total) { return std::min(256u, 16u * 1024u / (total * 2u) / 8u * 8u); }
+  static bool wholeVectors(const Model &model, const Match &m) {
+    return std::all_of(m.inputs.begin(), m.inputs.end(), [&](int t) { return model.tensors()[t].channels % 8 == 0; });
+  }
+  std::vector<unsigned> acceptMatch(const Model &model, const Match &m, const CompileOptions &) const override {
+    unsigned total = 0;
+    for (int t : m.inputs) total += model.tensors()[t].channels;
+    if (!wholeVectors(model, m) && pixelsPerGroup(total) < 8) return {};
+    return {0};
+  }
+
+  void implement(OpImpl &impl, const Model &model, const Match &m, unsigned, SymGraph &sym, const CompileOptions &) const override {
+    const TensorNode &out = model.tensors()[m.output];
+    const unsigned ca = model.tensors()[m.inputs[0]].channels, cb = m.inputs.size() > 1 ? model.tensors()[m.inputs[1]].channels : 0;
+    const unsigned vec = wholeVectors(model, m) ? 8 : 1, pq = pixelsPerGroup(ca + cb);
+    auto k = m_compiler->read("gather.hip");
+    k.define("CA", ca); k.define("CB", cb); k.define("VEC", vec);
+    if (vec == 1) k.define("PQ", pq);
+    const Op *act = nullptr, *crop = nullptr, *concat = nullptr;
+    for (int o : m.ops) {
+      const Op &op = model.ops()[o];
+      if (op.kind == OpKind::Activation) act = &op;
+      if (op.kind == OpKind::Slice) crop = &op;
+      if (op.kind == OpKind::Concat) concat = &op;
+    }
+    // what lies between source s and the concat (or, without one, the layers behind)
+    const Op *front[2] = {nullptr, nullptr};
+    for (size_t s = 0; s < m.inputs.size(); ++s) {
+      const int end = concat ? concat->inputs[s] : -1;
+      if (concat) front[s] = end == m.inputs[s] ? nullptr : &model.ops()[model.tensors()[end].producer];
+      else if (model.ops()[m.ops[0]].kind == OpKind::Upsample || model.ops()[m.ops[0]].kind == OpKind::Pad) front[s] = &model.ops()[m.ops[0]];
+    }
+    std::string nm, entry = "gather_c";
+    const unsigned ch[2] = {ca, cb};
+    for (size_t s = 0; s < m.inputs.size(); ++s) {
+      const bool up = front[s] && front[s]->kind == OpKind::Upsample, pad = front[s] && front[s]->kind == OpKind::Pad;
+      k.define(s ? "UPB" : "UPA", up ? front[s]->scale : 1u);
+      if (pad) k.define(s ? "PADB" : "PADA", 1);
+      entry += (s ? "_c" : "") + std::to_string(ch[s]) + (up ? "u" + std::to_string(front[s]->scale) : "") + (pad ? "e" : "");
+      if (front[s]) nm += up ? "upsample+" : "pad+";
+    }
+    k.define("ACT", act ? (act->func == ActivationFunction::ReLU ? 1 : 2) : 0);
+    if (act && act->func == ActivationFunction::LeakyReLU) k.define("ALPHA", fmtFloat(act->alpha));
+    if (concat) nm += "concat+";
+    if (act) { nm += act->func == ActivationFunction::ReLU ? "relu+" : "leaky_relu+"; entry += act->func == ActivationFunction::ReLU ? "_relu" : "_lrelu"; }
+    if (crop) { nm += "slice+"; entry += "_crop"; }
+    nm.pop_back();
+    entry += "v" + std::to_string(vec);
+    k.define("KERNEL_NAME", entry);
+    auto d = impl.registerDispatch(k, entry, vec == 8 ? rowGrid(sym, out.width, (ca + cb) / 8) : sym.cdiv(out.width, pq), out.height, Sym::Const(1), WG_BANDWIDTH);
+    Sym reads = Sym::Const(0);
+    for (int t : m.inputs) {
+      d.addBinding(dnx::Access::ReadOnly, t);
+      reads = sym.add(reads, bytesOf(sym, model.tensors()[t]));
+    }
+    d.addBinding(dnx::Access::WriteOnly, m.output);
+    d.addPushConstant(out.width);
+    d.addPushConstant(crop ? crop->left : Sym::Const(0)); d.addPushConstant(crop ? crop->top : Sym::Const(0));
+    for (size_t s = 0; s < 2; ++s) {
+      const TensorNode *n = s < m.inputs.size() ? &model.tensors()[m.inputs[s]] : nullptr;
+      const bool pad = n && front[s] && front[s]->kind == OpKind::Pad;
+      d.addPushConstant(n ? n->width : Sym::Const(0)); d.addPushConstant(n ? n->height : Sym::Const(0));
+      d.addPushConstant(pad ? front[s]->left : Sym::Const(0)); d.addPushConstant(pad ? front[s]->top : Sym::Const(0));
+    }
+    d.setName(nm); d.setOperation(nm); d.setConfig("vec" + std::to_string(vec) + (vec == 1 ? "/lds" : ""));
+    impl.edge().config = "vec" + std::to_string(vec);
+    d.setMemoryReads(reads); d.setMemoryWrites(bytesOf(sym, out));
+    d.setFlops(act ? sym.mul(sym.mul(out.width, out.height), static_cast<int64_t>(ca + cb)) : Sym::Const(0));
+  }
+
+private:
+  const hip::HipCompiler *m_compiler;
+};
+
 }
 
 } // namespace denox::compiler
+  s.push_back(std::make_unique<GatherShader>(c));
