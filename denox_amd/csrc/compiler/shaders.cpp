@@ -1015,28 +1015,6 @@ public:
   // also refuses PoolFunction::Avg (BasicPoolShader.cpp:170), which its model and ONNX importer accept
   // (frontend/onnx/details/ops/average_pool.cpp:154); the kernel here has an averaging mode, so such models compile.
   bool supports(const Op &op) const override { return op.kernelX == op.poolStrideX && op.kernelY == op.poolStrideY && op.poolPadX == 0 && op.poolPadY == 0; }
-  void implement(OpImpl &impl, const Model &model, const Match &m, unsigned, SymGraph &sym, const CompileOptions &) const override {
-    const Op &op = model.ops()[m.ops[0]];
-    const TensorNode &in = model.tensors()[m.inputs[0]], &out = model.tensors()[m.output];
-    const Placement place = placementOf(model, m, in.channels);
-    const unsigned vec = place.vec;
-    auto k = m_compiler->read("pool.hip");
-    const bool avg = op.poolFunc == PoolFunction::Avg;
-    k.define("CH", in.channels); k.define("KX", op.kernelX); k.define("KY", op.kernelY); k.define("VEC", vec);
-    if (avg) k.define("AVG", 1);
-    defineOutput(k, place);
-    const std::string entry = std::string(avg ? "pool_avg_c" : "pool_max_c") + std::to_string(in.channels) + "v" + std::to_string(vec) + (padded ? "e" : "") + place.suffix;
-    k.define("KERNEL_NAME", entry);
-    auto d = impl.registerDispatch(k, entry, rowGrid(sym, out.width, chunksPerPixel(kernelChannels(place, in.channels), vec)), out.height, gridZ(place), WG_BANDWIDTH);
-    d.addBinding(dnx::Access::ReadOnly, m.inputs[0]);
-    bindOutput(d, sym, model, m, place);
-    d.addPushConstant(in.width); d.addPushConstant(in.height);
-    if (padded) {
-      const Op &pad = model.ops()[m.ops[0]];
-      d.addPushConstant(pad.left); d.addPushConstant(pad.right); d.addPushConstant(pad.top); d.addPushConstant(pad.bottom);
-    }
-    d.setName(std::string(padded ? "pad+" : "") + (avg ? "avgpool" : "maxpool") + (place.view.valid ? "+concat" : "")); d.setOperation(std::string(padded ? "pad+" : "") + (avg ? "avgpool" : "maxpool")); d.setConfig("vec" + std::to_string(vec) + (place.planes ? "/chwc8" : ""));
-    if (place.planes) impl.edge().config = "chwc8";
   // a replicate pad in front of the pool is read through (clamped window coordinates), pixel-major tensors only
   std::vector<Match> matchAll(const Model &model, const CompileOptions &opt) const override {
     std::vector<Match> out = SingleOpShader::matchAll(model, opt);
@@ -1052,7 +1030,31 @@ public:
     }
     return out;
   }
-    d.setMemoryReads(bytesOf(sym, in)); d.setMemoryWrites(bytesOf(sym, out)); d.setFlops(Sym::Const(0));
+  void implement(OpImpl &impl, const Model &model, const Match &m, unsigned, SymGraph &sym, const CompileOptions &) const override {
+    const Op &op = model.ops()[m.ops.back()];
+    const bool padded = (m.pattern & PAT_PADA) != 0;
+    const TensorNode &src = model.tensors()[m.inputs[0]], &in = model.tensors()[op.inputs[0]], &out = model.tensors()[m.output];
+    const Placement place = placementOf(model, m, in.channels);
+    const unsigned vec = place.vec;
+    auto k = m_compiler->read("pool.hip");
+    const bool avg = op.poolFunc == PoolFunction::Avg;
+    k.define("CH", in.channels); k.define("KX", op.kernelX); k.define("KY", op.kernelY); k.define("VEC", vec);
+    if (avg) k.define("AVG", 1);
+    if (padded) k.define("PAD", 1);
+    defineOutput(k, place);
+    const std::string entry = std::string(avg ? "pool_avg_c" : "pool_max_c") + std::to_string(in.channels) + "v" + std::to_string(vec) + (padded ? "e" : "") + place.suffix;
+    k.define("KERNEL_NAME", entry);
+    auto d = impl.registerDispatch(k, entry, rowGrid(sym, out.width, chunksPerPixel(kernelChannels(place, in.channels), vec)), out.height, gridZ(place), WG_BANDWIDTH);
+    d.addBinding(dnx::Access::ReadOnly, m.inputs[0]);
+    bindOutput(d, sym, model, m, place);
+    d.addPushConstant(in.width); d.addPushConstant(in.height);
+    if (padded) {
+      const Op &pad = model.ops()[m.ops[0]];
+      d.addPushConstant(pad.left); d.addPushConstant(pad.right); d.addPushConstant(pad.top); d.addPushConstant(pad.bottom);
+    }
+    d.setName(std::string(padded ? "pad+" : "") + (avg ? "avgpool" : "maxpool") + (place.view.valid ? "+concat" : "")); d.setOperation(std::string(padded ? "pad+" : "") + (avg ? "avgpool" : "maxpool")); d.setConfig("vec" + std::to_string(vec) + (place.planes ? "/chwc8" : ""));
+    if (place.planes) impl.edge().config = "chwc8";
+    d.setMemoryReads(bytesOf(sym, src)); d.setMemoryWrites(bytesOf(sym, out)); d.setFlops(Sym::Const(0));
   }
 };
 
@@ -1061,10 +1063,8 @@ public:
   explicit BasicUpsampleShader(const hip::HipCompiler *c) : SingleOpShader(c, OpKind::Upsample) {}
   std::string name() const override { return "basic_upsample"; }
   void implement(OpImpl &impl, const Model &model, const Match &m, unsigned, SymGraph &sym, const CompileOptions &) const override {
-    const Op &op = model.ops()[m.ops.back()];
-    if (padded) k.define("PAD", 1);
-    const bool padded = (m.pattern & PAT_PADA) != 0;
-    const TensorNode &src = model.tensors()[m.inputs[0]], &in = model.tensors()[op.inputs[0]], &out = model.tensors()[m.output];
+    const Op &op = model.ops()[m.ops[0]];
+    const TensorNode &in = model.tensors()[m.inputs[0]], &out = model.tensors()[m.output];
     const Placement place = placementOf(model, m, in.channels);
     const unsigned vec = place.vec;
     auto k = m_compiler->read("upsample.hip");
@@ -1081,7 +1081,7 @@ public:
     d.addPushConstant(in.width); d.addPushConstant(in.height);
     d.setName(std::string("upsample") + (place.view.valid ? "+concat" : "")); d.setOperation("upsample"); d.setConfig("vec" + std::to_string(vec) + (flat ? "/rows" : "") + (place.planes ? "/chwc8" : ""));
     if (place.planes) impl.edge().config = "chwc8";
-    d.setMemoryReads(bytesOf(sym, src)); d.setMemoryWrites(bytesOf(sym, out)); d.setFlops(Sym::Const(0));
+    d.setMemoryReads(bytesOf(sym, in)); d.setMemoryWrites(bytesOf(sym, out)); d.setFlops(Sym::Const(0));
   }
 };
 
@@ -1267,26 +1267,6 @@ public:
   }
 };
 
-} // namespace
-
-std::vector<std::string> conv_config_names() {
-  std::vector<std::string> names;
-  for (const ConvConfig &c : kConvConfigs) names.push_back(c.name);
-  for (const PairConfig &c : kPairConfigs) names.push_back(c.name);
-  return names;
-}
-
-std::vector<std::unique_ptr<IShader>> get_all_shaders(const hip::HipCompiler *c) {
-  std::vector<std::unique_ptr<IShader>> s;
-  s.push_back(std::make_unique<ConvMfmaShader>(c));
-  s.push_back(std::make_unique<ConvPairShader>(c));
-  s.push_back(std::make_unique<BasicPoolShader>(c));
-  s.push_back(std::make_unique<BasicUpsampleShader>(c));
-  s.push_back(std::make_unique<CopyTransformShader>(c));
-  s.push_back(std::make_unique<BasicActivationShader>(c));
-  s.push_back(std::make_unique<MemoryPadShader>(c));
-  s.push_back(std::make_unique<MemorySliceShader>(c));
-  return s;
 // A chain of at least two data-movement layers in one pass (kernels/gather.hip): a source seen through a 2x or larger nearest
 // upsample or a replicate pad, or a concat of two such sources, then an activation and a crop.  Each part obeys the feature
 // switch of the same fusion into a convolution; layers that a convolution can absorb are still offered there.  Pixel-major only.
@@ -1431,7 +1411,27 @@ private:
   const hip::HipCompiler *m_compiler;
 };
 
+} // namespace
+
+std::vector<std::string> conv_config_names() {
+  std::vector<std::string> names;
+  for (const ConvConfig &c : kConvConfigs) names.push_back(c.name);
+  for (const PairConfig &c : kPairConfigs) names.push_back(c.name);
+  return names;
+}
+
+std::vector<std::unique_ptr<IShader>> get_all_shaders(const hip::HipCompiler *c) {
+  std::vector<std::unique_ptr<IShader>> s;
+  s.push_back(std::make_unique<ConvMfmaShader>(c));
+  s.push_back(std::make_unique<ConvPairShader>(c));
+  s.push_back(std::make_unique<BasicPoolShader>(c));
+  s.push_back(std::make_unique<BasicUpsampleShader>(c));
+  s.push_back(std::make_unique<CopyTransformShader>(c));
+  s.push_back(std::make_unique<BasicActivationShader>(c));
+  s.push_back(std::make_unique<MemoryPadShader>(c));
+  s.push_back(std::make_unique<MemorySliceShader>(c));
+  s.push_back(std::make_unique<GatherShader>(c));
+  return s;
 }
 
 } // namespace denox::compiler
-  s.push_back(std::make_unique<GatherShader>(c));
