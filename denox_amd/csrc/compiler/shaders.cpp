@@ -174,7 +174,7 @@ bool chooseKT(const ConvConfig &cfgIn, unsigned CA, unsigned CB, unsigned K, con
     const size_t lds = (cfg.resident ? static_cast<size_t>(taps * kb * blk) * (g.CPAD + 8) * 2u + 2u * static_cast<size_t>(haloPix) * ckp * 2u
                                      : (static_cast<size_t>(haloPix) * ckp + static_cast<size_t>(taps * kb * blk) * (cfg.ck + 8)) * 2u) +
                        static_cast<size_t>(kb * blk) * 4u + // + the staged bias (fp32)
-                       (cfg.ostage ? static_cast<size_t>(th * tw) * (kb * blk / 8 + 1) * 16u : 0u); // + the finished tile (one spare 16-byte slot per pixel)
+                       (cfg.ostage ? static_cast<size_t>(th * tw) * (kb * blk / 8 + 1) * 16u * (g.CPAD > cfg.ck ? 1u : 2u) : 0u); // + the finished tile (one spare 16-byte slot per pixel; two tiles where a tile is one step)
     if (lds > dev.maxComputeSharedMemory) continue;
     {
       // a thread stages at most 64 halo vectors per step (the kernels' bookkeeping is one bit per vector)
@@ -468,8 +468,8 @@ public:
         continue;
       }
       if (cfg.wideHalo && conv.strideX == 1 && conv.strideY == 1) continue;
-      if (cfg.ostage) { // whole 16-byte slots of a pixel-major result, at least two steps per tile
-        if ((m.pattern & (PAT_POOL | PAT_CROP)) || m.outputFormat || conv.K % 8 || (cpad + stepChannels(cfg, cpad) - 1) / stepChannels(cfg, cpad) < 2) continue; // (a shorter last step counts)
+      if (cfg.ostage) { // whole 16-byte slots of a pixel-major result
+        if ((m.pattern & (PAT_POOL | PAT_CROP)) || m.outputFormat || conv.K % 8) continue;
         if (m.outputVariant) {
           const ConcatView v = concatViewOf(model, m.output);
           if (!v.valid || v.pitch % 8 || v.channelOffset % 8) continue;

@@ -13,11 +13,14 @@
 //           PW further waves only stage halos, so that address arithmetic, load waits and LDS
 //           writes run beside the matrix work instead of in front of it (all waves of a
 //           workgroup meet at the step barrier, so inside one role nothing overlaps).
-//   OSTAGE  (with PW > 0, pixel-major result, at least two steps per tile) the finished tile goes to memory through
+//   OSTAGE  (with PW > 0, pixel-major result) the finished tile goes to memory through
 //           LDS: the computing waves leave it there as binary16, and the staging waves store it during the next tile's
 //           first step with consecutive lanes on consecutive 16 bytes -- whole pixels (KT channels), 1 KiB per store
 //           instruction, instead of 16 bytes per lane at a stride of one pixel.  The computing waves then never wait
-//           for memory at all.
+//           for memory at all.  With one step per tile (NCHUNK = 1: the layers with few input channels, whose time is their
+//           stores) a tile would be rewritten in the step that stores the one before, so the staged tile is doubled.
+//           At 1920 x 1080: 9 -> 64 channels 90 us with the best configuration that stores from its lanes, 53 so; 32 -> 64 91 and 78;
+//           no gain for 32 channels and fewer (16 -> 16 29 and 32).
 //
 // Workgroup b serves XCD b % 8 (workgroups are dealt round-robin to the 8 XCDs), and each
 // XCD walks its own contiguous band of tiles so that neighbouring halos meet in one L2.
@@ -38,9 +41,10 @@
 #define OSTAGE 0
 #endif
 #if OSTAGE
-static_assert(PW > 0 && MF == 32 && NCHUNK >= 2 && !POOL && !CROP && !LAYOUT_OUT && OVEC && OPITCH % 8 == 0 && KOUT % 8 == 0, "staged result: see above");
+static_assert(PW > 0 && MF == 32 && !POOL && !CROP && !LAYOUT_OUT && OVEC && OPITCH % 8 == 0 && KOUT % 8 == 0, "staged result: see above");
 #define SPP (KT / 8)                             // 16-byte slots of a pixel's KT channels
 #define OSLOTS (SPP + 1)                         // pitch of a pixel in the staged tile: odd, so that 16 consecutive pixels start in 16 different bank groups
+#define NOB (NCHUNK >= 2 ? 1 : 2)                // staged tiles: with one step per tile, the one being written and the one being stored
 #define NVO ((TH * TW * SPP + NSTAGE - 1) / NSTAGE) // slots per staging thread
 #endif
 
@@ -93,7 +97,7 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
   __shared__ __attribute__((aligned(16))) _Float16 sIn[2][HALO_ELEMS];
   __shared__ __attribute__((aligned(16))) bias_t sBias[KT];
 #if OSTAGE
-  __shared__ uint4v sOut[TH * TW * OSLOTS];
+  __shared__ uint4v sOut[NOB * TH * TW * OSLOTS];
 #endif
 #if CB == 0
   const _Float16 *B = nullptr;
@@ -279,7 +283,7 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
         const int p = i / SPP, sl = i - p * SPP; // pixel of the tile (row-major), slot of the pixel
         const int y = y0 + p / TW, x = x0 + p % TW;
         const bool ok = i < TH * TW * SPP && y < (int)CONV_OUT_H(pc) && x < (int)CONV_OUT_W(pc) && kt * KT + sl * 8 < KOUT;
-        const uint4v v = sOut[i < TH * TW * SPP ? p * OSLOTS + sl : 0];
+        const uint4v v = sOut[(n % NOB) * (TH * TW * OSLOTS) + (i < TH * TW * SPP ? p * OSLOTS + sl : 0)];
         const unsigned off = ((unsigned)(y * (int)CONV_OUT_W(pc) + x) * (unsigned)OPITCH + (unsigned)(kt * KT + sl * 8)) * 2u;
         __builtin_amdgcn_raw_buffer_store_b128(v, out, ok ? off : NO_STORE, 0, STORE_AUX);
       }
@@ -317,6 +321,9 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
     // ---- computing waves ----
     Acc acc;
     int cchunk = 0;
+#if OSTAGE
+    int half = 0; // which staged tile the current one goes to
+#endif
     for (int g = 0; g < steps; ++g) {
       DNX_SYNC();
       if (cchunk == 0)
@@ -333,7 +340,8 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
           for (int j = 0; j < RPW; ++j)
 #pragma unroll
             for (int e = 0; e < 2; ++e)
-              sOut[((wv * RPW + j) * TW + (lane & 31)) * OSLOTS + kb * 4 + (lane >> 5) * 2 + e] = __builtin_bit_cast(uint4v, pk.o[kb][j][e]);
+              sOut[half * (TH * TW * OSLOTS) + ((wv * RPW + j) * TW + (lane & 31)) * OSLOTS + kb * 4 + (lane >> 5) * 2 + e] = __builtin_bit_cast(uint4v, pk.o[kb][j][e]);
+        half = (half + 1) % NOB;
 #else
         store_tile(acc, out, tileY(tile), tileX(tile), kt, wv, lane, pc);
 #endif
