@@ -152,19 +152,25 @@ std::vector<size_t> minimum_cost_subgraph(const std::vector<bool> &isInput, cons
 std::vector<size_t> select_schedule(const Model &model, const SuperGraph &g, const std::vector<double> &edgeCost) {
   // Tensor t has four nodes, 4 t + 2 f + v: layout f (0 HWC, 1 CHWC8; SuperGraphEdge::outputFormat) and v = 1 for the tensor
   // as a channel range of its concat's output (SuperGraphEdge::outputVariant, HWC only).  Tensor handles are topologically
-  // ordered, and so are these.  Model inputs and outputs are HWC tensors of their own.
+  // ordered, and so are these.  Model inputs and outputs are tensors of their own, in HWC or, where they are marked
+  // (TensorNode::blockedInterface), in CHWC8.
+  // (The two layouts of a marked input change places: the other one is made from the one the caller gives.)
+  auto node = [&](int t, int f, int v) {
+    const TensorNode &n = model.tensors()[static_cast<size_t>(t)];
+    return 4 * t + 2 * (n.isInput && n.blockedInterface ? 1 - f : f) + v;
+  };
   std::vector<bool> isInput(4 * model.tensors().size(), false);
   for (size_t i = 0; i < model.tensors().size(); ++i) isInput[4 * i] = model.tensors()[i].isInput;
   std::vector<HyperEdge> edges;
   for (const auto &e : g.edges) {
     HyperEdge h;
     for (size_t i = 0; i < e.inputs.size(); ++i)
-      h.inputs.push_back(4 * e.inputs[i] + 2 * (e.inputFormats.empty() ? 0 : e.inputFormats[i]) + (e.inputVariants.empty() ? 0 : e.inputVariants[i]));
-    h.output = 4 * e.output + 2 * e.outputFormat + e.outputVariant;
+      h.inputs.push_back(node(e.inputs[i], e.inputFormats.empty() ? 0 : e.inputFormats[i], e.inputVariants.empty() ? 0 : e.inputVariants[i]));
+    h.output = node(e.output, e.outputFormat, e.outputVariant);
     edges.push_back(std::move(h));
   }
   std::vector<int> outputs;
-  for (TensorHandle o : model.outputs()) outputs.push_back(4 * o);
+  for (TensorHandle o : model.outputs()) outputs.push_back(node(o, model.tensors()[o].blockedInterface ? 1 : 0, 0));
   double total = 0.0;
   std::vector<size_t> chosen = minimum_cost_subgraph(isInput, edges, edgeCost, outputs, &total);
   if (total >= kInfiniteCost) fail(Status::Unsupported, "no kernel implements part of this graph (a layer has no matching shader)");
@@ -176,9 +182,10 @@ static dnx::ScalarSource src(Sym s, dnx::ScalarType t = dnx::ScalarType::I64) { 
 std::vector<uint8_t> compile(const Model &modelIn, const hip::HipCompiler &hipc, const Db *db, const CompileOptions &opt, CompileReport *report) {
   if (modelIn.outputs().empty()) fail(Status::InvalidArgument, "model has no outputs");
   Model model = modelIn; // the symbol graph grows while dispatches are built
+  markBlockedInterface(model, opt);
   SymGraph &sym = model.symGraph();
   const auto shaders = get_all_shaders(&hipc);
-  SuperGraph g = implement(model, sym, shaders, opt);
+  SuperGraph g = implement(model, sym, shaders, hipc, opt);
   const std::vector<int64_t> dp = assumed_symeval(model, sym, opt);
   std::vector<double> cost(g.edges.size());
   std::vector<bool> measured(g.edges.size());
@@ -268,54 +275,25 @@ std::vector<uint8_t> compile(const Model &modelIn, const hip::HipCompiler &hipc,
   };
 
   // ---- interface tensors and layout conversion ----
-  auto formatOf = [](const std::vector<InterfaceTensorDescriptor> &descs, const std::string &name, size_t index) {
-    for (const auto &d : descs) if (d.name == name) return d.format;
-    if (index < descs.size() && descs[index].name.empty()) return descs[index].format;
-    return dnx::TensorFormat::SSBO_HWC;
-  };
-  auto layoutId = [](dnx::TensorFormat f) -> int {
-    switch (f) {
-    case dnx::TensorFormat::SSBO_HWC: return 0;
-    case dnx::TensorFormat::SSBO_CHW: return 1;
-    case dnx::TensorFormat::SSBO_CHWC8: return 2;
-    default: fail(Status::Unsupported, "interface tensors must be SSBO_HWC, SSBO_CHW or SSBO_CHWC8");
-    }
-  };
   auto relayout = [&](TensorHandle t, dnx::TensorFormat from, dnx::TensorFormat to, bool external_is_source) -> uint32_t {
     // creates the externally visible tensor in its declared format plus the conversion dispatch
     const TensorNode &n = model.tensors()[t];
-    if ((from == dnx::TensorFormat::SSBO_CHWC8 || to == dnx::TensorFormat::SSBO_CHWC8) && n.channels % 8) fail(Status::InvalidArgument, "CHWC8 needs a channel count divisible by 8");
     SuperTensor ext = g.tensors[t];
     ext.format = external_is_source ? from : to;
     ext.name = n.name;
     g.tensors.push_back(ext);
     const uint32_t extId = static_cast<uint32_t>(g.tensors.size() - 1);
-    ComputeDispatch d;
-    d.kernel = hipc.read("relayout.hip");
-    d.kernel.define("CH", n.channels); d.kernel.define("SRC_LAYOUT", layoutId(from)); d.kernel.define("DST_LAYOUT", layoutId(to));
-    d.entryPoint = "relayout_c" + std::to_string(n.channels) + "_" + std::to_string(layoutId(from)) + "to" + std::to_string(layoutId(to));
-    d.kernel.define("KERNEL_NAME", d.entryPoint);
-    // HWC <-> CHWC8 moves one 16-byte vector per thread, every other pair one pixel per thread (see relayout.hip)
-    const bool blocky = from != dnx::TensorFormat::SSBO_CHW && to != dnx::TensorFormat::SSBO_CHW && n.channels % 8 == 0;
-    d.workgroupCountX = sym.cdiv(sym.mul(sym.mul(n.width, n.height), blocky ? static_cast<int64_t>(n.channels / 8) : 1), 256);
-    d.workgroupCountY = d.workgroupCountZ = Sym::Const(1);
-    d.workgroupSize[0] = 256;
-    TensorBinding in{0, 0, dnx::Access::ReadOnly, TensorId{external_is_source ? extId : static_cast<uint32_t>(t)}, BindingType::Input, false, Sym::Const(0)};
-    TensorBinding ob{0, 1, dnx::Access::WriteOnly, TensorId{external_is_source ? static_cast<uint32_t>(t) : extId}, BindingType::Output, false, Sym::Const(0)};
-    d.bindings = {in, ob};
-    d.pushConstants = {PushConstantDesc{n.width, dnx::ScalarType::U32}, PushConstantDesc{n.height, dnx::ScalarType::U32}};
-    d.info.name = "relayout"; d.info.operation = "relayout"; d.info.srcPath = "relayout.hip";
-    d.info.hasReads = d.info.hasWrites = d.info.hasFlops = true;
-    d.info.memoryReads = d.info.memoryWrites = g.tensors[t].byteSize;
-    d.info.flops = Sym::Const(0);
+    const uint32_t own = static_cast<uint32_t>(t);
+    const ComputeDispatch d = relayoutDispatch(hipc, sym, n, g.tensors[t].byteSize, from, to, external_is_source ? extId : own, external_is_source ? own : extId);
     emitDispatch(d);
     return place(extId);
   };
 
   for (size_t i = 0; i < model.inputs().size(); ++i) {
     const TensorHandle t = model.inputs()[i];
-    const dnx::TensorFormat f = formatOf(opt.inputDescriptors, model.tensors()[t].name, i);
+    const dnx::TensorFormat f = interfaceFormat(opt.inputDescriptors, model.tensors()[t].name, i);
     if (f == dnx::TensorFormat::SSBO_HWC) out.inputs.push_back(place(static_cast<uint32_t>(t)));
+    else if (model.tensors()[t].blockedInterface) out.inputs.push_back(place(static_cast<uint32_t>(t + g.modelTensorCount)));
     else out.inputs.push_back(relayout(t, f, dnx::TensorFormat::SSBO_HWC, true));
   }
 
@@ -376,8 +354,9 @@ std::vector<uint8_t> compile(const Model &modelIn, const hip::HipCompiler &hipc,
 
   for (size_t i = 0; i < model.outputs().size(); ++i) {
     const TensorHandle t = model.outputs()[i];
-    const dnx::TensorFormat f = formatOf(opt.outputDescriptors, model.tensors()[t].name, i);
+    const dnx::TensorFormat f = interfaceFormat(opt.outputDescriptors, model.tensors()[t].name, i);
     if (f == dnx::TensorFormat::SSBO_HWC) out.outputs.push_back(place(static_cast<uint32_t>(t)));
+    else if (model.tensors()[t].blockedInterface) out.outputs.push_back(place(static_cast<uint32_t>(t + g.modelTensorCount)));
     else out.outputs.push_back(relayout(t, dnx::TensorFormat::SSBO_HWC, f, false));
   }
 
@@ -410,9 +389,10 @@ std::vector<uint8_t> compile(const Model &modelIn, const hip::HipCompiler &hipc,
 
 size_t populate(Db &db, const Model &modelIn, const hip::HipCompiler &hipc, const CompileOptions &opt, bool compileKernels, unsigned shardIndex, unsigned shardCount) {
   Model model = modelIn;
+  markBlockedInterface(model, opt);
   SymGraph &sym = model.symGraph();
   const auto shaders = get_all_shaders(&hipc);
-  const SuperGraph g = implement(model, sym, shaders, opt);
+  const SuperGraph g = implement(model, sym, shaders, hipc, opt);
   const std::vector<int64_t> dp = assumed_symeval(model, sym, opt);
   size_t added = 0;
   for (const auto &edge : g.edges)

@@ -103,7 +103,58 @@ ConcatView concatViewOf(const Model &model, TensorHandle t) {
 
 void OpImpl::finish() { m_graph->edges.push_back(std::move(m_edge)); }
 
-SuperGraph implement(const Model &model, SymGraph &sym, const std::vector<std::unique_ptr<IShader>> &shaders, const CompileOptions &opt) {
+dnx::TensorFormat interfaceFormat(const std::vector<InterfaceTensorDescriptor> &descs, const std::string &name, size_t index) {
+  for (const auto &d : descs) if (d.name == name) return d.format;
+  if (index < descs.size() && descs[index].name.empty()) return descs[index].format;
+  return dnx::TensorFormat::SSBO_HWC;
+}
+
+void markBlockedInterface(Model &model, const CompileOptions &opt) {
+  if (!opt.features.enableBlockedLayout) return;
+  auto mark = [&](const std::vector<TensorHandle> &list, const std::vector<InterfaceTensorDescriptor> &descs) {
+    for (size_t i = 0; i < list.size(); ++i) {
+      const TensorNode &n = model.tensors()[static_cast<size_t>(list[i])];
+      if (interfaceFormat(descs, n.name, i) != dnx::TensorFormat::SSBO_CHWC8 || n.channels % 8 || (n.isInput && n.isOutput)) continue;
+      if (n.isOutput && !n.consumers.empty()) continue;
+      if (std::count(list.begin(), list.end(), list[i]) != 1) continue;
+      model.setBlockedInterface(list[i]);
+    }
+  };
+  mark(model.inputs(), opt.inputDescriptors);
+  mark(model.outputs(), opt.outputDescriptors);
+}
+
+ComputeDispatch relayoutDispatch(const hip::HipCompiler &hipc, SymGraph &sym, const TensorNode &n, Sym bytes, dnx::TensorFormat from, dnx::TensorFormat to, uint32_t src, uint32_t dst) {
+  auto layoutId = [](dnx::TensorFormat f) -> int {
+    switch (f) {
+    case dnx::TensorFormat::SSBO_HWC: return 0;
+    case dnx::TensorFormat::SSBO_CHW: return 1;
+    case dnx::TensorFormat::SSBO_CHWC8: return 2;
+    default: fail(Status::Unsupported, "interface tensors must be SSBO_HWC, SSBO_CHW or SSBO_CHWC8");
+    }
+  };
+  if ((from == dnx::TensorFormat::SSBO_CHWC8 || to == dnx::TensorFormat::SSBO_CHWC8) && n.channels % 8) fail(Status::InvalidArgument, "CHWC8 needs a channel count divisible by 8");
+  ComputeDispatch d;
+  d.kernel = hipc.read("relayout.hip");
+  d.kernel.define("CH", n.channels); d.kernel.define("SRC_LAYOUT", layoutId(from)); d.kernel.define("DST_LAYOUT", layoutId(to));
+  d.entryPoint = "relayout_c" + std::to_string(n.channels) + "_" + std::to_string(layoutId(from)) + "to" + std::to_string(layoutId(to));
+  d.kernel.define("KERNEL_NAME", d.entryPoint);
+  // HWC <-> CHWC8 moves one 16-byte vector per thread, every other pair one pixel per thread (see relayout.hip)
+  const bool blocky = from != dnx::TensorFormat::SSBO_CHW && to != dnx::TensorFormat::SSBO_CHW && n.channels % 8 == 0;
+  d.workgroupCountX = sym.cdiv(sym.mul(sym.mul(n.width, n.height), blocky ? static_cast<int64_t>(n.channels / 8) : 1), 256);
+  d.workgroupCountY = d.workgroupCountZ = Sym::Const(1);
+  d.workgroupSize[0] = 256;
+  d.bindings = {TensorBinding{0, 0, dnx::Access::ReadOnly, TensorId{src}, BindingType::Input, false, Sym::Const(0)},
+                TensorBinding{0, 1, dnx::Access::WriteOnly, TensorId{dst}, BindingType::Output, false, Sym::Const(0)}};
+  d.pushConstants = {PushConstantDesc{n.width, dnx::ScalarType::U32}, PushConstantDesc{n.height, dnx::ScalarType::U32}};
+  d.info.name = "relayout"; d.info.operation = "relayout"; d.info.srcPath = "relayout.hip";
+  d.info.hasReads = d.info.hasWrites = d.info.hasFlops = true;
+  d.info.memoryReads = d.info.memoryWrites = bytes;
+  d.info.flops = Sym::Const(0);
+  return d;
+}
+
+SuperGraph implement(const Model &model, SymGraph &sym, const std::vector<std::unique_ptr<IShader>> &shaders, const hip::HipCompiler &hipc, const CompileOptions &opt) {
   SuperGraph g;
   g.tensors.reserve(model.tensors().size() + 64);
   for (size_t i = 0; i < model.tensors().size(); ++i) {
@@ -155,6 +206,22 @@ SuperGraph implement(const Model &model, SymGraph &sym, const std::vector<std::u
         impl.finish();
       }
     }
+  }
+  // an interface tensor kept in CHWC8 may also be converted
+  for (size_t i = 0; i < N; ++i) {
+    const TensorNode &n = model.tensors()[i];
+    if (!n.blockedInterface) continue;
+    const uint32_t hwc = static_cast<uint32_t>(i), blocked = static_cast<uint32_t>(i + N);
+    SuperGraphEdge e;
+    e.inputs = {static_cast<int>(i)};
+    e.output = static_cast<int>(i);
+    e.shader = "relayout";
+    e.config = n.isInput ? "chwc8>hwc" : "hwc>chwc8";
+    e.inputFormats = {n.isInput ? 1 : 0};
+    e.outputFormat = n.isInput ? 0 : 1;
+    e.dispatches.push_back(n.isInput ? relayoutDispatch(hipc, sym, n, g.tensors[i].byteSize, dnx::TensorFormat::SSBO_CHWC8, dnx::TensorFormat::SSBO_HWC, blocked, hwc)
+                                     : relayoutDispatch(hipc, sym, n, g.tensors[i].byteSize, dnx::TensorFormat::SSBO_HWC, dnx::TensorFormat::SSBO_CHWC8, hwc, blocked));
+    g.edges.push_back(std::move(e));
   }
   return g;
 }

@@ -195,7 +195,16 @@ std::vector<std::unique_ptr<IShader>> get_all_shaders(const hip::HipCompiler *co
 // every name `CompileOptions::forceConvConfig` accepts: the convolution shaders' configuration tables
 std::vector<std::string> conv_config_names();
 
+// the layout the caller declared for the index-th interface tensor
+dnx::TensorFormat interfaceFormat(const std::vector<InterfaceTensorDescriptor> &descs, const std::string &name, size_t index);
+// Marks the interface tensors declared CHWC8 that kernels may read or write as they are: whole 8-channel groups, an input that
+// is no output, or an output that nothing reads and that is declared once.  The conversion to and from HWC then is one more
+// edge of the super graph; every other conversion stays a dispatch outside the selection.
+void markBlockedInterface(Model &model, const CompileOptions &opt);
+// the dispatch that converts tensor n from `src` in layout `from` to `dst` in layout `to` (super-graph tensor ids)
+ComputeDispatch relayoutDispatch(const hip::HipCompiler &hipc, SymGraph &sym, const TensorNode &n, Sym bytes, dnx::TensorFormat from, dnx::TensorFormat to, uint32_t src, uint32_t dst);
+
 // Build the super graph: every shader x match x configuration.
-SuperGraph implement(const Model &model, SymGraph &sym, const std::vector<std::unique_ptr<IShader>> &shaders, const CompileOptions &opt);
+SuperGraph implement(const Model &model, SymGraph &sym, const std::vector<std::unique_ptr<IShader>> &shaders, const hip::HipCompiler &hipc, const CompileOptions &opt);
 
 } // namespace denox::compiler

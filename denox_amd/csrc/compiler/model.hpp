@@ -28,6 +28,9 @@ struct TensorNode {
   int producer = -1;            // op index, -1 for inputs
   std::vector<int> consumers;   // op indices
   bool isInput = false, isOutput = false;
+  // an interface tensor the caller keeps in CHWC8 and that kernels may access in that layout directly
+  // (set on the compiler's copy of the model, see markBlockedInterface)
+  bool blockedInterface = false;
 };
 
 struct Op {
@@ -75,6 +78,7 @@ public:
   Sym requireValueOfName(const std::string &name); // creates a free variable when unknown
 
   const std::vector<TensorNode> &tensors() const { return m_tensors; }
+  void setBlockedInterface(TensorHandle t) { m_tensors[static_cast<size_t>(t)].blockedInterface = true; }
   const std::vector<Op> &ops() const { return m_ops; }
   const std::vector<TensorHandle> &inputs() const { return m_inputs; }
   const std::vector<TensorHandle> &outputs() const { return m_outputs; }

@@ -116,16 +116,16 @@ constexpr unsigned kNumConvConfigs = sizeof(kConvConfigs) / sizeof(kConvConfigs[
 // Configurations that are also offered with channel-block-major (CHWC8) sources and / or result: one or two of each kernel
 // family and matrix shape, so that the layout alternative adds half as many candidates again instead of three times as many.
 bool offeredBlocked(const ConvConfig &cfg) {
-  for (const char *n : {"w4r2k16", "w8r2k32", "w4r1kfn", "p16r2k16", "s8r2k16", "t8r2k32", "t16r1k32", "m4r2k32x1", "m8r2k32x2", "m4r2kfx1", "q8r2k32x2", "s12r1k16", "r4r2k16n", "c4r2k32n", "s8r2k32s"})
+  for (const char *n : {"w4r2k16", "w8r2k32", "w4r2k32n", "w4r1kfn", "m4r1kfx1n", "p16r2k16", "s8r2k16", "t8r2k32", "t16r1k32", "m4r2k32x1", "m8r2k32x2", "m4r2kfx1", "q8r2k32x2", "s12r1k16", "r4r2k16n", "c4r2k32n", "s8r2k32s"})
     if (std::strcmp(n, cfg.name) == 0) return true;
   return false;
 }
 
-// A tensor that can exist in the blocked layout: whole 8-channel groups, and not an interface tensor (those keep the layout
-// the caller declared; the conversion from and to it is a dispatch of its own).
+// A tensor that can exist in the blocked layout: whole 8-channel groups, and not an interface tensor in another layout (those
+// keep the layout the caller declared; the conversion from and to it is a dispatch of its own).
 bool canBeBlocked(const Model &model, TensorHandle t) {
   const TensorNode &n = model.tensors()[t];
-  return n.channels % 8 == 0 && !n.isInput && !n.isOutput;
+  return n.channels % 8 == 0 && ((!n.isInput && !n.isOutput) || n.blockedInterface);
 }
 
 enum ConvPatternBits : unsigned { PAT_CONCAT = 1, PAT_UPSAMPLE = 2, PAT_ACT = 4, PAT_POOL = 8, PAT_PADA = 16, PAT_PADB = 32, PAT_CROP = 64, PAT_ACT_FIRST = 128 };
@@ -1103,7 +1103,9 @@ public:
       // Block-major sources: the concat is its first source's planes followed by its second source's.  When each source
       // is read by this concat only, the two are placed behind one another inside the result and no dispatch is needed
       // (the reference's implicit concat: placement/placement.cpp:232-255, CopyTransformShader.cpp:198-237).
-      if (opt.features.enableImplicitConcat && opt.features.enableBlockedLayout && m.inputs[0] != m.inputs[1] && canBeBlocked(model, m.output) &&
+      // (Interface tensors have memory of their own.)
+      auto internal = [&](int t) { return !model.tensors()[t].isInput && !model.tensors()[t].isOutput; };
+      if (opt.features.enableImplicitConcat && opt.features.enableBlockedLayout && m.inputs[0] != m.inputs[1] && internal(m.inputs[0]) && internal(m.inputs[1]) && internal(m.output) && canBeBlocked(model, m.output) &&
           canBeBlocked(model, m.inputs[0]) && canBeBlocked(model, m.inputs[1]) && singleUse(model, m.inputs[0]) && singleUse(model, m.inputs[1])) {
         Match v = m;
         v.inputFormats = {1, 1};
