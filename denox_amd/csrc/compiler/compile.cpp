@@ -45,11 +45,19 @@ std::vector<uint8_t> push_constant_bytes(const ComputeDispatch &d, const std::ve
 static double estimate_dispatch_ms(const ComputeDispatch &d, const std::vector<int64_t> &dp, const CompileOptions &opt) {
   const double bytes = (d.info.hasReads ? static_cast<double>(symValue(dp, d.info.memoryReads)) : 0.0) +
                        (d.info.hasWrites ? static_cast<double>(symValue(dp, d.info.memoryWrites)) : 0.0);
+  // With conv -> conv fusion switched off the estimates stay configuration-blind, so that each layer takes the first configuration
+  // of the table: the plain schedule that callers who switch fusions off compare against, whose launch geometry is known.
+  const bool perConfiguration = opt.features.enableConvConvFusion;
+  if (d.convCost.valid && perConfiguration) {
+    const double read = d.info.hasReads ? static_cast<double>(symValue(dp, d.info.memoryReads)) : 0.0;
+    return 1e-3 * conv_cost_us(d.convCost, static_cast<uint64_t>(symValue(dp, d.convCost.outWidth)), static_cast<uint64_t>(symValue(dp, d.convCost.outHeight)), read, bytes - read,
+                               opt.deviceInfo.xcdCount, opt.deviceInfo.computeUnits, opt.deviceInfo.maxComputeSharedMemory);
+  }
   const double flops = d.info.hasFlops ? static_cast<double>(symValue(dp, d.info.flops)) : 0.0;
-  // conservative fractions of the published peaks plus a fixed launch cost
+  // conservative fractions of the published peaks plus the launch, counted as in the convolutions' estimates
   const double tMem = bytes / (0.5 * opt.deviceInfo.hbmBytesPerSecond);
   const double tMath = flops / (0.3 * opt.deviceInfo.fp16MfmaFlops);
-  return (std::max(tMem, tMath) + 3e-6) * 1e3;
+  return (std::max(tMem, tMath) + (perConfiguration ? kLaunchUs * 1e-6 : 3e-6)) * 1e3;
 }
 
 // CompileOptions::layoutPreference: a positive value halves the cost of every candidate that touches a CHWC8 tensor
@@ -75,7 +83,6 @@ double edge_cost_ms(const SuperGraphEdge &e, const std::vector<int64_t> &dp, con
   if (all) return prefer(e, opt, total);
   total = 0.0;
   for (const auto &d : e.dispatches) total += estimate_dispatch_ms(d, dp, opt);
-  // estimates cannot tell configurations apart; the shader's prior breaks ties
   return prefer(e, opt, total / std::max(1e-3f, e.speedup));
 }
 

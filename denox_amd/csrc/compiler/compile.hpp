@@ -30,7 +30,7 @@ struct CompileReport {
 std::vector<int64_t> assumed_symeval(const Model &model, const SymGraph &sym, const CompileOptions &opt);
 
 // Cost of one super-graph edge in milliseconds: measured latencies from the
-// database where every dispatch of the edge has one, else a roofline estimate.
+// database where every dispatch of the edge has one, else an estimate (conv_cost.hpp for convolutions, bytes over bandwidth otherwise).
 double edge_cost_ms(const SuperGraphEdge &e, const std::vector<int64_t> &dp, const Db *db, const CompileOptions &opt, bool *measured);
 
 // Minimum-cost sub-hypergraph (common/src/denox/algorithm/minimum_const_subgraph.hpp:45-49 of

@@ -1,0 +1,151 @@
+// Why an estimate per configuration: a bytes-and-FLOP bound is the same for every configuration of a layer, so a schedule
+// without a timing table used one configuration (the first of the table) for every layer.  On the 1920 x 1080 U-Net that
+// cost 690 us against 510 us with a measured table, at 251 x 187 180 against 94, with doubled widths at 1917 x 1077 2320 against 1640.
+//
+// The form is the kernels' own: what the busiest compute unit does -- matrix instructions, halo staging and its memory round
+// trips, weight slices, stores -- against what the whole launch moves through memory; the parts that overlap combine as the root of
+// their squares.  The constants are fitted (least squares on the logarithm, near-best candidates weighted up) to the
+// latencies of 53 000 candidate dispatches measured on one MI355X: every candidate of the U-Net at eight extents from
+// 180 x 108 to 3840 x 2160 and at two widths, of the small U-Net, and of 16 single convolutions (1 x 1 to 5 x 5, stride 1 and 2,
+// 3 to 256 channels) at five extents.  Typical error 15 percent; the candidate it picks is 3 percent slower than the best one
+// of its layer on the U-Net (1.3 at doubled width), 0.3 - 16 percent on the single layers.  A timing table, where there is one,
+// still decides.
+#include "conv_cost.hpp"
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+
+namespace denox::compiler {
+
+namespace {
+
+struct KernelFit {
+  float matrix;  // time of a computing wave's matrix instructions over their issue time at 2 GHz
+  float step;    // us per LDS step: the round trip of a halo load that nothing hides
+  float vector;  // us per 16-byte vector a staging thread moves in a step
+  float barrier; // us per step that nothing overlaps
+  float spill;   // growth of matrix and staging time once the registers a wave needs exceed 55 % of its share
+  float crowded; // ... and beyond 80 %
+};
+const KernelFit kFit[] = {
+    /* Streamed   */ {0.824f, 0.0337f, 0.0865f, 0.0209f, 0.441f, 0.08f},
+    /* Resident   */ {1.467f, 0.0965f, 0.1360f, 0.0246f, 0.924f, 3.06f},
+    /* Staged     */ {1.191f, 0.0288f, 0.0759f, 0.0096f, 0.539f, 5.74f},
+    /* StagedTile */ {1.373f, 0.0333f, 0.0806f, 0.0252f, 0.510f, 5.00f},
+    /* TwoPhase   */ {1.634f, 0.0598f, 0.2382f, 0.0203f, 3.940f, 3.29f},
+    /* Fold       */ {1.388f, 0.5124f, 0.1078f, 0.0299f, 0.000f, 0.00f},
+    /* FoldStaged */ {2.886f, 0.2374f, 0.0641f, 0.0286f, 0.000f, 0.00f},
+    /* Pair       */ {1.122f, 0.1087f, 0.0748f, 0.0273f, 0.000f, 0.00f},
+    /* PairStaged */ {1.296f, 0.4625f, 0.0629f, 0.0305f, 0.000f, 0.00f},
+};
+// what is left to the configuration itself, as a factor
+const struct { const char *name; float factor; } kFactor[] = {
+    {"c4r2k16m", 0.81f}, {"c4r2k16n", 0.85f}, {"c4r2k32n", 0.80f}, {"d4r2k64", 0.88f}, {"f4r1", 0.78f}, {"f4r2", 0.76f}, {"f8r1", 0.84f},
+    {"g4r1", 0.57f}, {"g4r1k32", 0.58f}, {"g4r1k32n", 0.54f}, {"g4r1n", 0.55f}, {"g4r1p", 0.52f}, {"h4r2", 0.57f}, {"h4r2k32n", 0.53f},
+    {"h4r2k32p", 0.53f}, {"h4r2n", 0.53f}, {"h4r2p", 0.51f}, {"m2r1k32x1n", 0.79f}, {"m4r1k32x2", 1.01f}, {"m4r1kfx1n", 1.01f}, {"m4r1kfx2", 1.24f},
+    {"m4r2k32x1", 1.01f}, {"m4r2k32x1n", 1.11f}, {"m4r2k32x2", 1.09f}, {"m4r2k32x2n", 1.18f}, {"m4r2k64x2", 1.11f}, {"m4r2kfx1", 1.14f},
+    {"m4r2kfx1n", 1.10f}, {"m4r4k32x1", 1.09f}, {"m8r2k32x2", 1.19f}, {"p16r1k16", 1.05f}, {"p16r1k32", 0.95f}, {"p16r2k16", 0.98f},
+    {"p4r1k32", 0.93f}, {"p4r1k32n", 0.84f}, {"p4r2k32", 0.96f}, {"p4r2k32n", 0.92f}, {"p4r4k16", 0.91f}, {"p4r4k32", 0.84f}, {"p8r1k16", 0.99f},
+    {"p8r1k32", 0.97f}, {"p8r2k16", 0.97f}, {"p8r2k32", 0.94f}, {"p8r2k32s", 0.87f}, {"p8r4k16", 1.02f}, {"q4r2k32x1n", 0.93f}, {"q4r2k32x2", 0.86f},
+    {"q8r1k32x2", 1.02f}, {"q8r2k32x1", 0.97f}, {"q8r2k32x2", 0.98f}, {"r4r1k16n", 0.87f}, {"r4r2k16", 0.89f}, {"r4r2k16n", 0.85f},
+    {"r4r2k32n", 0.85f}, {"r8r1k16n", 0.90f}, {"s12r1k16", 1.03f}, {"s8r2k16", 0.95f}, {"s8r2k16s", 0.99f}, {"s8r2k32s", 1.37f}, {"t16r1k16", 1.01f},
+    {"t16r1k32", 0.95f}, {"t16r2k16", 1.06f}, {"t4r2k32", 0.86f}, {"t8r1k16", 0.91f}, {"t8r2k16", 0.85f}, {"t8r2k32", 0.81f}, {"t8r4k16", 0.89f},
+    {"u16r1k32x2", 1.01f}, {"u4r2k32", 0.77f}, {"u8r2k32x2", 0.75f}, {"v4r2k16", 0.85f}, {"v4r2k64", 0.80f}, {"w2r1k16n", 0.82f}, {"w2r2k16n", 0.98f},
+    {"w2r2k32", 0.89f}, {"w2r2k32n", 0.86f}, {"w2r2kfn", 1.09f}, {"w4r1k16", 1.01f}, {"w4r1k32", 0.95f}, {"w4r1k32n", 1.03f}, {"w4r1kfm", 0.99f},
+    {"w4r1kfn", 1.00f}, {"w4r1khn", 1.04f}, {"w4r2k16", 1.25f}, {"w4r2k16s", 1.15f}, {"w4r2k32", 1.13f}, {"w4r2k32n", 1.19f}, {"w4r2k32s", 1.06f},
+    {"w4r2k64", 1.11f}, {"w4r2kfn", 1.22f}, {"w4r2khn", 1.36f}, {"w4r4k16", 1.41f}, {"w4r4k32", 1.24f}, {"w8r1k16", 1.25f}, {"w8r2k16", 1.40f},
+    {"w8r2k32", 1.30f}, {"x4r2k16", 1.33f}, {"x4r2k32", 1.07f}, {"x4r4k16", 1.22f}, {"x8r2k16", 1.12f}, {"y4r2k32", 0.81f}, {"z4r2k64", 0.82f},
+};
+
+float factorOf(const char *name) {
+  for (const auto &f : kFactor) if (std::strcmp(f.name, name) == 0) return f.factor;
+  return 1.2f; // a configuration without a measurement: behind those that have one
+}
+
+double cdiv(double a, double b) { return std::ceil(a / b); }
+
+} // namespace
+
+double conv_cost_us(const ConvCost &c, uint64_t outWidth, uint64_t outHeight, double bytesRead, double bytesWritten, unsigned xcds, unsigned cus, unsigned ldsBytes) {
+  const double ow = static_cast<double>(outWidth), oh = static_cast<double>(outHeight);
+  const KernelFit &f = kFit[static_cast<int>(c.kernel)];
+  const double W = c.waves, RPW = c.rpw, KT = c.KT, CK = c.ck, stagers = (c.pw ? c.pw : c.waves) * 64.0, wavesPerSimd = std::max(1.0, W / 4.0);
+  const bool pair = c.kernel == ConvKernel::Pair || c.kernel == ConvKernel::PairStaged, fold = c.kernel == ConvKernel::Fold || c.kernel == ConvKernel::FoldStaged;
+  // per compute unit: rounds of tiles, LDS steps, matrix cycles of a wave, LDS reads; per step: halo bytes; per launch: resident weights
+  double rounds, steps, cycles, ldsReads, halo, haloSteps, resident = 0, tileBytes, overfetch, weightStep = 0, over = 0, groups = 0, rereads = 1;
+  if (pair) {
+    const double cpad = cdiv(c.CA + c.CB, 16) * 16, ck = std::min(CK, cpad), chunks = cdiv(cpad, ck), rowsPerStep = W * RPW, strips = cdiv(ow, 30);
+    const double wanted = std::max(1.0, std::floor(cus / strips));
+    const double rows = cdiv(cdiv(oh, wanted) + 2, rowsPerStep) * rowsPerStep, segments = cdiv(oh, rows - 2); // as conv3x3_pair.hip cuts the image
+    rounds = (rows / rowsPerStep + 1) * cdiv(strips * segments, cus);
+    const double mfma = 9 * (cpad / 16) * RPW + (c.tapm ? RPW * 6 : RPW * 18);
+    steps = haloSteps = rounds * chunks;
+    halo = (rowsPerStep + 2) * 34 * ck * 2;
+    resident = 9 * 32 * cpad * 2;
+    tileBytes = rowsPerStep * 32 * 32 * 2;
+    overfetch = 34 * (rowsPerStep + 2) / (30 * rowsPerStep);
+    cycles = mfma * 32 * wavesPerSimd * rounds;
+    ldsReads = rounds * W * (mfma + 9 * (cpad / 16));
+  } else if (fold) {
+    const bool staged = c.kernel == ConvKernel::FoldStaged;
+    const double cap = cdiv(c.CA, 16) * 16, cbp = c.CB ? cdiv(c.CB, 16) * 16 : 0, rows = W / c.ksplit * RPW, kbw = KT / 32 / c.ksplit;
+    const double slices = cdiv(cdiv(c.K, 32) * 32, KT), classes = staged ? 2 : 4, cols = staged ? 2 : 1;
+    const double tiles = cdiv(cdiv(ow, 2), 32) * cdiv(cdiv(oh, 2), rows), walkers = std::max(1.0, std::floor(cus / (xcds * classes * slices))) * xcds;
+    rounds = cdiv(tiles, walkers);
+    const double mfma = (4 * cap / 16 + 9 * cbp / 16) * kbw * RPW * cols, stepsA = staged ? std::floor(cap / c.cka) : 1, perTile = stepsA + (c.CB ? 1 : 0);
+    steps = haloSteps = rounds * perTile;
+    halo = ((rows + 1) * 34 * cap + (2 * rows + 1) * 66 * cbp) * 2 / perTile;
+    resident = (4 * cols * cap + 9 * cbp) * KT * 2;
+    tileBytes = rows * 32 * cols * KT * 2;
+    overfetch = 1.15 * classes * slices;
+    cycles = mfma * 32 * wavesPerSimd * rounds;
+    ldsReads = rounds * W * mfma * (1 + 1 / RPW);
+  } else {
+    const double kstep = c.mf == 32 ? 16 : 32, cpad = cdiv(c.CA + c.CB, kstep) * kstep, chunks = cdiv(cpad, CK), taps = c.R * c.S, xb = c.mf == 32 ? 1 : c.xb;
+    const double tw = c.mf == 32 ? 32 : 16 * xb, th = W * RPW, kb = KT / c.mf, slices = cdiv(cdiv(c.K, c.mf) * c.mf, KT), tiles = cdiv(ow, tw) * cdiv(oh, th);
+    const double haloPix = ((th - 1) * c.SY + c.R) * ((tw - 1) * c.SX + c.S), mfma = cpad / kstep * taps * kb * RPW * xb;
+    const double shared = c.SY > 1 || c.R == 1 ? 1.0 : (RPW + c.R - 1) / (RPW * c.R); // pixel fragments reused across vertical taps
+    const double accRegs = c.mf == 32 ? kb * RPW * 16 : kb * RPW * xb * 4, haloRegs = 4 * cdiv(std::floor(haloPix * CK * 2 / 16), stagers);
+    const double fragRegs = c.swp ? 8 * kb * c.R + 8 * (RPW + 2) : 4 * kb + 4 * ((RPW - 1) * c.SY + c.R) * xb;
+    halo = haloPix * CK * 2;
+    tileBytes = th * tw * KT * 2;
+    overfetch = haloPix / (th * tw * c.SY * c.SX);
+    double regs;
+    if (c.kernel == ConvKernel::Streamed) {
+      const double weights = taps * KT * CK, lds = (haloPix * (c.hrot ? CK : CK + 8) + taps * KT * (CK + 8)) * 2 + KT * 4;
+      const double weightRegs = 4 * cdiv(std::floor(weights / 8), W * 64);
+      const double perWave = std::min(512.0, accRegs + haloRegs + weightRegs + 64), simdWaves = std::floor(512 / perWave) * 4;
+      const double resident_ = std::max(1.0, std::min({std::floor(ldsBytes / lds), std::floor(simdWaves / W), 8.0})); // workgroups of one compute unit at a time
+      rounds = cdiv(tiles * slices, cus);
+      groups = rounds;
+      rereads = 1 + 0.530 * (slices - 1); // every slice of output channels walks the image again
+      steps = chunks * cdiv(rounds, std::min(resident_, rounds));
+      haloSteps = chunks * rounds;
+      weightStep = weights * 2;
+      regs = accRegs + haloRegs + weightRegs + fragRegs;
+    } else {
+      rounds = cdiv(tiles, static_cast<double>(c.slots) * xcds);
+      rereads = 1 + 0.628 * (slices - 1);
+      steps = haloSteps = rounds * chunks;
+      resident = taps * KT * cpad * 2;
+      regs = std::max(accRegs + fragRegs, c.pw ? 2 * haloRegs : 0) + (c.pw ? 0 : 2 * haloRegs);
+    }
+    over = regs / std::min(256.0, 512.0 / cdiv(W + c.pw, 4));
+    cycles = mfma * (c.mf == 32 ? 32 : 16) * wavesPerSimd * rounds;
+    ldsReads = cpad / kstep * taps * (kb + RPW * xb * shared) * W * rounds;
+  }
+  const double spill = std::exp(f.spill * std::max(0.0, over - 0.55) + f.crowded * std::max(0.0, over - 0.8));
+  const double matrix = cycles / 2000.0 * f.matrix * (c.mf == 16 ? 1.325 : 1) * (c.swp ? 1.008 : 1) * spill;
+  const double lds = ldsReads * 0.556e-3;
+  const bool ragged = c.CA % 8 || c.CB % 8;
+  const double staging = steps * (f.step + halo / 16 / stagers * f.vector * (ragged ? 2.373 : 1)) * spill * (c.blockedIn ? 0.862 : 1);
+  const double weights = haloSteps * weightStep * 31.095e-6;
+  // 8-byte pieces where a 16-channel block has no partner; a block-major result leaves the lanes in longer runs
+  const double stores = rounds * tileBytes * 2.149e-5 * (c.blockedOut ? 0.659 : 1) * (c.ntStore ? 0.749 : 1) * (c.mf == 16 && (c.KT / 16) % 2 ? 3.851 : 1);
+  const double memory = (bytesRead * std::min(overfetch, 4.0) * rereads + bytesWritten) / 5.661e6;
+  const double moved = staging + weights + stores;
+  const double start = (resident > 0 ? 0.795 + resident * 1.064e-5 : 0) + (c.weightsInRegisters ? 1.154 : 0);
+  return kLaunchUs + start + factorOf(c.config) * (std::sqrt(matrix * matrix + memory * memory + moved * moved + lds * lds) + steps * f.barrier + groups * 0.0139);
+}
+
+} // namespace denox::compiler

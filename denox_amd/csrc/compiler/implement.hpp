@@ -13,6 +13,7 @@
 // A dispatch names a HIP kernel variant (source + definitions, identified by
 // its SHA-256) where the reference names a GLSL variant.
 #pragma once
+#include "conv_cost.hpp"
 #include "../common/dnx.hpp"
 #include "../hip/hip_compiler.hpp"
 #include "model.hpp"
@@ -56,6 +57,7 @@ struct ComputeDispatch {
   uint32_t workgroupSize[3] = {1, 1, 1};
   std::vector<TensorBinding> bindings;
   ComputeDispatchInfo info;
+  ConvCost convCost; // set by the convolution shaders: what the dispatch takes where no timing table has it
   // index of a push constant whose bit 0 selects a reversed tile walk, -1 if the kernel has none;
   // the compiler alternates it along the selected schedule (it is 0 in every table row)
   int traversalFlagIndex = -1;
@@ -132,6 +134,7 @@ public:
   void setSourcePath(const std::string &p) { self().info.srcPath = p; }
   void setMemoryReads(Sym s) { self().info.memoryReads = s; self().info.hasReads = true; }
   void setMemoryWrites(Sym s) { self().info.memoryWrites = s; self().info.hasWrites = true; }
+  void setConvCost(const ConvCost &c) { self().convCost = c; }
   void setFlops(Sym s) { self().info.flops = s; self().info.hasFlops = true; }
   // assigns binding numbers in class order Input < Output < Param < Read < Write
   // (ComputeDispatchBuilder.cpp:100-176 of the reference); all in descriptor set 0

@@ -630,6 +630,16 @@ public:
     d.setMemoryReads(reads);
     d.setMemoryWrites(bytesOf(sym, model.tensors()[m.output]));
     d.setFlops(sym.mul(sym.mul(OW, OH), static_cast<int64_t>(2) * conv.R * conv.S * conv.C * conv.K));
+    ConvCost cost;
+    cost.valid = true;
+    cost.kernel = cfg.fold ? (cfg.pw ? ConvKernel::FoldStaged : ConvKernel::Fold) : !cfg.resident ? ConvKernel::Streamed : cfg.ostage ? ConvKernel::StagedTile : cfg.pp ? ConvKernel::TwoPhase : cfg.pw ? ConvKernel::Staged : ConvKernel::Resident;
+    cost.config = cfg.name;
+    cost.waves = cfg.waves; cost.pw = cfg.pw; cost.rpw = cfg.rpw; cost.ck = cfg.fold ? 16u : stepChannels(cfg, g.CPAD); cost.mf = cfg.mf; cost.xb = cfg.xb; cost.KT = g.KT; cost.K = conv.K;
+    cost.CA = CA; cost.CB = CB; cost.R = conv.R; cost.S = conv.S; cost.SY = conv.strideY; cost.SX = conv.strideX; cost.slots = g.slots;
+    cost.cka = cfg.fold ? fg.cka : 0; cost.ksplit = cfg.ksplit; cost.hrot = cfg.hrot; cost.swp = cfg.swp; cost.ntStore = cfg.ntStore;
+    cost.blockedIn = blockedIn; cost.blockedOut = blockedOut;
+    cost.outWidth = OW; cost.outHeight = OH;
+    d.setConvCost(cost);
   }
 
 private:
@@ -907,6 +917,14 @@ public:
     d.setMemoryReads(reads);
     d.setMemoryWrites(bytesOf(sym, model.tensors()[m.output]));
     d.setFlops(sym.mul(sym.mul(convIn.width, convIn.height), static_cast<int64_t>(2) * 9 * (static_cast<int64_t>(first.C) * first.K + static_cast<int64_t>(second.C) * second.K)));
+    ConvCost cost;
+    cost.valid = true;
+    cost.kernel = cfg.pw ? ConvKernel::PairStaged : ConvKernel::Pair;
+    cost.config = cfg.name;
+    cost.waves = cfg.waves; cost.pw = cfg.pw; cost.rpw = cfg.rpw; cost.ck = g.ck; cost.KT = 32; cost.K = second.K; cost.CA = CA; cost.CB = CB; cost.slots = g.slots; cost.tapm = g.tapm; cost.weightsInRegisters = cfg.w1reg;
+    cost.blockedIn = blockedIn; cost.blockedOut = blockedOut;
+    cost.outWidth = convIn.width; cost.outHeight = convIn.height; // (both convolutions keep the extent)
+    d.setConvCost(cost);
   }
 
 private:

@@ -170,7 +170,7 @@ typedef struct denox_hip_compile_options {
                                         that path); 0: cost alone decides */
 } denox_hip_compile_options;
 void denox_hip_compile_options_default(denox_hip_compile_options *opt);
-/* db may be NULL (roofline estimates drive the selection).  The blob is
+/* db may be NULL (estimates per configuration drive the selection).  The blob is
  * malloc'ed; release it with denox_hip_free. */
 int denox_hip_compile(const denox_hip_builder *b, const denox_hip_compile_options *opt, const denox_hip_db *db,
                       void **out_dnx, size_t *out_size);
