@@ -139,9 +139,12 @@ ComputeDispatch relayoutDispatch(const hip::HipCompiler &hipc, SymGraph &sym, co
   d.kernel.define("CH", n.channels); d.kernel.define("SRC_LAYOUT", layoutId(from)); d.kernel.define("DST_LAYOUT", layoutId(to));
   d.entryPoint = "relayout_c" + std::to_string(n.channels) + "_" + std::to_string(layoutId(from)) + "to" + std::to_string(layoutId(to));
   d.kernel.define("KERNEL_NAME", d.entryPoint);
-  // HWC <-> CHWC8 moves one 16-byte vector per thread, every other pair one pixel per thread (see relayout.hip)
+  // HWC <-> CHWC8 moves one 16-byte vector per thread, HWC <-> CHW of whole 8-channel groups a tile of pixels per workgroup (MODE_BLOCK),
+  // every other pair one pixel per thread (see relayout.hip)
   const bool blocky = from != dnx::TensorFormat::SSBO_CHW && to != dnx::TensorFormat::SSBO_CHW && n.channels % 8 == 0;
-  d.workgroupCountX = sym.cdiv(sym.mul(sym.mul(n.width, n.height), blocky ? static_cast<int64_t>(n.channels / 8) : 1), 256);
+  const bool hwc = from == dnx::TensorFormat::SSBO_HWC || to == dnx::TensorFormat::SSBO_HWC, chw = from == dnx::TensorFormat::SSBO_CHW || to == dnx::TensorFormat::SSBO_CHW;
+  const int64_t tile = hwc && chw && n.channels % 8 == 0 && n.channels <= 256 ? (n.channels <= 32 ? 512 : n.channels <= 64 ? 256 : n.channels <= 128 ? 128 : 64) : 256;
+  d.workgroupCountX = sym.cdiv(sym.mul(sym.mul(n.width, n.height), blocky ? static_cast<int64_t>(n.channels / 8) : 1), tile);
   d.workgroupCountY = d.workgroupCountZ = Sym::Const(1);
   d.workgroupSize[0] = 256;
   d.bindings = {TensorBinding{0, 0, dnx::Access::ReadOnly, TensorId{src}, BindingType::Input, false, Sym::Const(0)},
