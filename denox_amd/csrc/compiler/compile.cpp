@@ -47,7 +47,9 @@ static double estimate_dispatch_ms(const ComputeDispatch &d, const std::vector<i
                        (d.info.hasWrites ? static_cast<double>(symValue(dp, d.info.memoryWrites)) : 0.0);
   // With conv -> conv fusion switched off the estimates stay configuration-blind, so that each layer takes the first configuration
   // of the table: the plain schedule that callers who switch fusions off compare against, whose launch geometry is known.
-  const bool perConfiguration = opt.features.enableConvConvFusion;
+  // So do they with a forced configuration, which is then taken wherever it exists (a forced conv -> conv kernel would
+  // otherwise lose to two single convolutions on extents it does not suit).
+  const bool perConfiguration = opt.features.enableConvConvFusion && opt.forceConvConfig.empty();
   if (d.convCost.valid && perConfiguration) {
     const double read = d.info.hasReads ? static_cast<double>(symValue(dp, d.info.memoryReads)) : 0.0;
     return 1e-3 * conv_cost_us(d.convCost, static_cast<uint64_t>(symValue(dp, d.convCost.outWidth)), static_cast<uint64_t>(symValue(dp, d.convCost.outHeight)), read, bytes - read,
