@@ -145,7 +145,11 @@ double conv_cost_us(const ConvCost &c, uint64_t outWidth, uint64_t outHeight, do
   const double memory = (bytesRead * std::min(overfetch, 4.0) * rereads + bytesWritten) / 5.661e6;
   const double moved = staging + weights + stores;
   const double start = (resident > 0 ? 0.795 + resident * 1.064e-5 : 0) + (c.weightsInRegisters ? 1.154 : 0);
-  return kLaunchUs + start + factorOf(c.config) * (std::sqrt(matrix * matrix + memory * memory + moved * moved + lds * lds) + steps * f.barrier + groups * 0.0139);
+  // Fewer than 8 channels are read in pieces, which the persistent kernels' long-lived loaders feel more than the streaming ones'
+  // (medians of measured over estimated time above 10 us: 1.3 and, with staging waves, 1.55 against 0.97).
+  const bool persistent = !pair && !fold && c.kernel != ConvKernel::Streamed;
+  const double few = persistent && c.CA < 8 ? (c.pw ? 1.55 : 1.3) : 1;
+  return kLaunchUs + start + few * factorOf(c.config) * (std::sqrt(matrix * matrix + memory * memory + moved * moved + lds * lds) + steps * f.barrier + groups * 0.0139);
 }
 
 } // namespace denox::compiler
