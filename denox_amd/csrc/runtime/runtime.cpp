@@ -573,16 +573,31 @@ void Instance::infer(const void *const *inputs, void *const *outputs) {
   if (!inputs || !outputs) fail(Status::InvalidArgument, "infer: null pointer array");
   m_model->context()->makeCurrent();
   hipStream_t s = m_model->context()->stream();
+  auto bytesOf = [&](uint32_t t) { return static_cast<uint64_t>(m.tensors[t].size.eval(m_sym)); };
+  std::vector<char> stageIn(m.inputs.size(), 0), stageOut(m.outputs.size(), 0);
+  uint64_t staged = 0;
+  for (size_t i = 0; i < m.inputs.size(); ++i)
+    if (inputs[i] && HostStaging::worthwhile(inputs[i], bytesOf(m.inputs[i]))) stageIn[i] = 1, staged += bytesOf(m.inputs[i]);
+  for (size_t i = 0; i < m.outputs.size(); ++i)
+    if (outputs[i] && HostStaging::worthwhile(outputs[i], bytesOf(m.outputs[i]))) stageOut[i] = 1, staged += bytesOf(m.outputs[i]);
+  std::unique_lock<std::mutex> stagingLock(m_model->context()->hostStagingMutex(), std::defer_lock);
+  HostStaging &staging = m_model->context()->hostStaging();
+  if (staged) {
+    stagingLock.lock();
+    staging.prepare(staged, s);
+  }
   for (size_t i = 0; i < m.inputs.size(); ++i) {
     if (!inputs[i]) fail(Status::InvalidArgument, "infer: null input pointer");
-    const uint64_t sz = static_cast<uint64_t>(m.tensors[m.inputs[i]].size.eval(m_sym));
-    hipCheck(hipMemcpyAsync(tensorPtr(m.inputs[i]), inputs[i], sz, hipMemcpyHostToDevice, s), "hipMemcpyAsync(input)");
+    const uint64_t sz = bytesOf(m.inputs[i]);
+    if (stageIn[i]) staging.upload(tensorPtr(m.inputs[i]), inputs[i], sz, s);
+    else hipCheck(hipMemcpyAsync(tensorPtr(m.inputs[i]), inputs[i], sz, hipMemcpyHostToDevice, s), "hipMemcpyAsync(input)");
   }
   inferDevice(nullptr, nullptr);
   for (size_t i = 0; i < m.outputs.size(); ++i) {
     if (!outputs[i]) fail(Status::InvalidArgument, "infer: null output pointer");
-    const uint64_t sz = static_cast<uint64_t>(m.tensors[m.outputs[i]].size.eval(m_sym));
-    hipCheck(hipMemcpyAsync(outputs[i], tensorPtr(m.outputs[i]), sz, hipMemcpyDeviceToHost, s), "hipMemcpyAsync(output)");
+    const uint64_t sz = bytesOf(m.outputs[i]);
+    if (stageOut[i]) staging.download(outputs[i], tensorPtr(m.outputs[i]), sz, s);
+    else hipCheck(hipMemcpyAsync(outputs[i], tensorPtr(m.outputs[i]), sz, hipMemcpyDeviceToHost, s), "hipMemcpyAsync(output)");
   }
   hipCheck(hipStreamSynchronize(s), "hipStreamSynchronize");
 }

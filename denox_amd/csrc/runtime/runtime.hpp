@@ -13,8 +13,10 @@
 // list captured once per Instance into a hipGraph.
 #pragma once
 #include "../common/dnx.hpp"
+#include "host_staging.hpp"
 #include <hip/hip_runtime_api.h>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -36,8 +38,15 @@ public:
   void *staticScratch() const { return m_staticScratch; }
   // recorded behind every call of the allocation-free entry point (created with the context: that call creates nothing)
   hipEvent_t staticScratchDone() const { return m_staticDone; }
+  // infer: page-locked memory for large pageable arrays, one for all instances of the context (allocating 50 MB takes 3 ms, which an
+  // instance's first call would pay each time).  A call holds the mutex while it uses it: calls of other threads on this
+  // context would wait for this one's work on the common stream anyway.
+  HostStaging &hostStaging() { return m_staging; }
+  std::mutex &hostStagingMutex() { return m_stagingMutex; }
 
 private:
+  HostStaging m_staging;
+  std::mutex m_stagingMutex;
   int m_device;
   hipStream_t m_stream = nullptr;
   hipDeviceProp_t m_props;
