@@ -14,7 +14,6 @@
 #include "implement.hpp"
 #include "../common/f16.hpp"
 #include <algorithm>
-#include <cmath>
 #include <cstring>
 #include <sstream>
 
@@ -285,28 +284,9 @@ bool chooseFold(const ConvConfig &cfg, unsigned CA, unsigned CB, unsigned K, con
   return false;
 }
 
-// The four folded taps of one (output channel, input channel, class): coinciding taps summed in fp32, then rounded to binary16 so
-// that their errors cancel: in falling order of magnitude, each value takes along what the one before lost (at most half a
-// unit of it, a unit of its own).  The four multiply neighbouring pixels, which are alike, so it is the error of their sum that
-// reaches the result: on the U-Net's decoder layers 2.4e-4 -> 1.2e-4 of the result with every tap rounded by itself and so.
-void foldTaps(const float (&sum)[4], uint16_t (&out)[4]) {
-  int order[4] = {0, 1, 2, 3};
-  std::stable_sort(order, order + 4, [&](int x, int y) { return std::fabs(sum[x]) > std::fabs(sum[y]); });
-  float carry = 0.0f;
-  for (int t : order) {
-    const float v = sum[t] + carry;
-    out[t] = f32_to_f16(v);
-    carry = v - f16_to_f32(out[t]);
-    if (!std::isfinite(carry)) { // weights beyond binary16: nothing to take along
-      out[t] = f32_to_f16(sum[t]);
-      carry = 0.0f;
-    }
-  }
-}
-
 // Folded weights: [class a*2+b][kt][A tap ty*2+tx][KT rows][CAP] [B tap r*3+s][KT rows][CBP].  Tap r of output row
 // parity a reads low-resolution row y + a - 1 + ty with ty = (r + 1) / 2 for a = 0 and r / 2 for a = 1 (columns alike);
-// coinciding taps are summed (foldTaps).
+// coinciding taps are summed in fp32 and rounded to binary16 once.
 std::vector<uint8_t> packFoldWeights(const Op &conv, const FoldGeometry &g) {
   const unsigned nkt = g.KOUTP / g.KT, C = g.CA + g.CB;
   std::vector<uint16_t> out(static_cast<size_t>(4) * g.KOUTP * (4 * g.CAP + 9 * g.CBP), 0);
@@ -315,18 +295,19 @@ std::vector<uint8_t> packFoldWeights(const Op &conv, const FoldGeometry &g) {
   for (unsigned cls = 0; cls < 4; ++cls) {
     const unsigned a = cls >> 1, b = cls & 1;
     for (unsigned kt = 0; kt < nkt; ++kt) {
-      for (unsigned row = 0; row < g.KT; ++row) {
-        const unsigned k = kt * g.KT + rowChannel(32, g.KT, row);
-        for (unsigned c = 0; k < g.K && c < g.CA; ++c) {
-          float sum[4] = {};
-          for (unsigned r = 0; r < 3; ++r)
-            for (unsigned s2 = 0; s2 < 3; ++s2) sum[tmap(a, r) * 2 + tmap(b, s2)] += f16_to_f32(conv.weights[((static_cast<size_t>(k) * C + c) * 3 + r) * 3 + s2]);
-          uint16_t taps[4];
-          foldTaps(sum, taps);
-          for (unsigned t = 0; t < 4; ++t) out[pos + (static_cast<size_t>(t) * g.KT + row) * g.CAP + c] = taps[t];
-        }
-      }
-      pos += static_cast<size_t>(4) * g.KT * g.CAP;
+      for (unsigned ty = 0; ty < 2; ++ty)
+        for (unsigned tx = 0; tx < 2; ++tx)
+          for (unsigned row = 0; row < g.KT; ++row) {
+            const unsigned k = kt * g.KT + rowChannel(32, g.KT, row);
+            for (unsigned c = 0; c < g.CAP; ++c, ++pos) {
+              if (k >= g.K || c >= g.CA) continue;
+              float sum = 0.0f;
+              for (unsigned r = 0; r < 3; ++r)
+                for (unsigned s2 = 0; s2 < 3; ++s2)
+                  if (tmap(a, r) == ty && tmap(b, s2) == tx) sum += f16_to_f32(conv.weights[((static_cast<size_t>(k) * C + c) * 3 + r) * 3 + s2]);
+              out[pos] = f32_to_f16(sum);
+            }
+          }
       for (unsigned tap = 0; tap < 9; ++tap)
         for (unsigned row = 0; row < g.KT; ++row) {
           const unsigned k = kt * g.KT + rowChannel(32, g.KT, row);

@@ -7,7 +7,8 @@ that a lane of the matrix instruction ends up with consecutive output channels -
 weight W[k][c][r][s] appears exactly once, at the position the layout assigns to it, everything else is zero, and the
 bias is the bias followed by zeros.  Checked on the bytes of compiled models (read with the FlatBuffers decoder of
 test_flatbuf.py), with the inverse of the layout restated here from its description, for both matrix shapes, streamed
-and resident weights, paired and unpaired 16-row blocks, and the two-convolution kernel's three parameter forms."""
+and resident weights, paired and unpaired 16-row blocks, and the two-convolution kernel's three parameter forms.  The upsample-folding kernels' weights are sums of
+coinciding taps; each is the binary16 value nearest to its sum."""
 import re
 
 import numpy as np
@@ -126,3 +127,39 @@ def test_conv_pair_parameter_blobs(K2):
                 else:
                     assert (packed[r, row] == 0).all()
         assert (seen == 1).all()
+
+
+@pytest.mark.parametrize("config,CA,CB,K", [("f8r1", 16, 9, 32), ("g4r1", 24, 9, 32), ("h4r2p", 64, 9, 64)])
+@pytest.mark.parametrize("pruned", [0.0, 0.7])
+def test_folded_taps_are_nearest_to_their_sums(config, CA, CB, K, pruned):
+    """[class a*2+b][channel tile][A tap ty*2+tx][weight row][channel], then the second source's nine taps.  Row tap r of output row parity
+    a reads low-resolution row y + a - 1 + ty, ty = (r + 1) // 2 for a = 0 and r // 2 for a = 1 (columns alike).  Every folded tap is
+    its own sum rounded once: at most half a unit in its last place away (a lone bright pixel meets one tap, nothing a neighbouring
+    tap does makes up for its error), a sum that binary16 holds as it is, a single weight as it is, and a tap without weights is zero (the
+    output must not depend on a pixel the network does not read)."""
+    rng = np.random.default_rng(CA + K)
+    w = he_weights(rng, K, CA + CB)
+    w[rng.random(w.shape) < pruned] = 0
+    m = dx.Model()
+    a, b = m.input("a", m.sym("W") // 2, m.sym("H") // 2, CA), m.input("b", "W", "H", CB)
+    m.output(m.relu(m.conv2d(m.concat(m.upsample(a), b), w, np.zeros(K, np.float16))))
+    blob = dx.compile_model(m, conv_config=config)
+    assert config in dx.last_compile_report()
+    defines, (filt, _) = parameters(blob, W=64, H=64)
+    kt, cap, cbp, koutp = int(defines["KT"]), -(-CA // 16) * 16, -(-CB // 16) * 16, -(-K // 32) * 32
+    assert filt.size == 4 * koutp * (4 * cap + 9 * cbp)
+    tmap = lambda parity, r: (r + 1) // 2 if parity == 0 else r // 2  # noqa: E731
+    pos = 0
+    for cls in range(4):
+        sums = np.zeros((K, CA, 4), np.float32)
+        for r in range(3):
+            for s in range(3):
+                sums[:, :, tmap(cls >> 1, r) * 2 + tmap(cls & 1, s)] += w[:, :CA, r, s].astype(np.float32)
+        for t in range(koutp // kt):
+            block = filt[pos:pos + 4 * kt * cap].view(np.float16).reshape(4, kt, cap)
+            pos += block.size + 9 * kt * cbp
+            rows = [t * kt + row_channel(32, kt, row) for row in range(kt)]
+            for tap in range(4):
+                got = np.stack([block[tap, i, :CA] for i, k in enumerate(rows) if k < K])
+                np.testing.assert_array_equal(got, sums[[k for k in rows if k < K], :, tap].astype(np.float16), f"class {cls} tap {tap}")
+    assert pos == filt.size
