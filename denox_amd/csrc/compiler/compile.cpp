@@ -69,6 +69,8 @@ static double prefer(const SuperGraphEdge &e, const CompileOptions &opt, double 
   return blocked ? 0.5 * cost : cost;
 }
 
+static constexpr double kUnmeasuredFoldMs = 1e9; // beyond any schedule without such a kernel
+
 double edge_cost_ms(const SuperGraphEdge &e, const std::vector<int64_t> &dp, const Db *db, const CompileOptions &opt, bool *measured) {
   double total = 0.0;
   bool all = db != nullptr;
@@ -84,7 +86,15 @@ double edge_cost_ms(const SuperGraphEdge &e, const std::vector<int64_t> &dp, con
   if (measured) *measured = all;
   if (all) return prefer(e, opt, total);
   total = 0.0;
-  for (const auto &d : e.dispatches) total += estimate_dispatch_ms(d, dp, opt);
+  for (const auto &d : e.dispatches) {
+    total += estimate_dispatch_ms(d, dp, opt);
+    // The upsample-folding kernels multiply sums of weights that are rounded to binary16 once more (the 1920 x 1080 U-Net's output is 1.34e-3
+    // from binary64 with them, 1.22e-3 without): callers take that on with a timing table or by name, an estimate does not
+    // decide it for them, although it costs them time (592 us; 517 with folded kernels).  Finite: a layer that nothing else
+    // implements still compiles.
+    const bool fold = d.convCost.valid && (d.convCost.kernel == ConvKernel::Fold || d.convCost.kernel == ConvKernel::FoldStaged);
+    if (fold && opt.forceConvConfig != d.convCost.config) total += kUnmeasuredFoldMs;
+  }
   return prefer(e, opt, total / std::max(1e-3f, e.speedup));
 }
 

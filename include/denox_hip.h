@@ -146,7 +146,8 @@ typedef struct denox_hip_compile_options {
   int32_t enable_slice_fusion;       /* conv stores only the cropped window */
   int32_t enable_alternating_traversal; /* consecutive conv dispatches walk their tiles in opposite directions (cache reuse) */
   int32_t enable_upsample_fold;      /* offer kernels that fold a fused 2x upsample into the weights: fewer multiplications, the
-                                        summed weights rounded to binary16 once more (no counterpart in the reference) */
+                                        summed weights rounded to binary16 once more (no counterpart in the reference).  Taken
+                                        where a timing table has measured them or force_conv_config names them, never on an estimate */
   int32_t enable_implicit_concat;    /* Features::enableImplicitConcat: a concat source whose only consumer is the concat may be
                                         written by its producer straight into the concat's output (no copy dispatch) */
   int32_t input_format;              /* DENOX_HIP_FORMAT_* of every model input  (0 = HWC) */
