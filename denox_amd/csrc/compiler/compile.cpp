@@ -45,12 +45,7 @@ std::vector<uint8_t> push_constant_bytes(const ComputeDispatch &d, const std::ve
 static double estimate_dispatch_ms(const ComputeDispatch &d, const std::vector<int64_t> &dp, const CompileOptions &opt) {
   const double bytes = (d.info.hasReads ? static_cast<double>(symValue(dp, d.info.memoryReads)) : 0.0) +
                        (d.info.hasWrites ? static_cast<double>(symValue(dp, d.info.memoryWrites)) : 0.0);
-  // With conv -> conv fusion switched off the estimates stay configuration-blind, so that each layer takes the first configuration
-  // of the table: the plain schedule that callers who switch fusions off compare against, whose launch geometry is known.
-  // So do they with a forced configuration, which is then taken wherever it exists (a forced conv -> conv kernel would
-  // otherwise lose to two single convolutions on extents it does not suit).
-  const bool perConfiguration = opt.features.enableConvConvFusion && opt.forceConvConfig.empty();
-  if (d.convCost.valid && perConfiguration) {
+  if (d.convCost.valid) {
     const double read = d.info.hasReads ? static_cast<double>(symValue(dp, d.info.memoryReads)) : 0.0;
     return 1e-3 * conv_cost_us(d.convCost, static_cast<uint64_t>(symValue(dp, d.convCost.outWidth)), static_cast<uint64_t>(symValue(dp, d.convCost.outHeight)), read, bytes - read,
                                opt.deviceInfo.xcdCount, opt.deviceInfo.computeUnits, opt.deviceInfo.maxComputeSharedMemory);
@@ -59,7 +54,7 @@ static double estimate_dispatch_ms(const ComputeDispatch &d, const std::vector<i
   // conservative fractions of the published peaks plus the launch, counted as in the convolutions' estimates
   const double tMem = bytes / (0.5 * opt.deviceInfo.hbmBytesPerSecond);
   const double tMath = flops / (0.3 * opt.deviceInfo.fp16MfmaFlops);
-  return (std::max(tMem, tMath) + (perConfiguration ? kLaunchUs * 1e-6 : 3e-6)) * 1e3;
+  return (std::max(tMem, tMath) + kLaunchUs * 1e-6) * 1e3;
 }
 
 // CompileOptions::layoutPreference: a positive value halves the cost of every candidate that touches a CHWC8 tensor
@@ -70,6 +65,9 @@ static double prefer(const SuperGraphEdge &e, const CompileOptions &opt, double 
 }
 
 static constexpr double kUnmeasuredFoldMs = 1e9; // beyond any schedule without such a kernel
+// A forced conv -> conv configuration is taken wherever it exists: single convolutions keep their choice beside it (a forced single one
+// is the only one offered), and on extents that do not suit it two of them may be estimated faster.
+static constexpr double kForcedPairFactor = 1e-3;
 
 double edge_cost_ms(const SuperGraphEdge &e, const std::vector<int64_t> &dp, const Db *db, const CompileOptions &opt, bool *measured) {
   double total = 0.0;
@@ -95,6 +93,10 @@ double edge_cost_ms(const SuperGraphEdge &e, const std::vector<int64_t> &dp, con
     const bool fold = d.convCost.valid && (d.convCost.kernel == ConvKernel::Fold || d.convCost.kernel == ConvKernel::FoldStaged);
     if (fold && opt.forceConvConfig != d.convCost.config) total += kUnmeasuredFoldMs;
   }
+  const bool forcedPair = !opt.forceConvConfig.empty() && std::any_of(e.dispatches.begin(), e.dispatches.end(), [&](const ComputeDispatch &d) {
+    return (d.convCost.kernel == ConvKernel::Pair || d.convCost.kernel == ConvKernel::PairStaged) && opt.forceConvConfig == d.convCost.config;
+  });
+  if (forcedPair) total *= kForcedPairFactor;
   return prefer(e, opt, total / std::max(1e-3f, e.speedup));
 }
 

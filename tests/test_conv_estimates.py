@@ -48,3 +48,33 @@ def test_a_table_or_a_name_takes_folded_weights(tmp_path):
         db.add_sample(i, 1_000.0 if folding([c.split("/")[0]]) else 10_000.0)
     dx.compile_model(model, db=db, **at)
     assert folding(configs())
+
+
+def single_convs(net, **kw):
+    """(configuration, estimated ms) of every single convolution of the schedule that compile_model selects without a table."""
+    dx.compile_model(networks.build(net)[0], assume={"H": 1080, "W": 1920}, **kw)
+    return [(line.split()[1].split("/")[0], float(line.split()[-2])) for line in dx.last_compile_report().splitlines()[1:] if line.startswith("conv3x3_mfma")]
+
+
+def test_estimates_per_configuration_whatever_is_fused():
+    """Switching the conv -> conv fusion off, or forcing one configuration of that kernel, says nothing about how the single
+    convolutions are estimated: the layers between keep the choice (and the time) they have by default."""
+    default = single_convs("oidn_unet")
+    assert len(set(c for c, _ in default)) >= 4
+    off = single_convs("oidn_unet", features=dict(conv_conv_fusion=False))
+    assert len(off) == 16 and len(set(c for c, _ in off)) >= 4 and [c for c, _ in off] != ["w4r2k16"] * 16
+    inner = lambda s: sum(ms for _, ms in s[-12:])  # noqa: E731
+    assert inner(off[2:14]) <= 1.02 * inner(default)  # (the pairs at the ends are two layers each)
+    forced = single_convs("oidn_unet", conv_config="x4r2k16")
+    assert "x4r2k16" in configs()
+    assert len(forced) == 12 and inner(forced) <= 1.02 * inner(default)
+
+
+@pytest.mark.parametrize("config", ["x4r2k16", "x8r2k16", "v4r2k64", "y4r2k32", "d4r2k64"])
+@pytest.mark.parametrize("H,W", [(16, 30), (64, 64), (300, 61), (1080, 1920)])
+def test_forced_pair_is_taken_on_any_extent(config, H, W):
+    rng = np.random.default_rng(0)
+    m = dx.Model()
+    m.output(m.conv2d(m.relu(m.conv2d(m.input("x", "W", "H", 64), he_weights(rng, 32, 64), np.zeros(32, np.float16))), he_weights(rng, 3, 32), np.zeros(3, np.float16)))
+    dx.compile_model(m, conv_config=config, assume={"H": H, "W": W})
+    assert configs() == [config]

@@ -60,7 +60,7 @@ def test_tiny_unet_schedule_and_geometry():
     m, _ = networks.build("tiny_unet")
     # by default the last two convolutions (16 channels between them, read by nobody else) are one dispatch
     assert _dispatch_names(dx.compile_model(m), H=128, W=128) == ["conv3x3+relu", "maxpool", "conv3x3+relu", "concat+upsample+conv3x3+relu+conv3x3"]
-    d = dx.describe(dx.compile_model(m, features=dict(conv_conv_fusion=False)), H=128, W=128)
+    d = dx.describe(dx.compile_model(m, conv_config="w4r2k16", features=dict(conv_conv_fusion=False)), H=128, W=128)  # (the geometry below is this configuration's)
     names = [x["name"] for x in d["dispatches"]]
     # e0 feeds both the pool and the skip, so the pool stays its own dispatch; upsample+concat fold into the conv
     assert names == ["conv3x3+relu", "maxpool", "conv3x3+relu", "concat+upsample+conv3x3+relu", "conv3x3"]
@@ -105,7 +105,8 @@ def test_oidn_unet_schedule_dispatch_geometry_covers_every_pixel():
         assert sum(x["flops"] for x in f["dispatches"]) == pytest.approx(523.9e9 * (Hp * Wp) / (1088 * 1920), rel=2e-3)
         for x in (f["dispatches"][0], f["dispatches"][-1]):  # persistent launches of one workgroup per compute unit
             assert x["workgroup_count"] == [256, 1, 1] and x["push_constants"][:2] == [Wp, Hp]
-        d = dx.describe(dx.compile_model(m, assume={"H": H, "W": W}, features=dict(conv_conv_fusion=False)), H=H, W=W)
+        # (the geometry below is that of 32-pixel tiles)
+        d = dx.describe(dx.compile_model(m, conv_config="w4r2k16", assume={"H": H, "W": W}, features=dict(conv_conv_fusion=False)), H=H, W=W)
         # pad and crop fold into the first / last conv: IN extent, then source extent + offsets or crop window
         assert d["dispatches"][0]["name"] == "pad+conv3x3+relu" and d["dispatches"][-1]["name"] == "conv3x3+slice"
         assert d["dispatches"][0]["push_constants"] == [Wp, Hp, W, H, 0, 0, 0]
@@ -269,7 +270,7 @@ def test_concat_of_concats_without_dispatches_shares_one_buffer(widths, features
     outermost result, at the sum of the offsets along the chain, not inside a buffer that the inner result has left."""
     m, leaves, out = _nested_concat_model(widths)
     H = W = 32
-    d = dx.describe(dx.compile_model(m, features=dict(features, conv_conv_fusion=False)), H=H, W=W)
+    d = dx.describe(dx.compile_model(m, conv_config="w4r2k16", features=dict(features, conv_conv_fusion=False)), H=H, W=W)
     names = [x["debug_info"].split(" | ")[0] for x in d["dispatches"]]
     if any("concat" in x["name"] for x in d["dispatches"]):
         pytest.skip(f"this selection copies: {names}")
