@@ -47,7 +47,9 @@ static double estimate_dispatch_ms(const ComputeDispatch &d, const std::vector<i
                        (d.info.hasWrites ? static_cast<double>(symValue(dp, d.info.memoryWrites)) : 0.0);
   if (d.convCost.valid) {
     const double read = d.info.hasReads ? static_cast<double>(symValue(dp, d.info.memoryReads)) : 0.0;
-    return 1e-3 * conv_cost_us(d.convCost, static_cast<uint64_t>(symValue(dp, d.convCost.outWidth)), static_cast<uint64_t>(symValue(dp, d.convCost.outHeight)), read, bytes - read,
+    // (an assumed extent may leave a layer nothing to compute; that is no reason to refuse the model)
+    auto extent = [&](Sym s) { return static_cast<uint64_t>(std::max<int64_t>(1, symValue(dp, s))); };
+    return 1e-3 * conv_cost_us(d.convCost, extent(d.convCost.outWidth), extent(d.convCost.outHeight), read, bytes - read,
                                opt.deviceInfo.xcdCount, opt.deviceInfo.computeUnits, opt.deviceInfo.maxComputeSharedMemory);
   }
   const double flops = d.info.hasFlops ? static_cast<double>(symValue(dp, d.info.flops)) : 0.0;

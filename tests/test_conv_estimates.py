@@ -78,3 +78,16 @@ def test_forced_pair_is_taken_on_any_extent(config, H, W):
     m.output(m.conv2d(m.relu(m.conv2d(m.input("x", "W", "H", 64), he_weights(rng, 32, 64), np.zeros(32, np.float16))), he_weights(rng, 3, 32), np.zeros(3, np.float16)))
     dx.compile_model(m, conv_config=config, assume={"H": H, "W": W})
     assert configs() == [config]
+
+
+@pytest.mark.parametrize("C,K,config", [(16, 32, None), (64, 64, None), (256, 256, None), (512, 512, None), (64, 64, "w4r2k16"), (32, 32, "x4r2k16")])
+@pytest.mark.parametrize("assume", [{"W": 1, "H": 1}, {"W": 2, "H": 1}, {"W": 0, "H": 64}, {"W": 100_000, "H": 100_000}])
+def test_any_assumed_extent_compiles(C, K, config, assume):
+    """The assumption guides an estimate and is no limit of the model: one at which a layer has nothing to compute (a pooled image of one
+    row, a filter larger than the image) still compiles, as does one beyond any memory."""
+    rng = np.random.default_rng(0)
+    m = dx.Model()
+    t = m.conv2d(m.relu(m.conv2d(m.pool(m.input("x", "W", "H", C)), he_weights(rng, K, C), np.zeros(K, np.float16))), he_weights(rng, K, K), np.zeros(K, np.float16))
+    m.output(m.conv2d(t, he_weights(rng, K, K), np.zeros(K, np.float16), padding=(0, 0)))
+    dx.compile_model(m, conv_config=config, assume=assume)
+    assert "nan" not in dx.last_compile_report().lower()
