@@ -13,33 +13,35 @@ namespace denox::runtime {
 
 namespace {
 
-constexpr uint64_t kChunk = 2ull << 20;    // one link transfer: ~40 us, against ~10 us to enqueue it
-constexpr uint64_t kMaxBytes = 64ull << 20; // page-locked memory of one context; larger arrays go through it in batches
 constexpr uint64_t kWorthwhile = 4ull << 20; // below, starting the threads costs what they save
-constexpr unsigned kThreads = 8;           // 37 MB: 1.35 ms with one thread, 0.50 with four, 0.38 with eight, no less with twelve
+constexpr unsigned kThreads = 8;             // 37 MB: 1.35 ms with one thread, 0.50 with four, 0.38 with eight, no less with twelve
 
-// Threads that take chunk indices in order; `copy(i)` runs for each exactly once.  gate: chunks [0, gate) may be taken.
+constexpr uint64_t kChunk = HostStaging::kChunk;
+constexpr uint64_t kPiece = 128ull << 10; // what a thread copies at a time: all of them share a chunk, so that the first one is soon on the link
+
+// Threads that copy an array piece by piece, in order; `copy(offset, bytes)` runs for each piece exactly once.
+// gate: the chunks [0, gate) may be copied (none at first).
 class Copiers {
 public:
-  Copiers(uint64_t chunks, uint64_t gate, std::function<void(uint64_t)> copy) : m_copy(std::move(copy)), m_done(chunks, 0), m_gate(gate) {
+  Copiers(uint64_t bytes, std::function<void(uint64_t, uint64_t)> copy) : m_bytes(bytes), m_copy(std::move(copy)) {
+    for (uint64_t at = 0; at < bytes; at += kChunk) m_left.push_back(pieces(std::min(kChunk, bytes - at)));
     const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-    const uint64_t n = std::min<uint64_t>(chunks, std::min(kThreads, hw));
+    const uint64_t n = std::min<uint64_t>(pieces(bytes), std::min(kThreads, hw));
     m_threads.reserve(n);
     for (uint64_t t = 0; t < n; ++t) {
       try {
-        m_threads.emplace_back([this, chunks] {
+        m_threads.emplace_back([this] {
           for (;;) {
-            const uint64_t i = m_next.fetch_add(1);
-            if (i >= chunks) return;
+            const uint64_t at = m_next.fetch_add(kPiece);
+            if (at >= m_bytes) return;
             {
               std::unique_lock<std::mutex> l(m_mutex);
-              m_cv.wait(l, [&] { return m_stop || i < m_gate; });
+              m_cv.wait(l, [&] { return m_stop || at / kChunk < m_gate; });
               if (m_stop) return;
             }
-            m_copy(i);
+            m_copy(at, std::min(kPiece, m_bytes - at));
             std::lock_guard<std::mutex> l(m_mutex);
-            m_done[i] = 1;
-            m_cv.notify_all();
+            if (--m_left[at / kChunk] == 0) m_cv.notify_all();
           }
         });
       } catch (const std::system_error &) {
@@ -63,19 +65,26 @@ public:
   // chunk i, which is behind the gate, has been copied
   void wait(uint64_t i) {
     if (m_threads.empty()) {
-      m_copy(i);
+      if (m_left[i]) m_copy(i * kChunk, std::min(kChunk, m_bytes - i * kChunk));
+      m_left[i] = 0;
       return;
     }
     std::unique_lock<std::mutex> l(m_mutex);
-    m_cv.wait(l, [&] { return m_done[i] != 0; });
+    m_cv.wait(l, [&] { return m_left[i] == 0; });
+  }
+  bool done(uint64_t i) {
+    std::lock_guard<std::mutex> l(m_mutex);
+    return m_left[i] == 0;
   }
 
 private:
-  std::function<void(uint64_t)> m_copy;
+  static uint64_t pieces(uint64_t bytes) { return (bytes + kPiece - 1) / kPiece; }
+  const uint64_t m_bytes;
+  std::function<void(uint64_t, uint64_t)> m_copy;
   std::mutex m_mutex;
   std::condition_variable m_cv;
-  std::vector<char> m_done;
-  uint64_t m_gate;
+  std::vector<uint64_t> m_left; // pieces of a chunk that have not been copied
+  uint64_t m_gate = 0;
   bool m_stop = false;
   std::atomic<uint64_t> m_next{0};
   std::vector<std::thread> m_threads;
@@ -83,9 +92,15 @@ private:
 
 } // namespace
 
-HostStaging::~HostStaging() {
-  for (hipEvent_t e : m_events) (void)hipEventDestroy(e);
+HostStaging::~HostStaging() { release(); }
+
+void HostStaging::release() {
+  for (hipEvent_t &e : m_events) {
+    if (e) (void)hipEventDestroy(e);
+    e = nullptr;
+  }
   if (m_pinned) (void)hipHostFree(m_pinned);
+  m_pinned = nullptr;
 }
 
 bool HostStaging::worthwhile(const void *host, uint64_t bytes) {
@@ -99,69 +114,93 @@ bool HostStaging::worthwhile(const void *host, uint64_t bytes) {
   return a.type == hipMemoryTypeUnregistered;
 }
 
-void HostStaging::reserve(uint64_t bytes, hipStream_t s) {
-  const uint64_t want = std::min(bytes, kMaxBytes);
-  if (m_used + want <= m_capacity) return;
-  hipCheck(hipStreamSynchronize(s), "hipStreamSynchronize"); // nothing on the link reads or writes the buffer any more
-  m_used = 0;
-  if (want <= m_capacity) return;
-  if (m_pinned) hipCheck(hipHostFree(m_pinned), "hipHostFree");
-  m_pinned = nullptr;
-  m_capacity = 0;
-  void *p = nullptr;
-  hipCheck(hipHostMalloc(&p, want, hipHostMallocDefault), "hipHostMalloc(staging)");
-  m_pinned = static_cast<uint8_t *>(p);
-  m_capacity = want;
+void HostStaging::prepare() {
+  if (m_pinned) return;
+  try {
+    void *p = nullptr;
+    hipCheck(hipHostMalloc(&p, kSlots * kChunk, hipHostMallocDefault), "hipHostMalloc(staging)");
+    m_pinned = static_cast<uint8_t *>(p);
+    for (hipEvent_t &e : m_events) hipCheck(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreateWithFlags");
+  } catch (...) {
+    release();
+    throw;
+  }
+}
+
+void HostStaging::begin(hipStream_t s) {
+  if (m_unsettled) { // a transfer ended half-way: the link may still read or write any slot
+    hipCheck(hipStreamSynchronize(s), "hipStreamSynchronize");
+    std::fill(std::begin(m_busy), std::end(m_busy), false);
+  }
+  m_unsettled = true;
+}
+
+// Slot `i` can be written again: its last transfer has passed, or `wait` for that.
+bool HostStaging::idle(size_t i, bool wait) {
+  if (!m_busy[i]) return true;
+  if (wait) hipCheck(hipEventSynchronize(m_events[i]), "hipEventSynchronize");
+  else {
+    const hipError_t e = hipEventQuery(m_events[i]);
+    if (e == hipErrorNotReady) return false;
+    hipCheck(e, "hipEventQuery");
+  }
+  m_busy[i] = false;
+  return true;
 }
 
 void HostStaging::upload(void *device, const void *host, uint64_t bytes, hipStream_t s) {
+  begin(s);
   const uint8_t *src = static_cast<const uint8_t *>(host);
   uint8_t *dst = static_cast<uint8_t *>(device);
-  while (bytes) {
-    reserve(bytes, s);
-    const uint64_t n = std::min(bytes, m_capacity - m_used), chunks = (n + kChunk - 1) / kChunk;
-    uint8_t *stage = m_pinned + m_used;
-    auto size = [n](uint64_t i) { return std::min(kChunk, n - i * kChunk); };
-    Copiers copiers(chunks, chunks, [=](uint64_t i) { std::memcpy(stage + i * kChunk, src + i * kChunk, size(i)); });
+  const uint64_t chunks = (bytes + kChunk - 1) / kChunk, first = m_next;
+  auto size = [=](uint64_t i) { return std::min(kChunk, bytes - i * kChunk); };
+  auto slot = [=](uint64_t i) { return static_cast<size_t>((first + i) % kSlots); };
+  uint8_t *ring = m_pinned;
+  uint64_t open = 0; // chunks whose slot may be written
+  {
+    Copiers copiers(bytes, [=](uint64_t at, uint64_t n) { std::memcpy(ring + slot(at / kChunk) * kChunk + at % kChunk, src + at, n); });
     for (uint64_t i = 0; i < chunks; ++i) {
+      while (open < chunks && open < i + kSlots && idle(slot(open), open == i)) ++open;
+      copiers.open(open);
       copiers.wait(i);
-      m_used = std::max<uint64_t>(m_used, static_cast<uint64_t>(stage - m_pinned) + i * kChunk + size(i));
-      hipCheck(hipMemcpyAsync(dst + i * kChunk, stage + i * kChunk, size(i), hipMemcpyHostToDevice, s), "hipMemcpyAsync(input)");
+      hipCheck(hipMemcpyAsync(dst + i * kChunk, ring + slot(i) * kChunk, size(i), hipMemcpyHostToDevice, s), "hipMemcpyAsync(input)");
+      hipCheck(hipEventRecord(m_events[slot(i)], s), "hipEventRecord");
+      m_busy[slot(i)] = true;
     }
-    src += n; dst += n; bytes -= n;
   }
+  m_next = (first + chunks) % kSlots;
+  m_unsettled = false;
 }
 
 void HostStaging::download(void *host, const void *device, uint64_t bytes, hipStream_t s) {
+  begin(s);
   uint8_t *dst = static_cast<uint8_t *>(host);
   const uint8_t *src = static_cast<const uint8_t *>(device);
-  while (bytes) {
-    reserve(bytes, s);
-    const uint64_t n = std::min(bytes, m_capacity - m_used), chunks = (n + kChunk - 1) / kChunk;
-    uint8_t *stage = m_pinned + m_used;
-    auto size = [n](uint64_t i) { return std::min(kChunk, n - i * kChunk); };
-    while (m_events.size() < chunks) {
-      hipEvent_t e = nullptr;
-      hipCheck(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreateWithFlags");
-      m_events.push_back(e);
-    }
-    m_used += n; // the link writes there until the last event below has passed
+  const uint64_t chunks = (bytes + kChunk - 1) / kChunk, first = m_next;
+  auto size = [=](uint64_t i) { return std::min(kChunk, bytes - i * kChunk); };
+  auto slot = [=](uint64_t i) { return static_cast<size_t>((first + i) % kSlots); };
+  const uint8_t *ring = m_pinned;
+  uint64_t sent = 0;
+  auto send = [&] { // (an upload that still reads the slot comes first in stream order)
+    hipCheck(hipMemcpyAsync(m_pinned + slot(sent) * kChunk, src + sent * kChunk, size(sent), hipMemcpyDeviceToHost, s), "hipMemcpyAsync(output)");
+    hipCheck(hipEventRecord(m_events[slot(sent)], s), "hipEventRecord");
+    m_busy[slot(sent)] = true;
+    ++sent;
+  };
+  while (sent < std::min<uint64_t>(chunks, kSlots)) send();
+  {
+    // the threads start while the kernels still run
+    Copiers copiers(bytes, [=](uint64_t at, uint64_t n) { std::memcpy(dst + at, ring + slot(at / kChunk) * kChunk + at % kChunk, n); });
     for (uint64_t i = 0; i < chunks; ++i) {
-      hipCheck(hipMemcpyAsync(stage + i * kChunk, src + i * kChunk, size(i), hipMemcpyDeviceToHost, s), "hipMemcpyAsync(output)");
-      hipCheck(hipEventRecord(m_events[i], s), "hipEventRecord");
+      if (sent == i) copiers.wait(i - kSlots); // every slot is waiting to be copied out
+      while (sent < chunks && sent < i + kSlots && copiers.done(sent - kSlots)) send();
+      (void)idle(slot(i), true);
+      copiers.open(i + 1);
     }
-    {
-      // the threads start while the kernels still run
-      Copiers copiers(chunks, 0, [=](uint64_t i) { std::memcpy(dst + i * kChunk, stage + i * kChunk, size(i)); });
-      for (uint64_t i = 0; i < chunks; ++i) {
-        hipCheck(hipEventSynchronize(m_events[i]), "hipEventSynchronize");
-        copiers.open(i + 1);
-      }
-      for (uint64_t i = 0; i < chunks; ++i) copiers.wait(i);
-    }
-    m_used = 0; // in stream order everything before the last event has passed as well
-    dst += n; src += n; bytes -= n;
+    for (uint64_t i = 0; i < chunks; ++i) copiers.wait(i);
   }
+  m_next = (first + chunks) % kSlots;
+  m_unsettled = false;
 }
 
 } // namespace denox::runtime

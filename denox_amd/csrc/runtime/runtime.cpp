@@ -575,16 +575,16 @@ void Instance::infer(const void *const *inputs, void *const *outputs) {
   hipStream_t s = m_model->context()->stream();
   auto bytesOf = [&](uint32_t t) { return static_cast<uint64_t>(m.tensors[t].size.eval(m_sym)); };
   std::vector<char> stageIn(m.inputs.size(), 0), stageOut(m.outputs.size(), 0);
-  uint64_t staged = 0;
+  bool staged = false;
   for (size_t i = 0; i < m.inputs.size(); ++i)
-    if (inputs[i] && HostStaging::worthwhile(inputs[i], bytesOf(m.inputs[i]))) stageIn[i] = 1, staged += bytesOf(m.inputs[i]);
+    if (inputs[i] && HostStaging::worthwhile(inputs[i], bytesOf(m.inputs[i]))) stageIn[i] = 1, staged = true;
   for (size_t i = 0; i < m.outputs.size(); ++i)
-    if (outputs[i] && HostStaging::worthwhile(outputs[i], bytesOf(m.outputs[i]))) stageOut[i] = 1, staged += bytesOf(m.outputs[i]);
+    if (outputs[i] && HostStaging::worthwhile(outputs[i], bytesOf(m.outputs[i]))) stageOut[i] = 1, staged = true;
   std::unique_lock<std::mutex> stagingLock(m_model->context()->hostStagingMutex(), std::defer_lock);
   HostStaging &staging = m_model->context()->hostStaging();
   if (staged) {
     stagingLock.lock();
-    staging.prepare(staged, s);
+    staging.prepare();
   }
   for (size_t i = 0; i < m.inputs.size(); ++i) {
     if (!inputs[i]) fail(Status::InvalidArgument, "infer: null input pointer");

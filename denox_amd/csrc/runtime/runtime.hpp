@@ -38,8 +38,8 @@ public:
   void *staticScratch() const { return m_staticScratch; }
   // recorded behind every call of the allocation-free entry point (created with the context: that call creates nothing)
   hipEvent_t staticScratchDone() const { return m_staticDone; }
-  // infer: page-locked memory for large pageable arrays, one for all instances of the context (allocating 50 MB takes 3 ms, which an
-  // instance's first call would pay each time).  A call holds the mutex while it uses it: calls of other threads on this
+  // infer: page-locked memory for large pageable arrays, one ring for all instances of the context (made by the first call that has use
+  // for it).  A call holds the mutex while it uses it: calls of other threads on this
   // context would wait for this one's work on the common stream anyway.
   HostStaging &hostStaging() { return m_staging; }
   std::mutex &hostStagingMutex() { return m_stagingMutex; }

@@ -1,0 +1,174 @@
+// Test program for denox_amd/csrc/runtime/host_staging.cpp without a GPU: the HIP calls it makes are stood in for by one
+// "stream" thread that runs copies and events in order, as late as it is told to.
+// usage: host_staging_probe CASE; prints "ok" or what went wrong.
+#include "../denox_amd/csrc/runtime/host_staging.cpp"
+#include <atomic>
+#include <chrono>
+#include <cstdio>
+#include <cstdlib>
+#include <deque>
+#include <random>
+
+namespace {
+std::mutex g_mutex;
+std::condition_variable g_cv;
+struct Work { std::function<void()> run; };
+std::deque<Work> g_queue;
+uint64_t g_enqueued = 0, g_finished = 0;
+std::atomic<int> g_delayUs{0}, g_failCopy{-1}, g_pinned{0}, g_events{0};
+struct Event { uint64_t at = 0; };
+
+void stream() {
+  for (;;) {
+    Work w;
+    {
+      std::unique_lock<std::mutex> l(g_mutex);
+      g_cv.wait(l, [] { return !g_queue.empty(); });
+      w = std::move(g_queue.front());
+      g_queue.pop_front();
+    }
+    if (!w.run) return;
+    if (const int d = g_delayUs) std::this_thread::sleep_for(std::chrono::microseconds(d));
+    w.run();
+    std::lock_guard<std::mutex> l(g_mutex);
+    ++g_finished;
+    g_cv.notify_all();
+  }
+}
+void push(std::function<void()> f) {
+  std::lock_guard<std::mutex> l(g_mutex);
+  const bool work = static_cast<bool>(f);
+  g_queue.push_back(Work{std::move(f)});
+  if (work) ++g_enqueued;
+  g_cv.notify_all();
+}
+} // namespace
+
+extern "C" {
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+  *p = std::malloc(n);
+  ++g_pinned;
+  return hipSuccess;
+}
+hipError_t hipHostFree(void *p) {
+  std::free(p);
+  --g_pinned;
+  return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+  *e = reinterpret_cast<hipEvent_t>(new Event);
+  ++g_events;
+  return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e) {
+  delete reinterpret_cast<Event *>(e);
+  --g_events;
+  return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
+  std::lock_guard<std::mutex> l(g_mutex);
+  reinterpret_cast<Event *>(e)->at = g_enqueued;
+  return hipSuccess;
+}
+hipError_t hipEventQuery(hipEvent_t e) {
+  std::lock_guard<std::mutex> l(g_mutex);
+  return g_finished >= reinterpret_cast<Event *>(e)->at ? hipSuccess : hipErrorNotReady;
+}
+hipError_t hipEventSynchronize(hipEvent_t e) {
+  std::unique_lock<std::mutex> l(g_mutex);
+  const uint64_t at = reinterpret_cast<Event *>(e)->at;
+  g_cv.wait(l, [&] { return g_finished >= at; });
+  return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) {
+  std::unique_lock<std::mutex> l(g_mutex);
+  g_cv.wait(l, [] { return g_finished == g_enqueued; });
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) {
+  if (g_failCopy >= 0 && g_failCopy-- == 0) return hipErrorUnknown;
+  push([=] { std::memcpy(d, s, n); });
+  return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *, const void *) { return hipErrorInvalidValue; }
+hipError_t hipGetLastError() { return hipSuccess; }
+const char *hipGetErrorString(hipError_t) { return "error"; }
+}
+
+namespace denox::runtime {
+void hipCheck(hipError_t e, const char *what) {
+  if (e != hipSuccess) fail(Status::HipError, what);
+}
+} // namespace denox::runtime
+
+using denox::runtime::HostStaging;
+static std::mt19937 rng(1);
+static std::vector<uint8_t> bytes(uint64_t n) {
+  std::vector<uint8_t> v(n);
+  for (auto &b : v) b = static_cast<uint8_t>(rng());
+  return v;
+}
+static void need(bool ok, const char *what) {
+  if (ok) return;
+  std::printf("wrong: %s\n", what);
+  std::fflush(stdout);
+  std::_Exit(1);
+}
+
+// uploads of the given sizes behind one another, then the same arrays down again
+static void roundTrip(HostStaging &st, const std::vector<uint64_t> &sizes) {
+  st.prepare();
+  std::vector<std::vector<uint8_t>> host, device;
+  for (uint64_t n : sizes) {
+    host.push_back(bytes(n));
+    device.emplace_back(n);
+    std::vector<uint8_t> mine = host.back();
+    st.upload(device.back().data(), mine.data(), n, nullptr);
+    std::fill(mine.begin(), mine.end(), uint8_t(0)); // the caller may reuse its array at once
+  }
+  for (size_t i = 0; i < sizes.size(); ++i) {
+    std::vector<uint8_t> back(sizes[i]);
+    st.download(back.data(), device[i].data(), sizes[i], nullptr);
+    need(back == host[i], "array came back changed");
+  }
+}
+
+int main(int argc, char **argv) {
+  const std::string c = argc > 1 ? argv[1] : "";
+  std::thread worker(stream);
+  const uint64_t M = 1ull << 20, C = HostStaging::kChunk, R = HostStaging::kSlots * C;
+  {
+    HostStaging st;
+    if (c == "sizes") {
+      for (int delay : {0, 200})
+        for (uint64_t n : {uint64_t(1), C - 1, C, C + 1, 4 * M, R - 1, R, R + 1, 3 * R + 12345, 2 * R}) {
+          g_delayUs = delay;
+          roundTrip(st, {n});
+          roundTrip(st, {n, C / 2 + 3, n + 7});
+        }
+      need(g_pinned == 1 && g_events == static_cast<int>(HostStaging::kSlots), "one ring, one event per slot");
+    } else if (c == "failed_transfer") {
+      for (int at : {0, 1, static_cast<int>(HostStaging::kSlots), 3 * static_cast<int>(HostStaging::kSlots) - 1}) {
+        st.prepare();
+        std::vector<uint8_t> host = bytes(3 * R), device(3 * R);
+        for (bool down : {false, true}) {
+          g_delayUs = 300;
+          g_failCopy = at;
+          bool threw = false;
+          try {
+            if (down) st.download(host.data(), device.data(), host.size(), nullptr);
+            else st.upload(device.data(), host.data(), host.size(), nullptr);
+          } catch (const denox::Error &) { threw = true; }
+          need(threw, "an error of the link is reported");
+          g_failCopy = -1;
+          roundTrip(st, {2 * R + 5});
+        }
+      }
+    } else need(false, "no such case");
+  }
+  need(g_pinned == 0 && g_events == 0, "memory or events left behind");
+  push(nullptr);
+  worker.join();
+  std::printf("ok\n");
+  return 0;
+}

@@ -1,6 +1,6 @@
-"""The blocking call on large pageable arrays (host_staging.cpp: page-locked chunks of 2 MiB, at most 64 MiB of them): copies only, so
+"""The blocking call on large pageable arrays (host_staging.cpp: a ring of four page-locked chunks of 4 MiB): copies only, so
 the result has the bits of the same call through small or page-locked arrays.  Sizes around the 4 MiB threshold, one chunk more and
-less, several inputs and outputs, arrays larger than the staging memory, and calls from two threads on two instances."""
+less, several inputs and outputs, arrays larger than the ring, and calls from two threads on two instances."""
 import threading
 
 import numpy as np
