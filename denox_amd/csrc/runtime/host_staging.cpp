@@ -114,17 +114,16 @@ bool HostStaging::worthwhile(const void *host, uint64_t bytes) {
   return a.type == hipMemoryTypeUnregistered;
 }
 
-void HostStaging::prepare() {
-  if (m_pinned) return;
-  try {
-    void *p = nullptr;
-    hipCheck(hipHostMalloc(&p, kSlots * kChunk, hipHostMallocDefault), "hipHostMalloc(staging)");
-    m_pinned = static_cast<uint8_t *>(p);
-    for (hipEvent_t &e : m_events) hipCheck(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreateWithFlags");
-  } catch (...) {
-    release();
-    throw;
-  }
+bool HostStaging::ready() {
+  if (m_pinned) return true;
+  void *p = nullptr;
+  bool ok = hipHostMalloc(&p, kSlots * kChunk, hipHostMallocDefault) == hipSuccess;
+  if (ok) m_pinned = static_cast<uint8_t *>(p);
+  for (size_t i = 0; ok && i < kSlots; ++i) ok = hipEventCreateWithFlags(&m_events[i], hipEventDisableTiming) == hipSuccess;
+  if (ok) return true;
+  (void)hipGetLastError();
+  release();
+  return false;
 }
 
 void HostStaging::begin(hipStream_t s) {

@@ -24,8 +24,8 @@ public:
   // Whether a transfer of `bytes` at `host` gains from staging: large enough to pay for the threads, and not page-locked
   // already (then the link can read it directly).
   static bool worthwhile(const void *host, uint64_t bytes);
-  // Makes the page-locked memory on the first call.
-  void prepare();
+  // Page-locked memory is there (made on the first call).  false: it cannot be had, transfer directly.
+  bool ready();
   // Enqueues the copy on `s`; returns when the whole array has been read.
   void upload(void *device, const void *host, uint64_t bytes, hipStream_t s);
   // Waits for what is enqueued on `s` and copies; returns when the whole array has been written.

@@ -584,7 +584,10 @@ void Instance::infer(const void *const *inputs, void *const *outputs) {
   HostStaging &staging = m_model->context()->hostStaging();
   if (staged) {
     stagingLock.lock();
-    staging.prepare();
+    if (!staging.ready()) { // no page-locked memory: the driver's own path takes pageable arrays as well
+      std::fill(stageIn.begin(), stageIn.end(), 0);
+      std::fill(stageOut.begin(), stageOut.end(), 0);
+    }
   }
   for (size_t i = 0; i < m.inputs.size(); ++i) {
     if (!inputs[i]) fail(Status::InvalidArgument, "infer: null input pointer");

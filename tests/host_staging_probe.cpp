@@ -1,5 +1,5 @@
 // Test program for denox_amd/csrc/runtime/host_staging.cpp without a GPU: the HIP calls it makes are stood in for by one
-// "stream" thread that runs copies and events in order, as late as it is told to.
+// "stream" thread that runs copies and events in order, as late as it is told to, and by allocations that fail on demand.
 // usage: host_staging_probe CASE; prints "ok" or what went wrong.
 #include "../denox_amd/csrc/runtime/host_staging.cpp"
 #include <atomic>
@@ -15,7 +15,7 @@ std::condition_variable g_cv;
 struct Work { std::function<void()> run; };
 std::deque<Work> g_queue;
 uint64_t g_enqueued = 0, g_finished = 0;
-std::atomic<int> g_delayUs{0}, g_failCopy{-1}, g_pinned{0}, g_events{0};
+std::atomic<int> g_delayUs{0}, g_failPinned{0}, g_failEvents{0}, g_failCopy{-1}, g_pinned{0}, g_events{0};
 struct Event { uint64_t at = 0; };
 
 void stream() {
@@ -46,6 +46,7 @@ void push(std::function<void()> f) {
 
 extern "C" {
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+  if (g_failPinned) return hipErrorOutOfMemory;
   *p = std::malloc(n);
   ++g_pinned;
   return hipSuccess;
@@ -56,6 +57,7 @@ hipError_t hipHostFree(void *p) {
   return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+  if (g_failEvents && g_events >= 2) return hipErrorOutOfMemory;
   *e = reinterpret_cast<hipEvent_t>(new Event);
   ++g_events;
   return hipSuccess;
@@ -117,7 +119,7 @@ static void need(bool ok, const char *what) {
 
 // uploads of the given sizes behind one another, then the same arrays down again
 static void roundTrip(HostStaging &st, const std::vector<uint64_t> &sizes) {
-  st.prepare();
+  need(st.ready(), "ready");
   std::vector<std::vector<uint8_t>> host, device;
   for (uint64_t n : sizes) {
     host.push_back(bytes(n));
@@ -147,9 +149,19 @@ int main(int argc, char **argv) {
           roundTrip(st, {n, C / 2 + 3, n + 7});
         }
       need(g_pinned == 1 && g_events == static_cast<int>(HostStaging::kSlots), "one ring, one event per slot");
+    } else if (c == "no_page_locked_memory") {
+      g_failPinned = 1;
+      need(!st.ready() && g_pinned == 0 && g_events == 0, "ready without memory");
+      g_failPinned = 0;
+      roundTrip(st, {5 * M});
+    } else if (c == "no_events") {
+      g_failEvents = 1;
+      need(!st.ready() && g_pinned == 0 && g_events == 0, "ready without events");
+      g_failEvents = 0;
+      roundTrip(st, {5 * M});
     } else if (c == "failed_transfer") {
       for (int at : {0, 1, static_cast<int>(HostStaging::kSlots), 3 * static_cast<int>(HostStaging::kSlots) - 1}) {
-        st.prepare();
+        need(st.ready(), "ready");
         std::vector<uint8_t> host = bytes(3 * R), device(3 * R);
         for (bool down : {false, true}) {
           g_delayUs = 300;
