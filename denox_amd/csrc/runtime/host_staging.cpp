@@ -6,7 +6,6 @@
 #include <cstring>
 #include <functional>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 namespace denox::runtime {
@@ -29,7 +28,7 @@ public:
     const uint64_t n = std::min<uint64_t>(pieces(bytes), std::min(kThreads, hw));
     m_threads.reserve(n);
     for (uint64_t t = 0; t < n; ++t) {
-      try {
+      try { // (the vector's memory is there; the thread and its state may be refused)
         m_threads.emplace_back([this] {
           for (;;) {
             const uint64_t at = m_next.fetch_add(kPiece);
@@ -44,7 +43,7 @@ public:
             if (--m_left[at / kChunk] == 0) m_cv.notify_all();
           }
         });
-      } catch (const std::system_error &) {
+      } catch (...) {
         break; // those that started do all the work; without any, wait() does it
       }
     }

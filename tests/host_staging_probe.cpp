@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <deque>
+#include <new>
 #include <random>
 
 namespace {
@@ -16,6 +17,7 @@ struct Work { std::function<void()> run; };
 std::deque<Work> g_queue;
 uint64_t g_enqueued = 0, g_finished = 0;
 std::atomic<int> g_delayUs{0}, g_failPinned{0}, g_failEvents{0}, g_failCopy{-1}, g_pinned{0}, g_events{0};
+std::atomic<long> g_failNew{-1}; // operator new fails from the n-th call on
 struct Event { uint64_t at = 0; };
 
 void stream() {
@@ -43,6 +45,17 @@ void push(std::function<void()> f) {
   g_cv.notify_all();
 }
 } // namespace
+
+void *operator new(size_t n) {
+  if (g_failNew >= 0 && g_failNew-- == 0) {
+    g_failNew = 0; // and every one after it
+    throw std::bad_alloc();
+  }
+  if (void *p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
 
 extern "C" {
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
@@ -176,6 +189,28 @@ int main(int argc, char **argv) {
           roundTrip(st, {2 * R + 5});
         }
       }
+    } else if (c == "no_memory_for_threads") {
+      need(st.ready(), "ready");
+      std::vector<uint8_t> host = bytes(3 * R + 1), device(3 * R + 1), back(3 * R + 1);
+      // whichever allocation is the first to fail, the call throws bad_alloc or does the work; it never ends the process
+      for (bool down : {false, true})
+        for (long at = 0; at < 40; ++at) {
+          (void)hipStreamSynchronize(nullptr);
+          std::fill(back.begin(), back.end(), uint8_t(0));
+          std::memcpy(device.data(), host.data(), host.size());
+          bool threw = false;
+          g_failNew = at;
+          try {
+            // (the stand-in's own queue allocates as well: a failure there surfaces as one of the call's)
+            if (down) st.download(back.data(), device.data(), back.size(), nullptr);
+            else st.upload(device.data(), host.data(), host.size(), nullptr);
+          } catch (const std::bad_alloc &) { threw = true; }
+          g_failNew = -1;
+          (void)hipStreamSynchronize(nullptr);
+          if (down && !threw) need(back == host, "wrong bytes after a failed thread");
+          if (!down && !threw) need(device == host, "wrong bytes after a failed thread");
+        }
+      roundTrip(st, {5 * M});
     } else need(false, "no such case");
   }
   need(g_pinned == 0 && g_events == 0, "memory or events left behind");

@@ -1,6 +1,6 @@
 """Transfers of large pageable arrays (runtime/host_staging.cpp) without a GPU: the source compiled against stand-ins for the HIP calls
 it makes (host_staging_probe.cpp).  Sizes around a chunk and around the ring, several arrays in a row, a link that lags behind;
-page-locked memory and events that cannot be had; a transfer that fails half-way and the ones after it."""
+page-locked memory, events, threads that cannot be had; a transfer that fails half-way and the ones after it."""
 import os
 import subprocess
 
@@ -18,7 +18,7 @@ def probe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("case", ["sizes", "no_page_locked_memory", "no_events", "failed_transfer"])
+@pytest.mark.parametrize("case", ["sizes", "no_page_locked_memory", "no_events", "failed_transfer", "no_memory_for_threads"])
 def test_staged_transfers(probe, case):
     r = subprocess.run([probe, case], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and r.stdout == "ok\n", (r.returncode, r.stdout, r.stderr)
