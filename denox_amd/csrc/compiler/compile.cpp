@@ -66,11 +66,6 @@ static double prefer(const SuperGraphEdge &e, const CompileOptions &opt, double 
   return blocked ? 0.5 * cost : cost;
 }
 
-static constexpr double kUnmeasuredFoldMs = 1e9; // beyond any schedule without such a kernel
-// A forced conv -> conv configuration is taken wherever it exists: single convolutions keep their choice beside it (a forced single one
-// is the only one offered), and on extents that do not suit it two of them may be estimated faster.
-static constexpr double kForcedPairFactor = 1e-3;
-
 double edge_cost_ms(const SuperGraphEdge &e, const std::vector<int64_t> &dp, const Db *db, const CompileOptions &opt, bool *measured) {
   double total = 0.0;
   bool all = db != nullptr;
@@ -86,20 +81,28 @@ double edge_cost_ms(const SuperGraphEdge &e, const std::vector<int64_t> &dp, con
   if (measured) *measured = all;
   if (all) return prefer(e, opt, total);
   total = 0.0;
+  for (const auto &d : e.dispatches) total += estimate_dispatch_ms(d, dp, opt);
+  return prefer(e, opt, total / std::max(1e-3f, e.speedup));
+}
+
+// What the selection compares: an edge's cost, except where something else than time decides.
+static double selection_cost(const SuperGraphEdge &e, double cost, bool measured, const CompileOptions &opt) {
+  constexpr double unmeasuredFoldMs = 1e9; // beyond any schedule without such a kernel; finite, so that a layer that nothing else implements compiles
+  constexpr double forcedPairFactor = 1e-3;
+  if (measured) return cost;
   for (const auto &d : e.dispatches) {
-    total += estimate_dispatch_ms(d, dp, opt);
+    if (!d.convCost.valid) continue;
+    const ConvKernel k = d.convCost.kernel;
+    const bool forced = opt.forceConvConfig == d.convCost.config;
     // The upsample-folding kernels multiply sums of weights that are rounded to binary16 once more (the 1920 x 1080 U-Net's output is 1.34e-3
     // from binary64 with them, 1.22e-3 without): callers take that on with a timing table or by name, an estimate does not
-    // decide it for them, although it costs them time (592 us; 517 with folded kernels).  Finite: a layer that nothing else
-    // implements still compiles.
-    const bool fold = d.convCost.valid && (d.convCost.kernel == ConvKernel::Fold || d.convCost.kernel == ConvKernel::FoldStaged);
-    if (fold && opt.forceConvConfig != d.convCost.config) total += kUnmeasuredFoldMs;
+    // decide it for them, although it costs them time (592 us; 517 with folded kernels).
+    if ((k == ConvKernel::Fold || k == ConvKernel::FoldStaged) && !forced) cost += unmeasuredFoldMs;
+    // A forced conv -> conv configuration is taken wherever it exists: single convolutions keep their choice beside it (a forced
+    // single one is the only one offered), and on extents that do not suit it two of them may be estimated faster.
+    if ((k == ConvKernel::Pair || k == ConvKernel::PairStaged) && forced) cost *= forcedPairFactor;
   }
-  const bool forcedPair = !opt.forceConvConfig.empty() && std::any_of(e.dispatches.begin(), e.dispatches.end(), [&](const ComputeDispatch &d) {
-    return (d.convCost.kernel == ConvKernel::Pair || d.convCost.kernel == ConvKernel::PairStaged) && opt.forceConvConfig == d.convCost.config;
-  });
-  if (forcedPair) total *= kForcedPairFactor;
-  return prefer(e, opt, total / std::max(1e-3f, e.speedup));
+  return cost;
 }
 
 namespace {
@@ -210,14 +213,15 @@ std::vector<uint8_t> compile(const Model &modelIn, const hip::HipCompiler &hipc,
   const auto shaders = get_all_shaders(&hipc);
   SuperGraph g = implement(model, sym, shaders, hipc, opt);
   const std::vector<int64_t> dp = assumed_symeval(model, sym, opt);
-  std::vector<double> cost(g.edges.size());
+  std::vector<double> cost(g.edges.size()), preference(g.edges.size());
   std::vector<bool> measured(g.edges.size());
   for (size_t e = 0; e < g.edges.size(); ++e) {
     bool m = false;
     cost[e] = edge_cost_ms(g.edges[e], dp, db, opt, &m);
     measured[e] = m;
+    preference[e] = selection_cost(g.edges[e], cost[e], m, opt);
   }
-  const std::vector<size_t> chosen = select_schedule(model, g, cost);
+  const std::vector<size_t> chosen = select_schedule(model, g, preference);
 
   dnx::Model out;
   out.version = 0;
@@ -358,7 +362,7 @@ std::vector<uint8_t> compile(const Model &modelIn, const hip::HipCompiler &hipc,
     total += cost[e];
     if (report) {
       report->schedule.push_back(ScheduleEntry{edge.shader, edge.config, edge.dispatches.empty() ? "" : edge.dispatches[0].info.name, cost[e], measured[e]});
-      if (db && !measured[e]) report->warnings.push_back("no measured latency for " + edge.shader + " " + edge.config + "; used the roofline estimate");
+      if (db && !measured[e]) report->warnings.push_back("no measured latency for " + edge.shader + " " + edge.config + "; used the estimate");
     }
   }
 

@@ -1,4 +1,7 @@
 """Schedules selected without a timing table: what the estimates may decide and what they leave to a caller's table or to a name."""
+import os
+import re
+
 import numpy as np
 import pytest
 
@@ -78,6 +81,7 @@ def test_forced_pair_is_taken_on_any_extent(config, H, W):
     m.output(m.conv2d(m.relu(m.conv2d(m.input("x", "W", "H", 64), he_weights(rng, 32, 64), np.zeros(32, np.float16))), he_weights(rng, 3, 32), np.zeros(3, np.float16)))
     dx.compile_model(m, conv_config=config, assume={"H": H, "W": W})
     assert configs() == [config]
+    assert float(re.search(r"estimated_ms=(\S+)", dx.last_compile_report()).group(1)) > 5e-3  # the estimate itself: a launch at least
 
 
 @pytest.mark.parametrize("C,K,config", [(16, 32, None), (64, 64, None), (256, 256, None), (512, 512, None), (64, 64, "w4r2k16"), (32, 32, "x4r2k16")])
@@ -91,3 +95,12 @@ def test_any_assumed_extent_compiles(C, K, config, assume):
     m.output(m.conv2d(t, he_weights(rng, K, K), np.zeros(K, np.float16), padding=(0, 0)))
     dx.compile_model(m, conv_config=config, assume=assume)
     assert "nan" not in dx.last_compile_report().lower()
+
+
+def test_every_configuration_has_a_measured_factor():
+    """A configuration without an entry in conv_cost.cpp's table counts as slow and is hardly ever taken; one that has left the
+    library would keep its entry unnoticed."""
+    src = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(dx.__file__))), "denox_amd", "csrc", "compiler", "conv_cost.cpp")
+    table = open(src).read().split("kFactor[] = {")[1].split("};")[0]
+    names = re.findall(r'\{"(\w+)", [0-9.]+f\}', table)
+    assert len(names) == len(set(names)) and set(names) == set(dx.conv_config_names()), set(names) ^ set(dx.conv_config_names())
