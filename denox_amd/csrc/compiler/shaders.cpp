@@ -1289,7 +1289,9 @@ public:
 
 // A chain of at least two data-movement layers in one pass (kernels/gather.hip): a source seen through a 2x or larger nearest
 // upsample or a replicate pad, or a concat of two such sources, then an activation and a crop.  Each part obeys the feature
-// switch of the same fusion into a convolution; layers that a convolution can absorb are still offered there.  Pixel-major only.
+// switch of the same fusion into a convolution; layers that a convolution can absorb are still offered there.  Pixel-major sources, and a
+// result of its own: block-major tensors come from convolutions and go to them, and a result inside a concat's channel range would be
+// stored in the pieces of lines that this pass is there to avoid.  None of the package's networks leaves such a chain beside its convolutions.
 class GatherShader final : public IShader {
 public:
   explicit GatherShader(const hip::HipCompiler *c) : m_compiler(c) {}
