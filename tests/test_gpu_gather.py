@@ -30,6 +30,7 @@ CHAINS = {
     "upsample3_leaky": (lambda m, x: m.activation(m.upsample(x, 3), "leaky_relu", 0.3), 1),
     "second_upsampled": (lambda m, x: m.slice(m.activation(m.concat(x, m.upsample(m.pool(x))), "leaky_relu", 0.1), 1, x.width, 1, x.height), 2),  # (even extents)
     "both_upsampled": (lambda m, x: (lambda p: m.relu(m.concat(m.upsample(p), m.upsample(m.relu(p)))))(m.pool(x)), 3),  # (even extents)
+    "padded_pools_in_place_avg": (lambda m, x: m.concat(m.pool(m.pad(x, 2, 0, 0, 3)), m.pool(m.pad(m.relu(x), 0, 2, 3, 0), func="avg")), 3),  # into channel ranges
     "two_pads": (lambda m, x: m.relu(m.concat(m.pad(x, 4, 0, 0, 3), m.pad(m.relu(x), 0, 4, 3, 0))), 1),
 }
 
