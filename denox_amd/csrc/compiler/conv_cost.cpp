@@ -66,10 +66,24 @@ float factorOf(const char *name) {
 
 double cdiv(double a, double b) { return std::ceil(a / b); }
 
+// Kernels that share the products of an upsampled source (conv3x3_upshare.hip), one form for all of its configurations: a workgroup's units of
+// work one after the other -- the matrix instructions of the two waves of a SIMD at 2 GHz, 0.5 us per step (its barrier, the first
+// fragments behind it, loads that arrive late), the result's way out -- against the launch's memory traffic.  Fitted to 614 launches
+// of 12 layers (32 to 224 upsampled, 0 to 128 other channels, 16 to 224 outputs) at 96 x 64 to 1920 x 1088 in all layouts: measured over
+// estimated 0.89 - 1.16 for nine of ten, median 1.00.
+double share_cost_us(const ConvCost &c, double ow, double oh, double bytes, unsigned xcds) {
+  const double cap = cdiv(c.CA, 16) * 16, cbp = cdiv(c.CB, 16) * 16, rows = c.waves / (c.KT / 32) * c.rpw, slices = cdiv(cdiv(c.K, 32) * 32, c.KT);
+  const double units = cdiv(ow, 62) * cdiv(oh + 1, 2 * rows) * slices, rounds = cdiv(cdiv(units, xcds), c.slots * slices);
+  const double mfma = cap / 16 * (9 * c.rpw + 3) + cbp / 16 * 36 * c.rpw, steps = cap / c.ck + cbp / 16, tileKB = 2 * rows * 62 * c.KT * 2 / 1024;
+  const double work = rounds * (1.03 * mfma * 2 * 32 / 2000 + 0.506 * steps + 0.0142 * tileKB), memory = bytes / 5.183e6;
+  return kLaunchUs + std::sqrt(work * work + memory * memory);
+}
+
 } // namespace
 
 double conv_cost_us(const ConvCost &c, uint64_t outWidth, uint64_t outHeight, double bytesRead, double bytesWritten, unsigned xcds, unsigned cus, unsigned ldsBytes) {
   const double ow = static_cast<double>(outWidth), oh = static_cast<double>(outHeight);
+  if (c.kernel == ConvKernel::Share) return share_cost_us(c, ow, oh, bytesRead + bytesWritten, xcds);
   const KernelFit &f = kFit[static_cast<int>(c.kernel)];
   const double W = c.waves, RPW = c.rpw, KT = c.KT, CK = c.ck, stagers = (c.pw ? c.pw : c.waves) * 64.0, wavesPerSimd = std::max(1.0, W / 4.0);
   const bool pair = c.kernel == ConvKernel::Pair || c.kernel == ConvKernel::PairStaged, fold = c.kernel == ConvKernel::Fold || c.kernel == ConvKernel::FoldStaged;

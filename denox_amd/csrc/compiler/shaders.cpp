@@ -53,6 +53,8 @@ std::string fmtFloat(float v) {
 // w % ksplit of the 32-channel blocks and row group w / ksplit.
 // hrot: the staged halo unpadded, its 16-byte slots rotated per pixel instead (HROT in conv_common.h: 32-channel steps fit where the
 // padded form allowed 16).  swp: the matrix loop reads the next group's fragments while it issues the current group's (SWP).
+// On an upsampled source A the streaming configurations stand for conv3x3_upshare.hip (chooseShare below; rpw counts the edges between
+// low-resolution rows that a wave computes).
 struct ConvConfig { unsigned waves, rpw, ck; bool resident; unsigned pw; unsigned maxKT; unsigned mf, xb; const char *name; bool pp = false; bool fold = false; bool wideHalo = false; bool ntStore = false; bool ostage = false; unsigned ksplit = 1; bool hrot = false; bool swp = false; };
 const ConvConfig kConvConfigs[] = {
     // weights streamed per step
@@ -321,6 +323,62 @@ std::vector<uint8_t> packFoldWeights(const Op &conv, const FoldGeometry &g) {
   return bytes;
 }
 
+// ---- products of an upsampled source shared between the outputs (conv3x3_upshare.hip) ------------------------------
+struct ShareGeometry {
+  unsigned CA, CB, CAP, CBP, K, KOUTP, KT, cka, slots;
+};
+
+// Whether a configuration of a layer over an upsampled source is that kernel, and its geometry.
+bool chooseShare(const ConvConfig &cfg, const Op &conv, unsigned pattern, unsigned CA, unsigned CB, const DeviceInfo &dev, ShareGeometry &g) {
+  if (cfg.resident || cfg.fold || cfg.mf != 32 || cfg.waves != 8 || cfg.rpw > 2) return false;
+  if (!(pattern & PAT_UPSAMPLE) || (pattern & (PAT_POOL | PAT_CROP | PAT_PADA)) || conv.R != 3 || conv.S != 3 || conv.padX != 1 || conv.padY != 1 || conv.strideX != 1 || conv.strideY != 1) return false;
+  const unsigned K = conv.K;
+  // whole vectors of A; B's partial last vector is read ending at its last channel; two 16-byte stores per accumulator
+  if (CA % 8 || (CB > 0 && CB < 8) || K % 8) return false;
+  g.CA = CA; g.CB = CB; g.CAP = (CA + 15) / 16 * 16; g.CBP = CB ? (CB + 15) / 16 * 16 : 0; g.K = K; g.KOUTP = (K + 31) / 32 * 32;
+  g.cka = g.CAP % 32 ? 16 : 32;
+  if (cfg.rpw == 2 && cfg.ck != g.cka) return false;
+  for (unsigned kt = std::min(g.KOUTP, cfg.maxKT ? cfg.maxKT : 64u); kt >= 32; kt -= 32) {
+    const unsigned kb = kt / 32;
+    if (g.KOUTP % kt || cfg.waves % kb) continue;
+    // one of two buffers: a step's weight fragments and halo in whole loads of 64 lanes
+    const unsigned rows = cfg.waves / kb * cfg.rpw, a = 9 * kb * (g.cka / 16) + ((rows + 1) * 33 * (g.cka / 8) + 63) / 64, b = CB ? 9 * kb + ((2 * rows + 2) * 132 + 63) / 64 : 0;
+    const size_t lds = 2u * 1024u * std::max(a, b) + 4u * g.KOUTP + 4096u * cfg.waves; // two buffers, the bias, a row of each wave
+    if (lds > dev.maxComputeSharedMemory) continue;
+    g.KT = kt;
+    g.slots = std::max(1u, dev.computeUnits / (dev.xcdCount * (g.KOUTP / kt)));
+    return true;
+  }
+  return false;
+}
+
+// [slice of KT channels][step of A, cka channels][tap][32-channel block][16 channels] and behind a slice's steps of A those of B, 16 channels
+// each, in fragments of 64 lanes x 8 halves: lane l holds channels (l / 32) * 8 .. of weight row l % 32.
+std::vector<uint8_t> packShareWeights(const Op &conv, const ShareGeometry &g) {
+  std::vector<uint16_t> out(static_cast<size_t>(g.KOUTP) * 9 * (g.CAP + g.CBP), 0);
+  const unsigned C = g.CA + g.CB, kbs = g.KT / 32;
+  size_t pos = 0;
+  auto step = [&](unsigned kt, unsigned first, unsigned end, unsigned len) { // channels [first, first + len) of the layer; those from `end` on are padding
+    for (unsigned tap = 0; tap < 9; ++tap)
+      for (unsigned kb = 0; kb < kbs; ++kb)
+        for (unsigned ks = 0; ks < len / 16; ++ks)
+          for (unsigned lane = 0; lane < 64; ++lane) {
+            const unsigned k = kt * g.KT + rowChannel(32, g.KT, kb * 32 + lane % 32);
+            for (unsigned e = 0; e < 8; ++e, ++pos) {
+              const unsigned c = first + ks * 16 + lane / 32 * 8 + e;
+              if (k < g.K && c < end) out[pos] = conv.weights[(static_cast<size_t>(k) * C + c) * 9 + tap];
+            }
+          }
+  };
+  for (unsigned kt = 0; kt < g.KOUTP / g.KT; ++kt) {
+    for (unsigned c = 0; c < g.CAP; c += g.cka) step(kt, c, g.CA, g.cka);
+    for (unsigned c = 0; c < g.CBP; c += 16) step(kt, g.CA + c, C, 16);
+  }
+  std::vector<uint8_t> bytes(out.size() * 2);
+  std::memcpy(bytes.data(), out.data(), bytes.size());
+  return bytes;
+}
+
 bool isPairConfigName(const std::string &name); // a configuration of the conv -> conv shader below
 
 class ConvMfmaShader final : public IShader {
@@ -476,7 +534,8 @@ public:
         }
       }
       if (m.blocked()) {
-        if (!offeredBlocked(cfg)) continue;
+        ShareGeometry sg;
+        if (!offeredBlocked(cfg) && !sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg)) continue;
         // block-major sources are read through the per-step buffer resource: every LDS step must lie in one source
         if (!m.inputFormats.empty() && m.inputFormats[0] && CB && CA % stepChannels(cfg, cpad)) continue;
       }
@@ -486,7 +545,8 @@ public:
       if ((cfg.waves + cfg.pw) * 64 > opt.deviceInfo.maxComputeWorkGroupInvocations) continue;
       ConvGeometry g;
       g.R = conv.R; g.S = conv.S; g.SY = conv.strideY; g.SX = conv.strideX;
-      if (!chooseKT(cfg, CA, CB, conv.K, opt.deviceInfo, g)) continue;
+      ShareGeometry sg;
+      if (!sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg) && !chooseKT(cfg, CA, CB, conv.K, opt.deviceInfo, g)) continue;
       out.push_back(c);
     }
     bool forcedFold = false; // a forced upsample-folding configuration leaves matches without an upsample to nobody: not an error
@@ -494,6 +554,15 @@ public:
     if (out.empty() && !forced.empty() && !m.blocked() && !(forcedFold && !(m.pattern & PAT_UPSAMPLE)))
       fail(Status::Unsupported, "conv configuration '" + forced + "' is not valid for this layer");
     return out;
+  }
+
+  static bool sharesProducts(const ConvConfig &cfg, const Op &conv, const Model &model, const Match &m, unsigned CA, unsigned CB, const DeviceInfo &dev, ShareGeometry &g) {
+    if (m.outputVariant) { // whole 16-byte stores
+      const ConcatView v = concatViewOf(model, m.output);
+      if (!v.valid || v.pitch % 8 || v.channelOffset % 8) return false;
+    }
+    if (m.blocked() && !m.inputFormats.empty() && m.inputFormats[0] && CB && (CA % 16 || CB % 8)) return false;
+    return chooseShare(cfg, conv, m.pattern, CA, CB, dev, g);
   }
 
   size_t parameterMemorySize(const Model &model, const Match &m) const override {
@@ -512,7 +581,11 @@ public:
     ConvGeometry g;
     g.R = conv.R; g.S = conv.S; g.SY = conv.strideY; g.SX = conv.strideX;
     FoldGeometry fg{};
-    if (cfg.fold) {
+    ShareGeometry sg{};
+    const bool share = sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg);
+    if (share) {
+      g.CA = CA; g.CB = CB; g.C = CA + CB; g.K = conv.K; g.KOUTP = sg.KOUTP; g.KT = sg.KT; g.slots = sg.slots; g.CPAD = sg.CAP + sg.CBP;
+    } else if (cfg.fold) {
       if (!chooseFold(cfg, CA, CB, conv.K, opt.deviceInfo, fg)) fail(Status::Internal, "conv config rejected at implement time");
       g.CA = CA; g.CB = CB; g.C = CA + CB; g.K = conv.K; g.KOUTP = fg.KOUTP; g.KT = fg.KT; g.slots = fg.slots; g.CPAD = fg.CAP + fg.CBP;
     } else if (!chooseKT(cfg, CA, CB, conv.K, opt.deviceInfo, g)) fail(Status::Internal, "conv config rejected at implement time");
@@ -526,9 +599,10 @@ public:
     const bool pool = (m.pattern & PAT_POOL) != 0, up = (m.pattern & PAT_UPSAMPLE) != 0, crop = (m.pattern & PAT_CROP) != 0;
     const bool padA = (m.pattern & PAT_PADA) != 0, padB = (m.pattern & PAT_PADB) != 0;
 
-    hip::HipCompilerInstance k = m_compiler->read(cfg.fold ? (cfg.pw ? "conv3x3_upfold_ws.hip" : "conv3x3_upfold.hip") : cfg.resident ? "conv3x3_mfma_ws.hip" : "conv3x3_mfma.hip");
+    hip::HipCompilerInstance k = m_compiler->read(share ? "conv3x3_upshare.hip" : cfg.fold ? (cfg.pw ? "conv3x3_upfold_ws.hip" : "conv3x3_upfold.hip") : cfg.resident ? "conv3x3_mfma_ws.hip" : "conv3x3_mfma.hip");
     if (cfg.fold) k.define("BPITCH", fg.bpitch ? fg.bpitch : 8);
     if (cfg.fold && cfg.pw) k.define("CKA", fg.cka);
+    if (share) k.define("CKA", sg.cka);
     if (cfg.ksplit > 1) k.define("KSP", cfg.ksplit);
     if (cfg.ntStore) k.define("STORE_AUX", 2);
     if (cfg.ostage) k.define("OSTAGE", 1);
@@ -542,8 +616,8 @@ public:
     if (padA) k.define("PADA", 1);
     if (padB) k.define("PADB", 1);
     if (crop) k.define("CROP", 1);
-    k.define("WAVES", cfg.waves); k.define("RPW", cfg.rpw); k.define("CK", cfg.fold ? 16u : stepChannels(cfg, g.CPAD));
-    if (cfg.resident) { k.define("SLOTS", g.slots); k.define("NXCD", opt.deviceInfo.xcdCount); } // the grid below is xcdCount * nkt * slots workgroups
+    k.define("WAVES", cfg.waves); k.define("RPW", cfg.rpw); k.define("CK", cfg.fold || share ? 16u : stepChannels(cfg, g.CPAD));
+    if (cfg.resident || share) { k.define("SLOTS", g.slots); k.define("NXCD", opt.deviceInfo.xcdCount); } // the grid below is xcdCount * nkt * slots workgroups
     if (cfg.pw) k.define("PW", cfg.pw);
     if (cfg.pp) k.define("PP", 1);
     if (conv.R != 3 || conv.S != 3) { k.define("KR", conv.R); k.define("KS", conv.S); }
@@ -568,7 +642,8 @@ public:
     const Sym OW = convOut.width, OH = convOut.height;
     const unsigned th = cfg.waves * cfg.rpw;
     const unsigned nkt = g.KOUTP / g.KT;
-    auto d = cfg.fold ? impl.registerDispatch(k, entry, Sym::Const(opt.deviceInfo.xcdCount * (cfg.pw ? 2 : 4) * nkt * g.slots), Sym::Const(1), Sym::Const(1), (cfg.waves + cfg.pw) * 64)
+    auto d = share ? impl.registerDispatch(k, entry, Sym::Const(opt.deviceInfo.xcdCount * nkt * g.slots), Sym::Const(1), Sym::Const(1), cfg.waves * 64)
+           : cfg.fold ? impl.registerDispatch(k, entry, Sym::Const(opt.deviceInfo.xcdCount * (cfg.pw ? 2 : 4) * nkt * g.slots), Sym::Const(1), Sym::Const(1), (cfg.waves + cfg.pw) * 64)
            : cfg.resident ? impl.registerDispatch(k, entry, Sym::Const(opt.deviceInfo.xcdCount * nkt * g.slots), Sym::Const(1), Sym::Const(1), (cfg.waves + cfg.pw) * 64)
                           : impl.registerDispatch(k, entry, sym.cdiv(OW, cfg.mf == 32 ? 32 : 16 * cfg.xb), sym.cdiv(OH, th), Sym::Const(nkt), cfg.waves * 64);
     d.addBinding(dnx::Access::ReadOnly, m.inputs[0]);
@@ -581,7 +656,9 @@ public:
     } else d.addBinding(dnx::Access::WriteOnly, m.output);
     const Op convCopy = conv; // the lazy packers outlive the model reference
     const unsigned ck = cfg.resident ? g.CPAD : stepChannels(cfg, g.CPAD);
-    TensorId wt = cfg.fold ? impl.createParameter(static_cast<size_t>(4) * fg.KOUTP * (4 * fg.CAP + 9 * fg.CBP) * 2, dnx::ScalarType::F16,
+    TensorId wt = share ? impl.createParameter(static_cast<size_t>(sg.KOUTP) * 9 * (sg.CAP + sg.CBP) * 2, dnx::ScalarType::F16,
+                                                   [convCopy, sg]() { return packShareWeights(convCopy, sg); })
+                : cfg.fold ? impl.createParameter(static_cast<size_t>(4) * fg.KOUTP * (4 * fg.CAP + 9 * fg.CBP) * 2, dnx::ScalarType::F16,
                                                   [convCopy, fg]() { return packFoldWeights(convCopy, fg); })
                            : impl.createParameter(static_cast<size_t>(g.KOUTP) * conv.R * conv.S * g.CPAD * 2, dnx::ScalarType::F16,
                                                   [convCopy, g, ck, mf = cfg.mf]() { return packConvWeights(convCopy, g, ck, mf); });
@@ -632,9 +709,9 @@ public:
     d.setFlops(sym.mul(sym.mul(OW, OH), static_cast<int64_t>(2) * conv.R * conv.S * conv.C * conv.K));
     ConvCost cost;
     cost.valid = true;
-    cost.kernel = cfg.fold ? (cfg.pw ? ConvKernel::FoldStaged : ConvKernel::Fold) : !cfg.resident ? ConvKernel::Streamed : cfg.ostage ? ConvKernel::StagedTile : cfg.pp ? ConvKernel::TwoPhase : cfg.pw ? ConvKernel::Staged : ConvKernel::Resident;
+    cost.kernel = share ? ConvKernel::Share : cfg.fold ? (cfg.pw ? ConvKernel::FoldStaged : ConvKernel::Fold) : !cfg.resident ? ConvKernel::Streamed : cfg.ostage ? ConvKernel::StagedTile : cfg.pp ? ConvKernel::TwoPhase : cfg.pw ? ConvKernel::Staged : ConvKernel::Resident;
     cost.config = cfg.name;
-    cost.waves = cfg.waves; cost.pw = cfg.pw; cost.rpw = cfg.rpw; cost.ck = cfg.fold ? 16u : stepChannels(cfg, g.CPAD); cost.mf = cfg.mf; cost.xb = cfg.xb; cost.KT = g.KT; cost.K = conv.K;
+    cost.waves = cfg.waves; cost.pw = cfg.pw; cost.rpw = cfg.rpw; cost.ck = cfg.fold ? 16u : share ? sg.cka : stepChannels(cfg, g.CPAD); cost.mf = cfg.mf; cost.xb = cfg.xb; cost.KT = g.KT; cost.K = conv.K;
     cost.CA = CA; cost.CB = CB; cost.R = conv.R; cost.S = conv.S; cost.SY = conv.strideY; cost.SX = conv.strideX; cost.slots = g.slots;
     cost.cka = cfg.fold ? fg.cka : 0; cost.ksplit = cfg.ksplit; cost.hrot = cfg.hrot; cost.swp = cfg.swp; cost.ntStore = cfg.ntStore;
     cost.blockedIn = blockedIn; cost.blockedOut = blockedOut;

@@ -1,0 +1,95 @@
+"""Convolutions over an upsampled source with the products of a low-resolution pixel shared between its outputs (conv3x3_upshare.hip), at the
+edges of its tiles: strips of 31 source pixels, 8 or 16 output rows per workgroup, 62 stored columns, steps of 16 and 32 channels,
+partial vectors of the second source, slices and blocks of output channels past the last one, both layouts of every tensor.
+
+Inputs, weights and bias are small integers: every product and every partial sum is exact in binary32 (at most 9 * 224 * 2 * 2 + 3 < 2^24)
+and every result within 2048 in magnitude is exact in binary16, so the result has the oracle's bits whatever the order of the sums."""
+import numpy as np
+import pytest
+
+import denox_amd as dx
+from util import assert_bits_equal
+
+pytestmark = pytest.mark.gpu
+
+# CA (upsampled), CB, K, H, W of the result, replicate-padded second source, configurations that are this kernel
+SHAPES = [
+    (64, 9, 64, 34, 124, True), (64, 0, 64, 32, 126, False), (8, 8, 8, 2, 2, False), (16, 16, 32, 16, 62, False), (32, 24, 40, 18, 64, False),
+    (24, 73, 48, 30, 60, True), (96, 32, 112, 4, 250, False), (48, 12, 96, 62, 66, True), (112, 48, 96, 66, 130, False), (224, 20, 64, 10, 38, False),
+    (64, 9, 128, 130, 310, True), (48, 12, 64, 36, 72, True), (32, 64, 224, 14, 18, False),
+]
+
+
+def blocked(x):
+    H, W, C = x.shape
+    return np.ascontiguousarray(x.reshape(H, W, C // 8, 8).transpose(2, 0, 1, 3))
+
+
+def planar(y):
+    g, H, W, _ = y.shape
+    return y.transpose(1, 2, 0, 3).reshape(H, W, g * 8)
+
+
+def layer(CA, CB, K, H, W, padded, rng, act="relu"):
+    m = dx.Model()
+    feeds = {"lo": rng.integers(-2, 3, (H // 2, W // 2, CA)).astype(np.float16)}
+    t = m.upsample(m.input("lo", m.sym("W") // 2, m.sym("H") // 2, CA))
+    if CB:
+        h, w = (H - 3, W - 5) if padded else (H, W)
+        feeds["x"] = rng.integers(-2, 3, (h, w, CB)).astype(np.float16)
+        x = m.input("x", m.sym("W") - 5, m.sym("H") - 3, CB) if padded else m.input("x", "W", "H", CB)
+        t = m.concat(t, m.pad(x, 2, 3, 1, 2) if padded else x)
+    w = rng.choice([-1, 0, 0, 0, 1], (K, CA + CB, 3, 3)).astype(np.float16)
+    t = m.conv2d(t, w, rng.integers(-3, 4, K).astype(np.float16))
+    if act != "none":
+        t = m.activation(t, act, 0.5)
+    m.output(t, "out")
+    return m, t, feeds
+
+
+@pytest.mark.parametrize("config", ["w8r2k32", "w8r2k16", "w8r1k16"])
+@pytest.mark.parametrize("CA,CB,K,H,W,padded", SHAPES)
+def test_shared_products_equal_the_definition(oracle, config, CA, CB, K, H, W, padded):
+    rng = np.random.default_rng(CA + CB + K)
+    m, t, feeds = layer(CA, CB, K, H, W, padded, rng, "leaky_relu" if K % 64 else "relu")
+    want = oracle.run_graph(m.to_ops({"H": H, "W": W}), feeds, "fp32")[t.name]
+    assert np.abs(want).max() < 2048  # (a leaky slope of 1/2 leaves at most one bit below 1)
+    ran = 0
+    for blocked_in in (False, True):
+        for blocked_out in (False, True):
+            if blocked_in and (CA % 16 or CB % 8 or padded):
+                continue
+            layouts = dict(input_layout=dx.Layout.CHWC8 if blocked_in else dx.Layout.HWC, output_layout=dx.Layout.CHWC8 if blocked_out else dx.Layout.HWC)
+            try:
+                blob = dx.compile_model(m, conv_config=config, assume={"H": H, "W": W}, **layouts)
+            except dx.DenoxHipError as e:
+                assert e.status == 5
+                continue
+            d = dx.describe(blob, H=H, W=W)["dispatches"]
+            if not any("UPA=1" in x["debug_info"] and "CKA=" in x["debug_info"] for x in d):
+                continue  # no such kernel for these channels, or another combination of kernels is estimated faster
+            xs = [feeds[k] for k in ("lo", "x") if k in feeds]
+            got = dx.Module.load(blob).instance(H=H, W=W).infer(*[blocked(x) if blocked_in else x for x in xs])[0]
+            assert_bits_equal(planar(got) if blocked_out else got, want.astype(np.float16), f"{config} {layouts}")
+            ran += 1
+    if not ran:
+        pytest.skip("this configuration is another kernel here")
+
+
+@pytest.mark.parametrize("config", ["w8r2k32", "w8r1k16"])
+def test_not_a_number_reaches_its_neighbours_only(config):
+    """An infinity and a NaN of either source: exactly the outputs whose taps cover them are affected (padding channels, lanes that only
+    supply an edge and positions outside the image multiply zeros, never what memory holds there)."""
+    rng = np.random.default_rng(3)
+    H, W = 36, 130
+    m, t, feeds = layer(64, 9, 64, H, W, False, rng, "none")
+    feeds["lo"][7, 31, 5] = np.inf
+    feeds["x"][20, 62, 8] = np.nan
+    blob = dx.compile_model(m, conv_config=config, assume={"H": H, "W": W})
+    assert "CKA=" in dx.describe(blob, H=H, W=W)["dispatches"][0]["debug_info"]
+    got = dx.Module.load(blob).instance(H=H, W=W).infer(feeds["lo"], feeds["x"])[0]
+    bad = ~np.isfinite(got.astype(np.float32)).all(axis=2)
+    want = np.zeros((H, W), bool)
+    want[13:17, 61:65] = True  # source pixel (7, 31) is outputs 14 - 15 x 62 - 63, and one more on each side
+    want[19:22, 61:64] = True
+    assert (bad == want).all(), np.argwhere(bad != want)[:8]
