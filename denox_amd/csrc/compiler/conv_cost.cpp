@@ -79,11 +79,27 @@ double share_cost_us(const ConvCost &c, double ow, double oh, double bytes, unsi
   return kLaunchUs + std::sqrt(work * work + memory * memory);
 }
 
+// Streaming kernels whose weights and halos go straight into LDS (conv3x3_mfma_dl.hip), one form as well: matrix instructions, LDS reads and
+// loads of a unit of work overlap, a pixel-major result leaves the lanes in short pieces, and steps of 16 channels fetch a
+// pixel-major source's lines more than once.  Fitted to 1632 launches of 15 layers (16 to 256 channels, with and without a pool) at
+// 96 x 64 to 1920 x 1088 in all layouts: measured over estimated 0.88 - 1.14 for nine of ten, median 1.00.
+double streamed_lds_cost_us(const ConvCost &c, double ow, double oh, double bytesRead, double bytesWritten, unsigned xcds) {
+  const double kb = c.KT / 32, rows = 8.0 * c.rpw, slices = cdiv(cdiv(c.K, 32) * 32, c.KT), groups = c.CA / 16.0;
+  const double rounds = cdiv(cdiv(cdiv(ow, 32) * cdiv(oh, rows) * slices, xcds), c.slots * slices);
+  const double matrix = 0.865 * 9 * groups * kb * c.rpw * 2 * 32 / 2000, lds = 3.235e-3 * 8 * 3 * groups * (c.rpw + 2 + 3 * kb);
+  const double haloKB = (rows + 2) * 34 * c.CA * 2 / 1024, loads = 2.035e-2 * (haloKB + 9.0 * c.KT * c.CA * 2 / 1024);
+  const double stored = bytesWritten / std::max(1.0, 2 * ow * oh * c.K), tileKB = rows * 32 * c.KT * 2 / 1024 * stored; // (a pooled tile is a quarter)
+  const double unit = std::sqrt(matrix * matrix + lds * lds + loads * loads) + 0.0371 * c.CA / c.ck + (c.ck == 16 && !c.blockedIn ? 0.0036 * haloKB : 0) + (c.blockedOut ? 0 : 0.0141 * tileKB);
+  const double memory = (bytesRead + bytesWritten) / 5.712e6;
+  return kLaunchUs + std::pow(std::pow(rounds * unit, 1.2) + std::pow(memory, 1.2), 1 / 1.2);
+}
+
 } // namespace
 
 double conv_cost_us(const ConvCost &c, uint64_t outWidth, uint64_t outHeight, double bytesRead, double bytesWritten, unsigned xcds, unsigned cus, unsigned ldsBytes) {
   const double ow = static_cast<double>(outWidth), oh = static_cast<double>(outHeight);
   if (c.kernel == ConvKernel::Share) return share_cost_us(c, ow, oh, bytesRead + bytesWritten, xcds);
+  if (c.kernel == ConvKernel::StreamedLds) return streamed_lds_cost_us(c, ow, oh, bytesRead, bytesWritten, xcds);
   const KernelFit &f = kFit[static_cast<int>(c.kernel)];
   const double W = c.waves, RPW = c.rpw, KT = c.KT, CK = c.ck, stagers = (c.pw ? c.pw : c.waves) * 64.0, wavesPerSimd = std::max(1.0, W / 4.0);
   const bool pair = c.kernel == ConvKernel::Pair || c.kernel == ConvKernel::PairStaged, fold = c.kernel == ConvKernel::Fold || c.kernel == ConvKernel::FoldStaged;

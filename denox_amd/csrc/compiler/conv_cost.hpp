@@ -5,7 +5,7 @@
 
 namespace denox::compiler {
 
-enum class ConvKernel : uint8_t { Streamed, Resident, Staged, StagedTile, TwoPhase, Fold, FoldStaged, Pair, PairStaged, Share };
+enum class ConvKernel : uint8_t { Streamed, Resident, Staged, StagedTile, TwoPhase, Fold, FoldStaged, Pair, PairStaged, Share, StreamedLds };
 
 // What the estimate needs to know about a dispatch; the extents are those of the convolution's result before a fused pool or crop.
 struct ConvCost {

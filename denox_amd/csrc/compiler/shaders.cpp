@@ -53,8 +53,8 @@ std::string fmtFloat(float v) {
 // w % ksplit of the 32-channel blocks and row group w / ksplit.
 // hrot: the staged halo unpadded, its 16-byte slots rotated per pixel instead (HROT in conv_common.h: 32-channel steps fit where the
 // padded form allowed 16).  swp: the matrix loop reads the next group's fragments while it issues the current group's (SWP).
-// On an upsampled source A the streaming configurations stand for conv3x3_upshare.hip (chooseShare below; rpw counts the edges between
-// low-resolution rows that a wave computes).
+// On an upsampled source A the streaming configurations of 8 waves stand for conv3x3_upshare.hip (chooseShare below; rpw counts the edges between
+// low-resolution rows that a wave computes), on a plain source of whole steps of channels for conv3x3_mfma_dl.hip (chooseStreamedLds).
 struct ConvConfig { unsigned waves, rpw, ck; bool resident; unsigned pw; unsigned maxKT; unsigned mf, xb; const char *name; bool pp = false; bool fold = false; bool wideHalo = false; bool ntStore = false; bool ostage = false; unsigned ksplit = 1; bool hrot = false; bool swp = false; };
 const ConvConfig kConvConfigs[] = {
     // weights streamed per step
@@ -325,7 +325,7 @@ std::vector<uint8_t> packFoldWeights(const Op &conv, const FoldGeometry &g) {
 
 // ---- products of an upsampled source shared between the outputs (conv3x3_upshare.hip) ------------------------------
 struct ShareGeometry {
-  unsigned CA, CB, CAP, CBP, K, KOUTP, KT, cka, slots;
+  unsigned CA, CB, CAP, CBP, K, KOUTP, KT, cka, slots, rpw;
 };
 
 // Whether a configuration of a layer over an upsampled source is that kernel, and its geometry.
@@ -336,7 +336,7 @@ bool chooseShare(const ConvConfig &cfg, const Op &conv, unsigned pattern, unsign
   // whole vectors of A; B's partial last vector is read ending at its last channel; two 16-byte stores per accumulator
   if (CA % 8 || (CB > 0 && CB < 8) || K % 8) return false;
   g.CA = CA; g.CB = CB; g.CAP = (CA + 15) / 16 * 16; g.CBP = CB ? (CB + 15) / 16 * 16 : 0; g.K = K; g.KOUTP = (K + 31) / 32 * 32;
-  g.cka = g.CAP % 32 ? 16 : 32;
+  g.cka = g.CAP % 32 ? 16 : 32; g.rpw = cfg.rpw;
   if (cfg.rpw == 2 && cfg.ck != g.cka) return false;
   for (unsigned kt = std::min(g.KOUTP, cfg.maxKT ? cfg.maxKT : 64u); kt >= 32; kt -= 32) {
     const unsigned kb = kt / 32;
@@ -377,6 +377,24 @@ std::vector<uint8_t> packShareWeights(const Op &conv, const ShareGeometry &g) {
   std::vector<uint8_t> bytes(out.size() * 2);
   std::memcpy(bytes.data(), out.data(), bytes.size());
   return bytes;
+}
+
+// The streaming configurations of 8 waves on a plain source of whole steps are conv3x3_mfma_dl.hip; its geometry in the same form (CB = 0).
+bool chooseStreamedLds(const ConvConfig &cfg, const Op &conv, unsigned pattern, unsigned CA, unsigned CB, const DeviceInfo &dev, ShareGeometry &g) {
+  if (cfg.resident || cfg.fold || cfg.mf != 32 || cfg.waves != 8 || cfg.rpw != 2 || (cfg.ck != 16 && cfg.ck != 32)) return false;
+  if ((pattern & ~(PAT_ACT | PAT_POOL)) || CB || conv.R != 3 || conv.S != 3 || conv.padX != 1 || conv.padY != 1 || conv.strideX != 1 || conv.strideY != 1) return false;
+  if (CA % cfg.ck || conv.K % 8) return false;
+  g.CA = g.CAP = CA; g.CB = g.CBP = 0; g.K = conv.K; g.KOUTP = (conv.K + 31) / 32 * 32; g.cka = cfg.ck;
+  for (unsigned kt = std::min(g.KOUTP, 128u); kt >= 32; kt -= 32) {
+    if (g.KOUTP % kt) continue;
+    g.rpw = cfg.ck == 16 && kt <= 64 ? 4 : 2; // (with 16 channels a step's halo leaves room for tiles of 32 rows)
+    const size_t lds = 2u * 1024u * (9 * (kt / 32) * (cfg.ck / 16) + ((8 * g.rpw + 2) * 34 * (cfg.ck / 8) + 63) / 64) + 4u * g.KOUTP;
+    if (lds > dev.maxComputeSharedMemory) continue;
+    g.KT = kt;
+    g.slots = std::max(1u, dev.computeUnits / (dev.xcdCount * (g.KOUTP / kt)));
+    return true;
+  }
+  return false;
 }
 
 bool isPairConfigName(const std::string &name); // a configuration of the conv -> conv shader below
@@ -535,7 +553,7 @@ public:
       }
       if (m.blocked()) {
         ShareGeometry sg;
-        if (!offeredBlocked(cfg) && !sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg)) continue;
+        if (!offeredBlocked(cfg) && !sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg) && !streamsIntoLds(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg)) continue;
         // block-major sources are read through the per-step buffer resource: every LDS step must lie in one source
         if (!m.inputFormats.empty() && m.inputFormats[0] && CB && CA % stepChannels(cfg, cpad)) continue;
       }
@@ -546,7 +564,7 @@ public:
       ConvGeometry g;
       g.R = conv.R; g.S = conv.S; g.SY = conv.strideY; g.SX = conv.strideX;
       ShareGeometry sg;
-      if (!sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg) && !chooseKT(cfg, CA, CB, conv.K, opt.deviceInfo, g)) continue;
+      if (!sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg) && !streamsIntoLds(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg) && !chooseKT(cfg, CA, CB, conv.K, opt.deviceInfo, g)) continue;
       out.push_back(c);
     }
     bool forcedFold = false; // a forced upsample-folding configuration leaves matches without an upsample to nobody: not an error
@@ -563,6 +581,13 @@ public:
     }
     if (m.blocked() && !m.inputFormats.empty() && m.inputFormats[0] && CB && (CA % 16 || CB % 8)) return false;
     return chooseShare(cfg, conv, m.pattern, CA, CB, dev, g);
+  }
+  static bool streamsIntoLds(const ConvConfig &cfg, const Op &conv, const Model &model, const Match &m, unsigned CA, unsigned CB, const DeviceInfo &dev, ShareGeometry &g) {
+    if (m.outputVariant) { // whole 16-byte stores
+      const ConcatView v = concatViewOf(model, m.output);
+      if (!v.valid || v.pitch % 8 || v.channelOffset % 8) return false;
+    }
+    return chooseStreamedLds(cfg, conv, m.pattern, CA, CB, dev, g);
   }
 
   size_t parameterMemorySize(const Model &model, const Match &m) const override {
@@ -582,8 +607,8 @@ public:
     g.R = conv.R; g.S = conv.S; g.SY = conv.strideY; g.SX = conv.strideX;
     FoldGeometry fg{};
     ShareGeometry sg{};
-    const bool share = sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg);
-    if (share) {
+    const bool share = sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg), intoLds = !share && streamsIntoLds(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg);
+    if (share || intoLds) {
       g.CA = CA; g.CB = CB; g.C = CA + CB; g.K = conv.K; g.KOUTP = sg.KOUTP; g.KT = sg.KT; g.slots = sg.slots; g.CPAD = sg.CAP + sg.CBP;
     } else if (cfg.fold) {
       if (!chooseFold(cfg, CA, CB, conv.K, opt.deviceInfo, fg)) fail(Status::Internal, "conv config rejected at implement time");
@@ -599,7 +624,7 @@ public:
     const bool pool = (m.pattern & PAT_POOL) != 0, up = (m.pattern & PAT_UPSAMPLE) != 0, crop = (m.pattern & PAT_CROP) != 0;
     const bool padA = (m.pattern & PAT_PADA) != 0, padB = (m.pattern & PAT_PADB) != 0;
 
-    hip::HipCompilerInstance k = m_compiler->read(share ? "conv3x3_upshare.hip" : cfg.fold ? (cfg.pw ? "conv3x3_upfold_ws.hip" : "conv3x3_upfold.hip") : cfg.resident ? "conv3x3_mfma_ws.hip" : "conv3x3_mfma.hip");
+    hip::HipCompilerInstance k = m_compiler->read(share ? "conv3x3_upshare.hip" : intoLds ? "conv3x3_mfma_dl.hip" : cfg.fold ? (cfg.pw ? "conv3x3_upfold_ws.hip" : "conv3x3_upfold.hip") : cfg.resident ? "conv3x3_mfma_ws.hip" : "conv3x3_mfma.hip");
     if (cfg.fold) k.define("BPITCH", fg.bpitch ? fg.bpitch : 8);
     if (cfg.fold && cfg.pw) k.define("CKA", fg.cka);
     if (share) k.define("CKA", sg.cka);
@@ -616,8 +641,8 @@ public:
     if (padA) k.define("PADA", 1);
     if (padB) k.define("PADB", 1);
     if (crop) k.define("CROP", 1);
-    k.define("WAVES", cfg.waves); k.define("RPW", cfg.rpw); k.define("CK", cfg.fold || share ? 16u : stepChannels(cfg, g.CPAD));
-    if (cfg.resident || share) { k.define("SLOTS", g.slots); k.define("NXCD", opt.deviceInfo.xcdCount); } // the grid below is xcdCount * nkt * slots workgroups
+    k.define("WAVES", cfg.waves); k.define("RPW", intoLds ? sg.rpw : cfg.rpw); k.define("CK", cfg.fold || share ? 16u : stepChannels(cfg, g.CPAD));
+    if (cfg.resident || share || intoLds) { k.define("SLOTS", g.slots); k.define("NXCD", opt.deviceInfo.xcdCount); } // the grid below is xcdCount * nkt * slots workgroups
     if (cfg.pw) k.define("PW", cfg.pw);
     if (cfg.pp) k.define("PP", 1);
     if (conv.R != 3 || conv.S != 3) { k.define("KR", conv.R); k.define("KS", conv.S); }
@@ -642,7 +667,7 @@ public:
     const Sym OW = convOut.width, OH = convOut.height;
     const unsigned th = cfg.waves * cfg.rpw;
     const unsigned nkt = g.KOUTP / g.KT;
-    auto d = share ? impl.registerDispatch(k, entry, Sym::Const(opt.deviceInfo.xcdCount * nkt * g.slots), Sym::Const(1), Sym::Const(1), cfg.waves * 64)
+    auto d = share || intoLds ? impl.registerDispatch(k, entry, Sym::Const(opt.deviceInfo.xcdCount * nkt * g.slots), Sym::Const(1), Sym::Const(1), cfg.waves * 64)
            : cfg.fold ? impl.registerDispatch(k, entry, Sym::Const(opt.deviceInfo.xcdCount * (cfg.pw ? 2 : 4) * nkt * g.slots), Sym::Const(1), Sym::Const(1), (cfg.waves + cfg.pw) * 64)
            : cfg.resident ? impl.registerDispatch(k, entry, Sym::Const(opt.deviceInfo.xcdCount * nkt * g.slots), Sym::Const(1), Sym::Const(1), (cfg.waves + cfg.pw) * 64)
                           : impl.registerDispatch(k, entry, sym.cdiv(OW, cfg.mf == 32 ? 32 : 16 * cfg.xb), sym.cdiv(OH, th), Sym::Const(nkt), cfg.waves * 64);
@@ -656,7 +681,7 @@ public:
     } else d.addBinding(dnx::Access::WriteOnly, m.output);
     const Op convCopy = conv; // the lazy packers outlive the model reference
     const unsigned ck = cfg.resident ? g.CPAD : stepChannels(cfg, g.CPAD);
-    TensorId wt = share ? impl.createParameter(static_cast<size_t>(sg.KOUTP) * 9 * (sg.CAP + sg.CBP) * 2, dnx::ScalarType::F16,
+    TensorId wt = share || intoLds ? impl.createParameter(static_cast<size_t>(sg.KOUTP) * 9 * (sg.CAP + sg.CBP) * 2, dnx::ScalarType::F16,
                                                    [convCopy, sg]() { return packShareWeights(convCopy, sg); })
                 : cfg.fold ? impl.createParameter(static_cast<size_t>(4) * fg.KOUTP * (4 * fg.CAP + 9 * fg.CBP) * 2, dnx::ScalarType::F16,
                                                   [convCopy, fg]() { return packFoldWeights(convCopy, fg); })
@@ -709,9 +734,9 @@ public:
     d.setFlops(sym.mul(sym.mul(OW, OH), static_cast<int64_t>(2) * conv.R * conv.S * conv.C * conv.K));
     ConvCost cost;
     cost.valid = true;
-    cost.kernel = share ? ConvKernel::Share : cfg.fold ? (cfg.pw ? ConvKernel::FoldStaged : ConvKernel::Fold) : !cfg.resident ? ConvKernel::Streamed : cfg.ostage ? ConvKernel::StagedTile : cfg.pp ? ConvKernel::TwoPhase : cfg.pw ? ConvKernel::Staged : ConvKernel::Resident;
+    cost.kernel = share ? ConvKernel::Share : intoLds ? ConvKernel::StreamedLds : cfg.fold ? (cfg.pw ? ConvKernel::FoldStaged : ConvKernel::Fold) : !cfg.resident ? ConvKernel::Streamed : cfg.ostage ? ConvKernel::StagedTile : cfg.pp ? ConvKernel::TwoPhase : cfg.pw ? ConvKernel::Staged : ConvKernel::Resident;
     cost.config = cfg.name;
-    cost.waves = cfg.waves; cost.pw = cfg.pw; cost.rpw = cfg.rpw; cost.ck = cfg.fold ? 16u : share ? sg.cka : stepChannels(cfg, g.CPAD); cost.mf = cfg.mf; cost.xb = cfg.xb; cost.KT = g.KT; cost.K = conv.K;
+    cost.waves = cfg.waves; cost.pw = cfg.pw; cost.rpw = intoLds ? sg.rpw : cfg.rpw; cost.ck = cfg.fold ? 16u : share || intoLds ? sg.cka : stepChannels(cfg, g.CPAD); cost.mf = cfg.mf; cost.xb = cfg.xb; cost.KT = g.KT; cost.K = conv.K;
     cost.CA = CA; cost.CB = CB; cost.R = conv.R; cost.S = conv.S; cost.SY = conv.strideY; cost.SX = conv.strideX; cost.slots = g.slots;
     cost.cka = cfg.fold ? fg.cka : 0; cost.ksplit = cfg.ksplit; cost.hrot = cfg.hrot; cost.swp = cfg.swp; cost.ntStore = cfg.ntStore;
     cost.blockedIn = blockedIn; cost.blockedOut = blockedOut;

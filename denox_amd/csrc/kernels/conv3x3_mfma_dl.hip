@@ -1,0 +1,265 @@
+// conv3x3_mfma_dl.hip -- 3x3 convolution of one plain source (stride 1, extent kept) with weights and halos streamed straight into LDS.
+//
+// The streaming kernel (conv3x3_mfma.hip) loads a step's weights and halo into registers, writes them to LDS and lets every wave wait at
+// two barriers per step.  Here both go from memory into one of two LDS buffers (buffer_load ... lds) while the other is
+// multiplied: no registers, no LDS writes, one barrier per step, and a persistent workgroup asks for the next tile's first step
+// during the last step of the one before.  The loads are issued one by one between the matrix instructions (a memory instruction waits
+// for room in the memory pipeline; all of a step's at once leave the matrix cores idle), a finished tile is stored in portions during
+// the steps of the next.
+//
+// Mapping: as conv3x3_mfma.hip -- WAVES waves, each RPW rows of 32 pixels for all KT output channels of the workgroup.  The weights lie in
+// memory in the order of the fragments (1 KiB each, lane by lane): their copy is linear and their reads are conflict-free.  A halo pixel
+// takes CK / 8 slots of 16 bytes whose order is rotated by the pixel's column, so that 16 lanes reading the same channels of
+// 16 consecutive pixels hit 16 different bank groups.
+//
+// What bounds it: the LDS-fed matrix rate of the part under load, loads and stores overlapping it only in part (128 -> 64 channels at
+// 1920 x 1088: 257 us, 215 with neither loads nor stores, 800 MB of memory traffic are 156).  Tiles of 32 rows (RPW = 4, two blocks) halve the
+// LDS reads per matrix instruction of tiles of 16, which need steps of 16 channels to fit; those fetch a pixel-major source's lines
+// twice or more, so the large tiles pay on block-major sources (128 -> 64 257 us, pixel-major 313 and with 32-channel steps 277).
+// Microseconds a launch, the best of the other kernels before, block-major or pixel-major source: 96 -> 96 at 960 x 544 95 and 74,
+// 192 -> 192 at 480 x 272 86 and 70, 64 -> 96 pooled at 960 x 544 64 and 50, 128 -> 128 at 960 x 544 151 and 123, 128 -> 64 at 1920 x 1088 310 and 257.
+//
+// Launch: persistent, NXCD * NKT * SLOTS workgroups; a unit of work is (tile, slice of KT output channels), each XCD has a contiguous band.
+#include "conv_common.h"
+
+#ifndef KERNEL_NAME
+#define KERNEL_NAME conv3x3_mfma_dl
+#endif
+#ifndef NXCD
+#define NXCD 8
+#endif
+static_assert(CB == 0 && !UPA && !PADA && !CROP && MF == 32 && PW == 0 && KR == 3 && KS == 3 && PY == 1 && PX == 1 && SY == 1 && SX == 1, "one plain source, 3 x 3, extent kept");
+static_assert(CA % CK == 0 && (CK == 16 || CK == 32 || CK == 64), "whole steps of a power of two of vectors");
+static_assert(KOUT % 8 == 0 && OPITCH % 8 == 0 && OVEC, "two 16-byte stores per pixel and block: the wait for a step's loads counts them");
+
+#define NKT (KOUTP / KT)
+#define G8 (CK / 8)                     // slots per halo pixel
+#define WFRAGS (9 * KB * (CK / 16))     // weight fragments of a step
+#define HGROUPS ((HALO_PIX * G8 + 63) / 64) // halo loads of one wave's 64 lanes
+#define BUF_SLOTS (64 * (WFRAGS + HGROUPS))
+#define NVH ((HGROUPS + WAVES - 1) / WAVES)
+#define DEFER (KB * RPW <= 4)            // the registers hold a converted tile beside the next one's accumulators
+#define NSTORES (KB * OROWS * 2)        // store instructions of a wave per tile
+#define ITEMS (NVH + (WFRAGS + WAVES - 1) / WAVES) // load instructions of a wave per step
+
+extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
+    const _Float16 *__restrict__ A, _Float16 *__restrict__ OUT, const _Float16 *__restrict__ FILT,
+#if HAS_BIAS
+    const _Float16 *__restrict__ BIAS,
+#endif
+    PushConstants pc) {
+  // One LDS object: beside a second one the compiler waits for every load into LDS in front of every LDS read.
+  __shared__ uint4v sBuf[2 * BUF_SLOTS + KOUTP / 4];
+  bias_t *const sBias = (bias_t *)(sBuf + 2 * BUF_SLOTS);
+  const int tid = DNX_TID;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const OutBuf out = out_buffer(OUT, pc);
+  const Sources srcs = make_sources(A, nullptr, pc);
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(A), 0, (int)srcs.bytesA, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(FILT), 0, KOUTP * 9 * CA * 2, 0x00020000);
+  const int W = (int)pc.IN_W, H = (int)pc.IN_H;
+
+  const int tilesX = (W + TW - 1) / TW, tilesY = (H + TH - 1) / TH;
+  const int units = tilesX * tilesY * NKT;
+  const int perXcd = (units + NXCD - 1) / NXCD;
+  const int first = (int)(DNX_BID_X % NXCD) * perXcd;
+  const int last = first + perXcd < units ? first + perXcd : units;
+  int unit = first + (int)(DNX_BID_X / NXCD);
+  if (unit >= last)
+    return; // uniform for the workgroup
+  const bool rev = (pc.FLAGS & 1u) != 0;
+  struct Geo { int kt, x0, y0; };
+  auto geometry = [&](int u) {
+    Geo g;
+    g.kt = u % NKT;
+    int t = u / NKT;
+    t = rev ? tilesX * tilesY - 1 - t : t;
+    const int ty = t / tilesX;
+    g.x0 = (t - ty * tilesX) * TW;
+    g.y0 = ty * TH;
+    return g;
+  };
+
+#if HAS_BIAS
+  for (int i = tid; i < KOUTP; i += NT) sBias[i] = (float)BIAS[i];
+#endif
+
+  // What follows from the lane's number alone is derived again where it is needed rather than kept in registers.
+  auto fresh_lane = [&]() {
+    int l = lane;
+    __asm__ volatile("" : "+v"(l));
+    return l;
+  };
+  // Byte offsets of this lane's halo vectors in the source at channel 0; NO_LOAD outside the image (reads as zero).  From one unit to
+  // the next they move by the same amount where both halos lie inside the image.
+  unsigned hoff[NVH];
+  auto group = [&](int i) { return wv + i * WAVES < HGROUPS ? wv + i * WAVES : HGROUPS - 1; }; // a wave without one left repeats the last
+  auto inside = [&](const Geo &g) { return (g.y0 >= 1) & (g.y0 + HALO_H - 1 <= H) & (g.x0 >= 1) & (g.x0 + HALO_W - 1 <= W); };
+  auto aim = [&](const Geo &g) {
+    const unsigned ln = (unsigned)fresh_lane();
+#pragma unroll
+    for (int i = 0; i < NVH; ++i) {
+      const unsigned slot = (unsigned)group(i) * 64 + ln, pix = slot / G8;
+      unsigned hy = pix / HALO_W;
+      const unsigned hx = pix - hy * HALO_W, grp = (slot - hx / (16 / G8)) & (G8 - 1); // the channel group that belongs into this slot
+      hy = hy < HALO_H ? hy : HALO_H - 1;                                              // past the halo: its last row again
+      const int y = g.y0 - 1 + (int)hy, x = g.x0 - 1 + (int)hx;
+      const unsigned p = (unsigned)(y * W + x);
+      hoff[i] = (((unsigned)y < (unsigned)H) & ((unsigned)x < (unsigned)W)) ? (LAYIN ? p * 16u + grp * srcs.planeA : p * (CA * 2u) + grp * 16u) : NO_LOAD;
+    }
+  };
+  auto move = [&](const Geo &from, const Geo &to) {
+    if (inside(from) & inside(to)) {
+      const unsigned d = (unsigned)((to.y0 - from.y0) * W + to.x0 - from.x0) * (LAYIN ? 16u : CA * 2u);
+#pragma unroll
+      for (int i = 0; i < NVH; ++i) hoff[i] += d;
+    } else
+      aim(to);
+  };
+  auto item = [&](int buf, int kt, int k, int i) { // item i of the loads of the step with the channels from k * CK on
+    if (i < NVH) {
+      const unsigned off = hoff[i] + (LAYIN ? (unsigned)(k * G8) * srcs.planeA : (unsigned)(k * CK * 2));
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void_t *)(sBuf + buf * BUF_SLOTS + (WFRAGS + group(i)) * 64), 16, hoff[i] != NO_LOAD ? off : NO_LOAD, 0, 0, LOAD_AUX);
+    } else {
+      const int q = wv + (i - NVH) * WAVES, f = q < WFRAGS ? q : WFRAGS - 1;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_void_t *)(sBuf + buf * BUF_SLOTS + f * 64), 16, fresh_lane() * 16, ((kt * NCHUNK + k) * WFRAGS + f) * 1024, 0, 0);
+    }
+  };
+#define STEP_WAIT(n) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
+
+  Acc acc;
+  // Holds a step's matrix instructions in front of its barrier (they touch no memory: the compiler may collect several steps' worth behind it).
+  auto pin = [&]() {
+#pragma unroll
+    for (int b = 0; b < KB; ++b)
+#pragma unroll
+      for (int j = 0; j < RPW; ++j) __asm__ volatile("" : "+v"(acc.v[b][j]));
+  };
+  auto step = [&](int buf, auto load) { // load(i): item i of the loads for the next step
+    typedef __attribute__((address_space(3))) const char lds_char_t;
+    typedef __attribute__((address_space(3))) const half8 *lds_frag;
+    constexpr int KSN = CK / 16, NG = 3 * KSN, UNITS = 3 * NG;
+    const int ln = fresh_lane(), l32 = ln & 31, kh = ln >> 5;
+    lds_char_t *wb = (lds_char_t *)lds_opaque((const _Float16 *)(sBuf + buf * BUF_SLOTS + ln)), *pb[3][KSN];
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+#pragma unroll
+      for (int ks = 0; ks < KSN; ++ks) {
+        const int x = l32 + s;
+        pb[s][ks] = (lds_char_t *)lds_opaque((const _Float16 *)(sBuf + buf * BUF_SLOTS + WFRAGS * 64 + (wv * RPW * HALO_W + x) * G8 + ((2 * ks + kh + x / (16 / G8)) & (G8 - 1))));
+      }
+    // A group is a filter column s of one 16-channel slice: RPW + 2 pixel fragments; its three units (one per filter row) read KB weight
+    // fragments and feed KB * RPW matrix instructions.  Weights are read one or two units ahead, a group's pixels during the group before.
+    constexpr int WR = KB <= 2 ? 3 : 2; // weight sets: the one in use and those under way
+    half8 px[2][RPW + 2], w[WR][KB];
+    auto read_w = [&](int u) {
+      const int gr = u / 3, r = u % 3, s = gr / KSN, ks = gr % KSN;
+#pragma unroll
+      for (int b = 0; b < KB; ++b) w[u % WR][b] = *(lds_frag)(wb + (((r * 3 + s) * KB + b) * KSN + ks) * 1024);
+    };
+    auto read_p = [&](int gr, int t) {
+      const int s = gr / KSN, ks = gr % KSN;
+      px[gr & 1][t] = *(lds_frag)(pb[s][ks] + t * (HALO_W * G8 * 16));
+    };
+#pragma unroll
+    for (int t = 0; t < RPW + 2; ++t) read_p(0, t);
+#pragma unroll
+    for (int u = 0; u < WR - 1; ++u) read_w(u);
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+      const int gr = u / 3, r = u % 3;
+      if (u + WR - 1 < UNITS) read_w(u + WR - 1);
+      if (gr + 1 < NG) {
+#pragma unroll
+        for (int t = r * (RPW + 2) / 3; t < (r + 1) * (RPW + 2) / 3; ++t) read_p(gr + 1, t);
+      }
+#pragma unroll
+      for (int i = u * ITEMS / UNITS; i < (u + 1) * ITEMS / UNITS; ++i) load(i);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int b = 0; b < KB; ++b)
+#pragma unroll
+        for (int j = 0; j < RPW; ++j) acc.v[b][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[u % WR][b], px[gr & 1][j + r], acc.v[b][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    pin();
+  };
+
+  int buf = 0;
+  Geo g = geometry(unit);
+#if DEFER
+  Geo gd = g;
+#endif
+  aim(g);
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) item(0, g.kt, 0, i);
+  STEP_WAIT(0);
+  DNX_SYNC();
+#if DEFER
+  // The finished tile, converted; its stores go out in NPARTS portions in front of the next tile's steps (whole output rows: a line filled
+  // in two portions far apart in time is written to memory twice).
+  constexpr int NPARTS = NCHUNK < OROWS ? NCHUNK : OROWS;
+  Packed done;
+  bool pend = false;
+  auto store_part = [&](int part) {
+#pragma unroll
+    for (int p = 0; p < NPARTS; ++p)
+      if (part == p) store_packed(done, out, gd.y0, gd.x0, gd.kt, wv, fresh_lane(), pc, p, NPARTS);
+  };
+#endif
+  for (;;) {
+    const int next = unit + NKT * SLOTS;
+    const bool more = next < last;
+    const Geo gn = geometry(more ? next : unit); // (behind the last unit its own first step is loaded once more and not used)
+#if HAS_BIAS
+    const int hsel = fresh_lane() >> 5;
+#endif
+#pragma unroll
+    for (int b = 0; b < KB; ++b)
+#pragma unroll
+      for (int j = 0; j < RPW; ++j)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+#if HAS_BIAS
+          acc.v[b][j][i] = sBias[g.kt * KT + b * 32 + hsel * 16 + i];
+#else
+          acc.v[b][j][i] = 0.0f;
+#endif
+    for (int k = 0; k < NCHUNK - 1; ++k) {
+#if DEFER
+      if (pend & (k < NPARTS)) store_part(k);
+#endif
+      step(buf, [&](int i) { item(buf ^ 1, g.kt, k + 1, i); });
+      STEP_WAIT(0); // the next step's loads; the stores in front of them have had the step's matrix work to complete
+      DNX_SYNC();
+      buf ^= 1;
+    }
+#if DEFER
+    if (pend & (NCHUNK - 1 < NPARTS)) store_part(NCHUNK - 1);
+#endif
+    move(g, gn);
+    step(buf, [&](int i) { item(buf ^ 1, gn.kt, 0, i); });
+#if DEFER
+    pack_tile(acc, done);
+    STEP_WAIT(0);
+#else
+    store_tile(acc, out, g.y0, g.x0, g.kt, wv, fresh_lane(), pc);
+    STEP_WAIT(NSTORES); // the next unit's first step has landed; the stores behind its loads may still be on their way
+#endif
+    DNX_SYNC();
+    buf ^= 1;
+#if DEFER
+    gd = g;
+    pend = true;
+#endif
+    if (!more)
+      break;
+    unit = next;
+    g = gn;
+  }
+#if DEFER
+#pragma unroll
+  for (int p = 0; p < NPARTS; ++p) store_part(p);
+#endif
+}

@@ -1,0 +1,80 @@
+"""Convolutions whose weights and halos go straight into LDS (conv3x3_mfma_dl.hip) at the edges of what they do: one pixel, one tile and a
+pixel more or less (tiles of 32 columns and 16 or 32 rows), several units per workgroup, one step and many, slices of 32 to 128 output
+channels and channels past the last one, a pooled result of odd extents, a result inside a concat, both layouts of source and result.
+
+Inputs, weights and bias are small integers: every product and partial sum is exact in binary32 (at most 9 * 256 * 2 + 3 < 2^24) and every
+result within 2048 in magnitude is exact in binary16, so the result has the oracle's bits whatever the order of the sums."""
+import numpy as np
+import pytest
+
+import denox_amd as dx
+from util import assert_bits_equal
+
+pytestmark = pytest.mark.gpu
+
+# C, K, H, W, pooled
+SHAPES = [(16, 32, 1, 1, False), (16, 8, 2, 3, True), (32, 64, 16, 32, False), (32, 48, 33, 65, True), (64, 64, 31, 31, False), (64, 96, 34, 66, True), (96, 128, 17, 97, False),
+          (128, 160, 20, 40, True), (112, 112, 65, 33, False), (192, 192, 15, 70, False), (256, 64, 9, 130, False), (64, 64, 300, 420, False), (32, 96, 270, 510, True)]
+
+
+def blocked(x):
+    H, W, C = x.shape
+    return np.ascontiguousarray(x.reshape(H, W, C // 8, 8).transpose(2, 0, 1, 3))
+
+
+def planar(y):
+    g, H, W, _ = y.shape
+    return y.transpose(1, 2, 0, 3).reshape(H, W, g * 8)
+
+
+def is_this_kernel(d):
+    return d["workgroup_count"][1:] == [1, 1] and "SLOTS=" in d["debug_info"] and "WAVES=8" in d["debug_info"] and "UPA=0" in d["debug_info"]
+
+
+@pytest.mark.parametrize("config", ["w8r2k32", "w8r2k16"])
+@pytest.mark.parametrize("C,K,H,W,pooled", SHAPES)
+def test_streamed_into_lds_equals_the_definition(oracle, config, C, K, H, W, pooled):
+    rng = np.random.default_rng(C + K + H)
+    m = dx.Model()
+    t = m.conv2d(m.input("x", "W", "H", C), rng.choice([-1, 0, 0, 0, 1], (K, C, 3, 3)).astype(np.float16), rng.integers(-3, 4, K).astype(np.float16))
+    t = m.activation(t, "leaky_relu", 0.5) if K % 64 else m.relu(t)
+    if pooled:
+        t = m.pool(t)
+    m.output(t, "out")
+    x = rng.integers(-2, 3, (H, W, C)).astype(np.float16)
+    want = oracle.run_graph(m.to_ops({"H": H, "W": W}), {"x": x}, "fp32")[t.name]
+    assert np.abs(want).max(initial=0) < 1024  # (a leaky slope of 1/2 leaves at most one bit below 1)
+    ran = 0
+    for blocked_in in (False, True):
+        for blocked_out in (False, True):
+            layouts = dict(input_layout=dx.Layout.CHWC8 if blocked_in else dx.Layout.HWC, output_layout=dx.Layout.CHWC8 if blocked_out else dx.Layout.HWC)
+            try:
+                blob = dx.compile_model(m, conv_config=config, assume={"H": H, "W": W}, **layouts)
+            except dx.DenoxHipError as e:
+                assert e.status == 5
+                continue
+            if not any(is_this_kernel(d) for d in dx.describe(blob, H=H, W=W)["dispatches"]):
+                continue
+            got = dx.Module.load(blob).instance(H=H, W=W).infer(blocked(x) if blocked_in else x)[0]
+            assert_bits_equal(planar(got) if blocked_out else got, want.astype(np.float16), f"{config} {layouts}")
+            ran += 1
+    if not ran:
+        assert C % int(config[-2:])  # whole steps only
+        pytest.skip("not this kernel: no whole steps of channels")
+
+
+def test_result_inside_a_concat(oracle):
+    """The concat's sources written in place: a pixel pitch of two tensors, 16-byte aligned at the second one's first channel."""
+    rng = np.random.default_rng(5)
+    H, W = 35, 68
+    m = dx.Model()
+    x = m.input("x", "W", "H", 32)
+    conv = lambda k: m.relu(m.conv2d(x, rng.choice([-1, 0, 0, 1], (k, 32, 3, 3)).astype(np.float16), rng.integers(-3, 4, k).astype(np.float16)))  # noqa: E731
+    t = m.concat(conv(64), conv(40))
+    m.output(t, "out")
+    v = rng.integers(-2, 3, (H, W, 32)).astype(np.float16)
+    want = oracle.run_graph(m.to_ops({"H": H, "W": W}), {"x": v}, "fp32")[t.name]
+    for config in ("w8r2k32", "w8r2k16"):
+        blob = dx.compile_model(m, conv_config=config, assume={"H": H, "W": W})
+        assert sum(is_this_kernel(d) for d in dx.describe(blob, H=H, W=W)["dispatches"]) == 2
+        assert_bits_equal(dx.Module.load(blob).instance(H=H, W=W).infer(v)[0], want.astype(np.float16), config)
