@@ -82,14 +82,17 @@ double share_cost_us(const ConvCost &c, double ow, double oh, double bytes, unsi
 // Streaming kernels whose weights and halos go straight into LDS (conv3x3_mfma_dl.hip), one form as well: matrix instructions, LDS reads and
 // loads of a unit of work overlap, a pixel-major result leaves the lanes in short pieces, and steps of 16 channels fetch a
 // pixel-major source's lines more than once.  Fitted to 1632 launches of 15 layers (16 to 256 channels, with and without a pool) at
-// 96 x 64 to 1920 x 1088 in all layouts: measured over estimated 0.88 - 1.14 for nine of ten, median 1.00.
+// 96 x 64 to 1920 x 1088 in all layouts: measured over estimated 0.88 - 1.14 for nine of ten, median 1.00.  (5 x 5 with stride 2, 32 and 64 -> 64 channels at
+// 480 x 270 to 1920 x 1080: 0.92 - 1.27; the price of short pieces is four times as high there, every pixel lies in a phase of its own.)
 double streamed_lds_cost_us(const ConvCost &c, double ow, double oh, double bytesRead, double bytesWritten, unsigned xcds) {
   const double kb = c.KT / 32, rows = 8.0 * c.rpw, slices = cdiv(cdiv(c.K, 32) * 32, c.KT), groups = c.CA / 16.0;
   const double rounds = cdiv(cdiv(cdiv(ow, 32) * cdiv(oh, rows) * slices, xcds), c.slots * slices);
-  const double matrix = 0.865 * 9 * groups * kb * c.rpw * 2 * 32 / 2000, lds = 3.235e-3 * 8 * 3 * groups * (c.rpw + 2 + 3 * kb);
-  const double haloKB = (rows + 2) * 34 * c.CA * 2 / 1024, loads = 2.035e-2 * (haloKB + 9.0 * c.KT * c.CA * 2 / 1024);
+  // (a strided layer's taps fall into phases that each stage a halo of their own)
+  const double taps = c.R * c.S, phases = c.SY * c.SX, nr = cdiv(c.R, c.SY), nc = cdiv(c.S, c.SX);
+  const double matrix = 0.865 * taps * groups * kb * c.rpw * 2 * 32 / 2000, lds = 3.235e-3 * 8 * groups * (c.S * c.SY * (c.rpw - 1 + c.R / static_cast<double>(c.SY)) + taps * kb);
+  const double haloKB = phases * (rows + nr - 1) * (32 + nc - 1) * c.CA * 2 / 1024, loads = 2.035e-2 * (haloKB + taps * c.KT * c.CA * 2 / 1024);
   const double stored = bytesWritten / std::max(1.0, 2 * ow * oh * c.K), tileKB = rows * 32 * c.KT * 2 / 1024 * stored; // (a pooled tile is a quarter)
-  const double unit = std::sqrt(matrix * matrix + lds * lds + loads * loads) + 0.0371 * c.CA / c.ck + (c.ck == 16 && !c.blockedIn ? 0.0036 * haloKB : 0) + (c.blockedOut ? 0 : 0.0141 * tileKB);
+  const double unit = std::sqrt(matrix * matrix + lds * lds + loads * loads) + 0.0371 * phases * c.CA / c.ck + (c.ck == 16 && !c.blockedIn ? (phases > 1 ? 0.0144 : 0.0036) * haloKB : 0) + (c.blockedOut ? 0 : 0.0141 * tileKB);
   const double memory = (bytesRead + bytesWritten) / 5.712e6;
   return kLaunchUs + std::pow(std::pow(rounds * unit, 1.2) + std::pow(memory, 1.2), 1 / 1.2);
 }

@@ -325,7 +325,7 @@ std::vector<uint8_t> packFoldWeights(const Op &conv, const FoldGeometry &g) {
 
 // ---- products of an upsampled source shared between the outputs (conv3x3_upshare.hip) ------------------------------
 struct ShareGeometry {
-  unsigned CA, CB, CAP, CBP, K, KOUTP, KT, cka, slots, rpw;
+  unsigned CA, CB, CAP, CBP, K, KOUTP, KT, cka, slots;
 };
 
 // Whether a configuration of a layer over an upsampled source is that kernel, and its geometry.
@@ -336,7 +336,7 @@ bool chooseShare(const ConvConfig &cfg, const Op &conv, unsigned pattern, unsign
   // whole vectors of A; B's partial last vector is read ending at its last channel; two 16-byte stores per accumulator
   if (CA % 8 || (CB > 0 && CB < 8) || K % 8) return false;
   g.CA = CA; g.CB = CB; g.CAP = (CA + 15) / 16 * 16; g.CBP = CB ? (CB + 15) / 16 * 16 : 0; g.K = K; g.KOUTP = (K + 31) / 32 * 32;
-  g.cka = g.CAP % 32 ? 16 : 32; g.rpw = cfg.rpw;
+  g.cka = g.CAP % 32 ? 16 : 32;
   if (cfg.rpw == 2 && cfg.ck != g.cka) return false;
   for (unsigned kt = std::min(g.KOUTP, cfg.maxKT ? cfg.maxKT : 64u); kt >= 32; kt -= 32) {
     const unsigned kb = kt / 32;
@@ -379,22 +379,58 @@ std::vector<uint8_t> packShareWeights(const Op &conv, const ShareGeometry &g) {
   return bytes;
 }
 
-// The streaming configurations of 8 waves on a plain source of whole steps are conv3x3_mfma_dl.hip; its geometry in the same form (CB = 0).
-bool chooseStreamedLds(const ConvConfig &cfg, const Op &conv, unsigned pattern, unsigned CA, unsigned CB, const DeviceInfo &dev, ShareGeometry &g) {
+// ---- weights and halos straight into LDS (conv3x3_mfma_dl.hip) -------------------------------------------------------
+// The streaming configurations of 8 waves on a plain source of whole steps of channels.  A strided layer's taps fall into phases (see the
+// kernel); where they have fewer than four taps on average a step is shorter than its barrier and its loads are worth, and the
+// kernel that takes all taps at once stays.
+struct StreamedLdsGeometry {
+  unsigned K, KOUTP, KT, ck, slots, rpw;
+};
+
+bool chooseStreamedLds(const ConvConfig &cfg, const Op &conv, unsigned pattern, unsigned CA, unsigned CB, const DeviceInfo &dev, StreamedLdsGeometry &g) {
   if (cfg.resident || cfg.fold || cfg.mf != 32 || cfg.waves != 8 || cfg.rpw != 2 || (cfg.ck != 16 && cfg.ck != 32)) return false;
-  if ((pattern & ~(PAT_ACT | PAT_POOL)) || CB || conv.R != 3 || conv.S != 3 || conv.padX != 1 || conv.padY != 1 || conv.strideX != 1 || conv.strideY != 1) return false;
+  const unsigned R = conv.R, S = conv.S, sy = conv.strideY, sx = conv.strideX;
+  if ((pattern & ~(PAT_ACT | PAT_POOL)) || CB || sy > 2 || sx > 2 || R < sy || S < sx || R * S < 4 * sy * sx) return false;
   if (CA % cfg.ck || conv.K % 8) return false;
-  g.CA = g.CAP = CA; g.CB = g.CBP = 0; g.K = conv.K; g.KOUTP = (conv.K + 31) / 32 * 32; g.cka = cfg.ck;
+  g.K = conv.K; g.KOUTP = (conv.K + 31) / 32 * 32; g.ck = cfg.ck;
+  const unsigned nr = (R + sy - 1) / sy, nc = (S + sx - 1) / sx; // taps of the largest phase
   for (unsigned kt = std::min(g.KOUTP, 128u); kt >= 32; kt -= 32) {
     if (g.KOUTP % kt) continue;
     g.rpw = cfg.ck == 16 && kt <= 64 ? 4 : 2; // (with 16 channels a step's halo leaves room for tiles of 32 rows)
-    const size_t lds = 2u * 1024u * (9 * (kt / 32) * (cfg.ck / 16) + ((8 * g.rpw + 2) * 34 * (cfg.ck / 8) + 63) / 64) + 4u * g.KOUTP;
-    if (lds > dev.maxComputeSharedMemory) continue;
-    g.KT = kt;
-    g.slots = std::max(1u, dev.computeUnits / (dev.xcdCount * (g.KOUTP / kt)));
-    return true;
+    for (; g.rpw >= 2; g.rpw -= 2) {
+      const size_t lds = 2u * 1024u * (nr * nc * (kt / 32) * (cfg.ck / 16) + ((8 * g.rpw + nr - 1) * (32 + nc - 1) * (cfg.ck / 8) + 63) / 64) + 4u * g.KOUTP;
+      if (lds > dev.maxComputeSharedMemory) continue;
+      g.KT = kt;
+      g.slots = std::max(1u, dev.computeUnits / (dev.xcdCount * (g.KOUTP / kt)));
+      return true;
+    }
   }
   return false;
+}
+
+// [slice of KT channels][phase][step of ck channels][tap of the phase][32-channel block][16 channels] in fragments of 64 lanes x 8 halves: lane
+// l holds channels (l / 32) * 8 .. of weight row l % 32.
+std::vector<uint8_t> packStreamedLdsWeights(const Op &conv, const StreamedLdsGeometry &g) {
+  std::vector<uint16_t> out(static_cast<size_t>(g.KOUTP) * conv.R * conv.S * conv.C, 0);
+  size_t pos = 0;
+  for (unsigned kt = 0; kt < g.KOUTP / g.KT; ++kt)
+    for (unsigned py = 0; py < conv.strideY; ++py)
+      for (unsigned px = 0; px < conv.strideX; ++px)
+        for (unsigned c0 = 0; c0 < conv.C; c0 += g.ck)
+          for (unsigned r = (py + conv.padY) % conv.strideY; r < conv.R; r += conv.strideY)
+            for (unsigned s = (px + conv.padX) % conv.strideX; s < conv.S; s += conv.strideX)
+              for (unsigned kb = 0; kb < g.KT / 32; ++kb)
+                for (unsigned ks = 0; ks < g.ck / 16; ++ks)
+                  for (unsigned lane = 0; lane < 64; ++lane) {
+                    const unsigned k = kt * g.KT + rowChannel(32, g.KT, kb * 32 + lane % 32);
+                    for (unsigned e = 0; e < 8; ++e, ++pos) {
+                      const unsigned c = c0 + ks * 16 + lane / 32 * 8 + e;
+                      if (k < g.K) out[pos] = conv.weights[((static_cast<size_t>(k) * conv.C + c) * conv.R + r) * conv.S + s];
+                    }
+                  }
+  std::vector<uint8_t> bytes(out.size() * 2);
+  std::memcpy(bytes.data(), out.data(), bytes.size());
+  return bytes;
 }
 
 bool isPairConfigName(const std::string &name); // a configuration of the conv -> conv shader below
@@ -553,7 +589,8 @@ public:
       }
       if (m.blocked()) {
         ShareGeometry sg;
-        if (!offeredBlocked(cfg) && !sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg) && !streamsIntoLds(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg)) continue;
+        StreamedLdsGeometry lg;
+        if (!offeredBlocked(cfg) && !sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg) && !streamsIntoLds(cfg, conv, model, m, CA, CB, opt.deviceInfo, lg)) continue;
         // block-major sources are read through the per-step buffer resource: every LDS step must lie in one source
         if (!m.inputFormats.empty() && m.inputFormats[0] && CB && CA % stepChannels(cfg, cpad)) continue;
       }
@@ -564,7 +601,8 @@ public:
       ConvGeometry g;
       g.R = conv.R; g.S = conv.S; g.SY = conv.strideY; g.SX = conv.strideX;
       ShareGeometry sg;
-      if (!sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg) && !streamsIntoLds(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg) && !chooseKT(cfg, CA, CB, conv.K, opt.deviceInfo, g)) continue;
+      StreamedLdsGeometry lg;
+      if (!sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg) && !streamsIntoLds(cfg, conv, model, m, CA, CB, opt.deviceInfo, lg) && !chooseKT(cfg, CA, CB, conv.K, opt.deviceInfo, g)) continue;
       out.push_back(c);
     }
     bool forcedFold = false; // a forced upsample-folding configuration leaves matches without an upsample to nobody: not an error
@@ -582,7 +620,7 @@ public:
     if (m.blocked() && !m.inputFormats.empty() && m.inputFormats[0] && CB && (CA % 16 || CB % 8)) return false;
     return chooseShare(cfg, conv, m.pattern, CA, CB, dev, g);
   }
-  static bool streamsIntoLds(const ConvConfig &cfg, const Op &conv, const Model &model, const Match &m, unsigned CA, unsigned CB, const DeviceInfo &dev, ShareGeometry &g) {
+  static bool streamsIntoLds(const ConvConfig &cfg, const Op &conv, const Model &model, const Match &m, unsigned CA, unsigned CB, const DeviceInfo &dev, StreamedLdsGeometry &g) {
     if (m.outputVariant) { // whole 16-byte stores
       const ConcatView v = concatViewOf(model, m.output);
       if (!v.valid || v.pitch % 8 || v.channelOffset % 8) return false;
@@ -607,8 +645,11 @@ public:
     g.R = conv.R; g.S = conv.S; g.SY = conv.strideY; g.SX = conv.strideX;
     FoldGeometry fg{};
     ShareGeometry sg{};
-    const bool share = sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg), intoLds = !share && streamsIntoLds(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg);
-    if (share || intoLds) {
+    StreamedLdsGeometry lg{};
+    const bool share = sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg), intoLds = !share && streamsIntoLds(cfg, conv, model, m, CA, CB, opt.deviceInfo, lg);
+    if (intoLds) {
+      g.CA = CA; g.CB = 0; g.C = g.CPAD = CA; g.K = conv.K; g.KOUTP = lg.KOUTP; g.KT = lg.KT; g.slots = lg.slots;
+    } else if (share) {
       g.CA = CA; g.CB = CB; g.C = CA + CB; g.K = conv.K; g.KOUTP = sg.KOUTP; g.KT = sg.KT; g.slots = sg.slots; g.CPAD = sg.CAP + sg.CBP;
     } else if (cfg.fold) {
       if (!chooseFold(cfg, CA, CB, conv.K, opt.deviceInfo, fg)) fail(Status::Internal, "conv config rejected at implement time");
@@ -641,7 +682,7 @@ public:
     if (padA) k.define("PADA", 1);
     if (padB) k.define("PADB", 1);
     if (crop) k.define("CROP", 1);
-    k.define("WAVES", cfg.waves); k.define("RPW", intoLds ? sg.rpw : cfg.rpw); k.define("CK", cfg.fold || share ? 16u : stepChannels(cfg, g.CPAD));
+    k.define("WAVES", cfg.waves); k.define("RPW", intoLds ? lg.rpw : cfg.rpw); k.define("CK", cfg.fold || share ? 16u : stepChannels(cfg, g.CPAD));
     if (cfg.resident || share || intoLds) { k.define("SLOTS", g.slots); k.define("NXCD", opt.deviceInfo.xcdCount); } // the grid below is xcdCount * nkt * slots workgroups
     if (cfg.pw) k.define("PW", cfg.pw);
     if (cfg.pp) k.define("PP", 1);
@@ -681,7 +722,8 @@ public:
     } else d.addBinding(dnx::Access::WriteOnly, m.output);
     const Op convCopy = conv; // the lazy packers outlive the model reference
     const unsigned ck = cfg.resident ? g.CPAD : stepChannels(cfg, g.CPAD);
-    TensorId wt = share || intoLds ? impl.createParameter(static_cast<size_t>(sg.KOUTP) * 9 * (sg.CAP + sg.CBP) * 2, dnx::ScalarType::F16,
+    TensorId wt = intoLds ? impl.createParameter(static_cast<size_t>(lg.KOUTP) * conv.R * conv.S * CA * 2, dnx::ScalarType::F16, [convCopy, lg]() { return packStreamedLdsWeights(convCopy, lg); })
+                : share ? impl.createParameter(static_cast<size_t>(sg.KOUTP) * 9 * (sg.CAP + sg.CBP) * 2, dnx::ScalarType::F16,
                                                    [convCopy, sg]() { return packShareWeights(convCopy, sg); })
                 : cfg.fold ? impl.createParameter(static_cast<size_t>(4) * fg.KOUTP * (4 * fg.CAP + 9 * fg.CBP) * 2, dnx::ScalarType::F16,
                                                   [convCopy, fg]() { return packFoldWeights(convCopy, fg); })
@@ -736,7 +778,7 @@ public:
     cost.valid = true;
     cost.kernel = share ? ConvKernel::Share : intoLds ? ConvKernel::StreamedLds : cfg.fold ? (cfg.pw ? ConvKernel::FoldStaged : ConvKernel::Fold) : !cfg.resident ? ConvKernel::Streamed : cfg.ostage ? ConvKernel::StagedTile : cfg.pp ? ConvKernel::TwoPhase : cfg.pw ? ConvKernel::Staged : ConvKernel::Resident;
     cost.config = cfg.name;
-    cost.waves = cfg.waves; cost.pw = cfg.pw; cost.rpw = intoLds ? sg.rpw : cfg.rpw; cost.ck = cfg.fold ? 16u : share || intoLds ? sg.cka : stepChannels(cfg, g.CPAD); cost.mf = cfg.mf; cost.xb = cfg.xb; cost.KT = g.KT; cost.K = conv.K;
+    cost.waves = cfg.waves; cost.pw = cfg.pw; cost.rpw = intoLds ? lg.rpw : cfg.rpw; cost.ck = cfg.fold ? 16u : share ? sg.cka : intoLds ? lg.ck : stepChannels(cfg, g.CPAD); cost.mf = cfg.mf; cost.xb = cfg.xb; cost.KT = g.KT; cost.K = conv.K;
     cost.CA = CA; cost.CB = CB; cost.R = conv.R; cost.S = conv.S; cost.SY = conv.strideY; cost.SX = conv.strideX; cost.slots = g.slots;
     cost.cka = cfg.fold ? fg.cka : 0; cost.ksplit = cfg.ksplit; cost.hrot = cfg.hrot; cost.swp = cfg.swp; cost.ntStore = cfg.ntStore;
     cost.blockedIn = blockedIn; cost.blockedOut = blockedOut;

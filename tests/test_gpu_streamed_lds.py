@@ -63,6 +63,34 @@ def test_streamed_into_lds_equals_the_definition(oracle, config, C, K, H, W, poo
         pytest.skip("not this kernel: no whole steps of channels")
 
 
+# filter, stride, padding (y, x), C, K, H, W: phases of unequal taps, padding past the image, extents that leave a phase a row or column short
+STRIDED = [((5, 5), (2, 2), (2, 2), 32, 64, 45, 131), ((5, 5), (1, 1), (2, 2), 16, 40, 20, 70), ((4, 4), (2, 2), (1, 1), 32, 32, 34, 66), ((7, 3), (2, 1), (3, 0), 16, 64, 41, 37),
+           ((3, 7), (1, 2), (5, 2), 32, 96, 18, 140), ((2, 2), (1, 1), (0, 0), 48, 128, 33, 33), ((5, 5), (2, 2), (0, 4), 64, 48, 5, 40)]
+
+
+@pytest.mark.parametrize("config", ["w8r2k32", "w8r2k16"])
+@pytest.mark.parametrize("filt,stride,pad,C,K,H,W", STRIDED)
+def test_strides_and_filters(oracle, config, filt, stride, pad, C, K, H, W):
+    rng = np.random.default_rng(sum(filt) + C + K)
+    m = dx.Model()
+    t = m.relu(m.conv2d(m.input("x", "W", "H", C), rng.choice([-1, 0, 0, 0, 1], (K, C) + filt).astype(np.float16), rng.integers(-3, 4, K).astype(np.float16), stride=stride, padding=pad))
+    m.output(t, "out")
+    x = rng.integers(-2, 3, (H, W, C)).astype(np.float16)
+    want = oracle.run_graph(m.to_ops({"H": H, "W": W}), {"x": x}, "fp32")[t.name]
+    assert np.abs(want).max(initial=0) < 2048
+    for blocked_in in (False, True):
+        layout = dx.Layout.CHWC8 if blocked_in else dx.Layout.HWC
+        try:
+            blob = dx.compile_model(m, conv_config=config, assume={"H": H, "W": W}, input_layout=layout)
+        except dx.DenoxHipError as e:
+            assert e.status == 5 and C % int(config[-2:])
+            pytest.skip("not this kernel: no whole steps of channels")
+        if not any(is_this_kernel(d) for d in dx.describe(blob, H=H, W=W)["dispatches"]):
+            assert C % int(config[-2:])
+            pytest.skip("not this kernel: no whole steps of channels")
+        assert_bits_equal(dx.Module.load(blob).instance(H=H, W=W).infer(blocked(x) if blocked_in else x)[0], want.astype(np.float16), f"{config} {layout}")
+
+
 def test_result_inside_a_concat(oracle):
     """The concat's sources written in place: a pixel pitch of two tensors, 16-byte aligned at the second one's first channel."""
     rng = np.random.default_rng(5)
