@@ -240,7 +240,12 @@ Instance::Instance(ModelHandle model, const std::vector<ValueSpec> &specs) : m_m
     }
     m_boundInputs.assign(m.inputs.size(), nullptr);
     m_boundOutputs.assign(m.outputs.size(), nullptr);
-    m_useGraph = !std::getenv("DENOX_HIP_NO_GRAPH");
+    // Replaying a graph costs the host 16 us and the GPU a gap of 5 us however few dispatches it holds; a plain launch costs the
+    // host 2.6 us of its own.  Passes back to back over layers of 2 us each, graph against plain launches: 2 dispatches 16.1 and
+    // 7.5 us, 4 17.4 and 12.3, 8 21.6 both, 16 34.8 and 43.5; one pass that is waited for: 2 dispatches 32 and 17 us, 4 37 and 21,
+    // 8 39 and 52.  Longer layers hide the launches, but a waited-for pass still starts later from 8 on (8 layers of 3 us: 43 and 52).
+    constexpr size_t kPlainLaunches = 4;
+    m_useGraph = m_launches.size() > kPlainLaunches && !std::getenv("DENOX_HIP_NO_GRAPH");
     if (m_useGraph) selectGraph();
   } catch (...) {
     freeBuffers();
@@ -331,7 +336,7 @@ void Instance::launchAll(hipStream_t s) {
 
 void Instance::buildGraph() {
   // Whole-network capture: one graph launch per frame instead of one driver
-  // call per dispatch.
+  // call per dispatch (instances of more than a few dispatches).
   hipStream_t s = m_model->context()->stream();
   hipCheck(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
   try {

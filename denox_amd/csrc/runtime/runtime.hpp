@@ -10,7 +10,8 @@
 // addresses in (set, binding) order followed by the push-constant bytes, all
 // launches in program order on a single stream (which makes the reference's
 // barrier insertion, model.cpp:247-340, unnecessary), and the whole dispatch
-// list captured once per Instance into a hipGraph.
+// list captured once per Instance into a hipGraph (lists of a few dispatches
+// are launched one by one, which is cheaper).
 #pragma once
 #include "../common/dnx.hpp"
 #include "host_staging.hpp"

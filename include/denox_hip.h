@@ -273,7 +273,7 @@ int denox_hip_instance_infer_many(denox_hip_instance *inst, uint32_t frames, con
 int denox_hip_host_alloc(size_t bytes, void **out);
 void denox_hip_host_free(void *p);
 /* asynchronous on the context's stream; device arrays, entries (or the arrays
- * themselves) may be NULL to use the instance's own tensors.  The dispatch list is captured into a graph once per set of
+ * themselves) may be NULL to use the instance's own tensors.  A list of more than four dispatches is captured into a graph once per set of
  * interface addresses and the graphs of the last four sets are kept: a caller that rotates through more than four sets of
  * buffers pays a stream synchronisation and a new capture per call (keep to four, or copy into fixed buffers). */
 int denox_hip_instance_infer_device(denox_hip_instance *inst, const void *const *dev_inputs, void *const *dev_outputs);
