@@ -71,12 +71,15 @@ double cdiv(double a, double b) { return std::ceil(a / b); }
 // fragments behind it, loads that arrive late), the result's way out -- against the launch's memory traffic.  Fitted to 614 launches
 // of 12 layers (32 to 224 upsampled, 0 to 128 other channels, 16 to 224 outputs) at 96 x 64 to 1920 x 1088 in all layouts: measured over
 // estimated 0.89 - 1.16 for nine of ten, median 1.00.
+// (Its long straight-line code starts from cold instruction caches in a frame, which launches back to back do not show: 64 + 9 -> 64 at
+// 256 x 192 takes 12.6 us inside the U-Net, 11.0 without this.)
+constexpr double kShareStartUs = 1.6;
 double share_cost_us(const ConvCost &c, double ow, double oh, double bytes, unsigned xcds) {
   const double cap = cdiv(c.CA, 16) * 16, cbp = cdiv(c.CB, 16) * 16, rows = c.waves / (c.KT / 32) * c.rpw, slices = cdiv(cdiv(c.K, 32) * 32, c.KT);
   const double units = cdiv(ow, 62) * cdiv(oh + 1, 2 * rows) * slices, rounds = cdiv(cdiv(units, xcds), c.slots * slices);
   const double mfma = cap / 16 * (9 * c.rpw + 3) + cbp / 16 * 36 * c.rpw, steps = cap / c.ck + cbp / 16, tileKB = 2 * rows * 62 * c.KT * 2 / 1024;
   const double work = rounds * (1.03 * mfma * 2 * 32 / 2000 + 0.506 * steps + 0.0142 * tileKB), memory = bytes / 5.183e6;
-  return kLaunchUs + std::sqrt(work * work + memory * memory);
+  return kLaunchUs + kShareStartUs + std::sqrt(work * work + memory * memory);
 }
 
 // Streaming kernels whose weights and halos go straight into LDS (conv3x3_mfma_dl.hip), one form as well: matrix instructions, LDS reads and
