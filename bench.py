@@ -3,7 +3,8 @@
 
 A "step" is one whole-network inference of one synthetic frame that is already
 resident in HBM (device pointers in, device pointer out), launched through the
-C ABI (denox_hip_instance_infer_device) as one hipGraph on the library's stream.
+C ABI (denox_hip_instance_infer_device) on the library's stream: one hipGraph, or plain
+launches where the schedule has at most four dispatches.
 
 Prints ONE JSON line: Mpix/s (= 1920*1080 / time per frame) with ms/frame in
 `ms_per_step`, a `roofline` object for the dominant kernel (per-dispatch
@@ -410,7 +411,7 @@ def measure(args, workload: str, steps: int, warmup: int, brief: bool):
         "metric": "oidn_unet_fp16_hwc_1080p_throughput" if workload == "oidn_1080p" else f"{workload}_throughput", "value": H * W / (ms * 1e-3) * 1e-6, "unit": "Mpix/s",
         "n_gpus": 1, "steps": steps, "warmup": warmup, "ms_per_step": ms, "higher_is_better": True, "scaling": "weak",
         "vs_baseline": None, "dtype": "f16", "data": "synthetic",
-        "config": {"workload": f"{description}; {mod.runtime_model.dispatch_count} dispatches in one hipGraph", "device_bytes": inst.device_bytes,
+        "config": {"workload": f"{description}; {mod.runtime_model.dispatch_count} dispatches {'in one hipGraph' if mod.runtime_model.dispatch_count > 4 else 'as plain launches'}", "device_bytes": inst.device_bytes,
                    "schedule": "min-cost over measured dispatch latencies" if db is not None else "min-cost over roofline estimates",
                    "tuning_seconds": round(tune_s, 2), "host_pointer_path_ms_per_frame": round(host_ms, 3), "host_pointer_pipelined_ms_per_frame": round(pipelined_ms, 3),
                    "two_frames_in_flight_ms_per_frame": round(two_ms, 4) if two_ms else None,
