@@ -400,8 +400,10 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
     // piece q: pixel 16 q + lane / 4, group lane % 4, or pixel lane, group q
     const unsigned rd = LAYOUT_OUT ? (unsigned)((ln >> 2) * 256 + (((ln & 3) * 4) ^ (ln >> 2)) * 16) : (unsigned)((ln >> 4) * 256 + ((ln & 15) ^ (ln >> 4)) * 16);
     const int y = 2 * (g.y0 + rg * RPW) + 1 + r;
-    const OutBuf to = (unsigned)y < pc.IN_H ? out : nowhere;
-    const int rowBytes = (int)((unsigned)y * pc.IN_W * (LAYOUT_OUT ? 16u : OPITCH * 2u));
+    // (no scalar offset outside either: a range check of `size - scalar offset` would wrap for a size of 0)
+    const bool inside = (unsigned)y < pc.IN_H;
+    const OutBuf to = inside ? out : nowhere;
+    const int rowBytes = inside ? (int)((unsigned)y * pc.IN_W * (LAYOUT_OUT ? 16u : OPITCH * 2u)) : 0;
     uint4v v[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) v[q] = *(lds_slot_t *)(size_t)(row + (LAYOUT_OUT ? rd ^ (q * 16u) : (rd ^ (q * 64u)) + q * 1024u));

@@ -93,3 +93,26 @@ def test_not_a_number_reaches_its_neighbours_only(config):
     want[13:17, 61:65] = True  # source pixel (7, 31) is outputs 14 - 15 x 62 - 63, and one more on each side
     want[19:22, 61:64] = True
     assert (bad == want).all(), np.argwhere(bad != want)[:8]
+
+
+@pytest.mark.parametrize("config", ["w8r2k32", "w8r1k16"])
+@pytest.mark.parametrize("blocked_out", [False, True])
+def test_rows_outside_the_image_are_not_written(config, blocked_out):
+    """Every first tile computes the row in front of the image and most last tiles rows behind it: with the result in the middle of a
+    larger buffer, nothing around it changes."""
+    torch = pytest.importorskip("torch")
+    H, W, K = 38, 70, 64
+    m, t, feeds = layer(64, 9, K, H, W, False, np.random.default_rng(4))
+    blob = dx.compile_model(m, conv_config=config, assume={"H": H, "W": W}, output_layout=dx.Layout.CHWC8 if blocked_out else dx.Layout.HWC)
+    assert any("UPA=1" in d["debug_info"] and "CKA=" in d["debug_info"] for d in dx.describe(blob, H=H, W=W)["dispatches"])
+    inst = dx.Module.load(blob).instance(H=H, W=W)
+    want = inst.infer(feeds["lo"], feeds["x"])[0].reshape(-1).view(np.int16)
+    size, margin = H * W * K, 40 * W * K  # (more than the tiles' rows past the image, as planes or as whole pixels)
+    buf = torch.full((size + 2 * margin,), 0x5A5A, dtype=torch.int16, device="cuda")
+    d_in = [torch.from_numpy(feeds[k]).cuda() for k in ("lo", "x")]
+    torch.cuda.synchronize()
+    inst.infer_device([d.data_ptr() for d in d_in], [buf.data_ptr() + 2 * margin])
+    inst.synchronize()
+    got = buf.cpu().numpy()
+    assert (got[:margin] == 0x5A5A).all() and (got[margin + size:] == 0x5A5A).all()
+    np.testing.assert_array_equal(got[margin:margin + size], want)
