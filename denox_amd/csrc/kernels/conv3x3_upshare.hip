@@ -69,6 +69,14 @@ static_assert(CAP % CKA == 0 && (CKA == 16 || CKA == 32 || CKA == 64), "whole st
 #define NSTORES (OUT_ROWS * 4)        // store instructions of a wave per tile
 static_assert(NSTORES <= 63, "the wait's counter");
 
+// Between LDS accesses of one wave whose lanes read what other lanes wrote: the hardware serves them in order, and here the compiler
+// keeps that order too (it reasons lane by lane and may exchange accesses that never meet in one lane).  No instruction comes of it.
+__device__ DNX_INLINE void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // x - 1's value: lane i receives lane i - 1's (lanes 0 and 32 hold the pixel that only supplies its edge)
 __device__ DNX_INLINE float from_prev_lane(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, true)); // wave_shr:1
@@ -388,6 +396,7 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
     const unsigned row = (unsigned)(size_t)(lds_byte_t *)(__attribute__((address_space(3))) void *)(sRow + wv * 256);
     // byte address of pixel 2 l32, group 2 (lane / 32); pixel 2 l32 + b and group + e are at its XOR with 64 b + 16 e
     const unsigned wr = (unsigned)((l32 >> 1) * 256 + ((((l32 & 1) * 8 + (ln >> 5) * 2) ^ (l32 >> 1)) * 16));
+    wave_lds_order(); // the row before has been read
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
       float v[16];
@@ -397,6 +406,7 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
 #pragma unroll
       for (int e = 0; e < 2; ++e) *(lds_slot_t *)(size_t)(row + (wr ^ (b * 64u + e * 16u))) = __builtin_bit_cast(uint4v, h[e]);
     }
+    wave_lds_order();
     // piece q: pixel 16 q + lane / 4, group lane % 4, or pixel lane, group q
     const unsigned rd = LAYOUT_OUT ? (unsigned)((ln >> 2) * 256 + (((ln & 3) * 4) ^ (ln >> 2)) * 16) : (unsigned)((ln >> 4) * 256 + ((ln & 15) ^ (ln >> 4)) * 16);
     const int y = 2 * (g.y0 + rg * RPW) + 1 + r;
