@@ -42,9 +42,9 @@ const KernelFit kFit[] = {
 };
 // what is left to the configuration itself, as a factor
 const struct { const char *name; float factor; } kFactor[] = {
-    {"c4r2k16m", 0.81f}, {"c4r2k16n", 0.85f}, {"c4r2k32n", 0.80f}, {"d4r2k64", 0.88f}, {"f4r1", 0.78f}, {"f4r2", 0.76f}, {"f8r1", 0.84f},
+    {"c4r2k16m", 0.81f}, {"c4r2k16n", 0.85f}, {"c4r2k32n", 0.80f}, {"d4r2k64", 0.88f}, {"e8r1", 1.00f}, {"e8r2", 1.00f}, {"f4r1", 0.78f}, {"f4r2", 0.76f}, {"f8r1", 0.84f},
     {"g4r1", 0.57f}, {"g4r1k32", 0.58f}, {"g4r1k32n", 0.54f}, {"g4r1n", 0.55f}, {"g4r1p", 0.52f}, {"h4r2", 0.57f}, {"h4r2k32n", 0.53f},
-    {"h4r2k32p", 0.53f}, {"h4r2n", 0.53f}, {"h4r2p", 0.51f}, {"m2r1k32x1n", 0.79f}, {"m4r1k32x2", 1.01f}, {"m4r1kfx1n", 1.01f}, {"m4r1kfx2", 1.24f},
+    {"h4r2k32p", 0.53f}, {"h4r2n", 0.53f}, {"h4r2p", 0.51f}, {"l8k16", 1.00f}, {"l8k32", 1.00f}, {"m2r1k32x1n", 0.79f}, {"m4r1k32x2", 1.01f}, {"m4r1kfx1n", 1.01f}, {"m4r1kfx2", 1.24f},
     {"m4r2k32x1", 1.01f}, {"m4r2k32x1n", 1.11f}, {"m4r2k32x2", 1.09f}, {"m4r2k32x2n", 1.18f}, {"m4r2k64x2", 1.11f}, {"m4r2kfx1", 1.14f},
     {"m4r2kfx1n", 1.10f}, {"m4r4k32x1", 1.09f}, {"m8r2k32x2", 1.19f}, {"p16r1k16", 1.05f}, {"p16r1k32", 0.95f}, {"p16r2k16", 0.98f},
     {"p4r1k32", 0.93f}, {"p4r1k32n", 0.84f}, {"p4r2k32", 0.96f}, {"p4r2k32n", 0.92f}, {"p4r4k16", 0.91f}, {"p4r4k32", 0.84f}, {"p8r1k16", 0.99f},
@@ -79,7 +79,7 @@ double share_cost_us(const ConvCost &c, double ow, double oh, double bytes, unsi
   const double units = cdiv(ow, 62) * cdiv(oh + 1, 2 * rows) * slices, rounds = cdiv(cdiv(units, xcds), c.slots * slices);
   const double mfma = cap / 16 * (9 * c.rpw + 3) + cbp / 16 * 36 * c.rpw, steps = cap / c.ck + cbp / 16, tileKB = 2 * rows * 62 * c.KT * 2 / 1024;
   const double work = rounds * (1.03 * mfma * 2 * 32 / 2000 + 0.506 * steps + 0.0142 * tileKB), memory = bytes / 5.183e6;
-  return kLaunchUs + kShareStartUs + std::sqrt(work * work + memory * memory);
+  return kLaunchUs + factorOf(c.config) * (kShareStartUs + std::sqrt(work * work + memory * memory));
 }
 
 // Streaming kernels whose weights and halos go straight into LDS (conv3x3_mfma_dl.hip), one form as well: matrix instructions, LDS reads and
@@ -97,7 +97,7 @@ double streamed_lds_cost_us(const ConvCost &c, double ow, double oh, double byte
   const double stored = bytesWritten / std::max(1.0, 2 * ow * oh * c.K), tileKB = rows * 32 * c.KT * 2 / 1024 * stored; // (a pooled tile is a quarter)
   const double unit = std::sqrt(matrix * matrix + lds * lds + loads * loads) + 0.0371 * phases * c.CA / c.ck + (c.ck == 16 && !c.blockedIn ? (phases > 1 ? 0.0144 : 0.0036) * haloKB : 0) + (c.blockedOut ? 0 : 0.0141 * tileKB);
   const double memory = (bytesRead + bytesWritten) / 5.712e6;
-  return kLaunchUs + std::pow(std::pow(rounds * unit, 1.2) + std::pow(memory, 1.2), 1 / 1.2);
+  return kLaunchUs + factorOf(c.config) * std::pow(std::pow(rounds * unit, 1.2) + std::pow(memory, 1.2), 1 / 1.2);
 }
 
 } // namespace

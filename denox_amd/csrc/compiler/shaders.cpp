@@ -53,9 +53,11 @@ std::string fmtFloat(float v) {
 // w % ksplit of the 32-channel blocks and row group w / ksplit.
 // hrot: the staged halo unpadded, its 16-byte slots rotated per pixel instead (HROT in conv_common.h: 32-channel steps fit where the
 // padded form allowed 16).  swp: the matrix loop reads the next group's fragments while it issues the current group's (SWP).
-// On an upsampled source A the streaming configurations of 8 waves stand for conv3x3_upshare.hip (chooseShare below; rpw counts the edges between
-// low-resolution rows that a wave computes), on a plain source of whole steps of channels for conv3x3_mfma_dl.hip (chooseStreamedLds).
-struct ConvConfig { unsigned waves, rpw, ck; bool resident; unsigned pw; unsigned maxKT; unsigned mf, xb; const char *name; bool pp = false; bool fold = false; bool wideHalo = false; bool ntStore = false; bool ostage = false; unsigned ksplit = 1; bool hrot = false; bool swp = false; };
+// share: products of an upsampled source A shared between its outputs (conv3x3_upshare.hip, chooseShare below; rpw counts the edges between
+// low-resolution rows that a wave computes).  intoLds: weights and halos of a plain source straight into LDS (conv3x3_mfma_dl.hip, chooseStreamedLds).
+struct ConvConfig { unsigned waves, rpw, ck; bool resident; unsigned pw; unsigned maxKT; unsigned mf, xb; const char *name; bool pp = false; bool fold = false; bool wideHalo = false; bool ntStore = false; bool ostage = false; unsigned ksplit = 1; bool hrot = false; bool swp = false; bool share = false; bool intoLds = false; };
+constexpr ConvConfig sharedProducts(unsigned rpw, const char *name) { ConvConfig c{8, rpw, 16, false, 0, 0, 32, 1, name}; c.share = true; return c; }
+constexpr ConvConfig streamedIntoLds(unsigned ck, const char *name) { ConvConfig c{8, 2, ck, false, 0, 0, 32, 1, name}; c.intoLds = true; return c; }
 const ConvConfig kConvConfigs[] = {
     // weights streamed per step
     {4, 2, 16, false, 0, 0, 32, 1, "w4r2k16"}, {4, 2, 32, false, 0, 0, 32, 1, "w4r2k32"}, {4, 4, 16, false, 0, 0, 32, 1, "w4r4k16"}, {4, 4, 32, false, 0, 0, 32, 1, "w4r4k32"},
@@ -112,6 +114,10 @@ const ConvConfig kConvConfigs[] = {
     // stride 4 fits the LDS next to its weights with nothing larger
     {2, 1, 16, false, 0, 32, 32, 1, "w2r1k16n", false, false, true}, {2, 1, 32, false, 0, 16, 16, 1, "m2r1k32x1n", false, false, true},
     {2, 2, 16, false, 0, 32, 32, 1, "w2r2k16n", false, false, true},
+    // products of an upsampled source shared, two edges per wave (large images) or one; weights and halos straight into LDS, 16 or 32 channels per step.
+    // They do not replace the streaming configurations of 8 waves, which stay the faster ones where an image has few tiles (w8r2k16 and l8k16,
+    // 32 -> 64, 5 x 5 with stride 2: 10 and 21 us a launch at 480 x 270, 30 and 24 at 960 x 540).
+    sharedProducts(2, "e8r2"), sharedProducts(1, "e8r1"), streamedIntoLds(16, "l8k16"), streamedIntoLds(32, "l8k32"),
 };
 constexpr unsigned kNumConvConfigs = sizeof(kConvConfigs) / sizeof(kConvConfigs[0]);
 
@@ -328,16 +334,14 @@ struct ShareGeometry {
   unsigned CA, CB, CAP, CBP, K, KOUTP, KT, cka, slots;
 };
 
-// Whether a configuration of a layer over an upsampled source is that kernel, and its geometry.
 bool chooseShare(const ConvConfig &cfg, const Op &conv, unsigned pattern, unsigned CA, unsigned CB, const DeviceInfo &dev, ShareGeometry &g) {
-  if (cfg.resident || cfg.fold || cfg.mf != 32 || cfg.waves != 8 || cfg.rpw > 2) return false;
+  if (!cfg.share) return false;
   if (!(pattern & PAT_UPSAMPLE) || (pattern & (PAT_POOL | PAT_CROP | PAT_PADA)) || conv.R != 3 || conv.S != 3 || conv.padX != 1 || conv.padY != 1 || conv.strideX != 1 || conv.strideY != 1) return false;
   const unsigned K = conv.K;
   // whole vectors of A; B's partial last vector is read ending at its last channel; two 16-byte stores per accumulator
   if (CA % 8 || (CB > 0 && CB < 8) || K % 8) return false;
   g.CA = CA; g.CB = CB; g.CAP = (CA + 15) / 16 * 16; g.CBP = CB ? (CB + 15) / 16 * 16 : 0; g.K = K; g.KOUTP = (K + 31) / 32 * 32;
   g.cka = g.CAP % 32 ? 16 : 32;
-  if (cfg.rpw == 2 && cfg.ck != g.cka) return false;
   for (unsigned kt = std::min(g.KOUTP, cfg.maxKT ? cfg.maxKT : 64u); kt >= 32; kt -= 32) {
     const unsigned kb = kt / 32;
     if (g.KOUTP % kt || cfg.waves % kb) continue;
@@ -380,7 +384,7 @@ std::vector<uint8_t> packShareWeights(const Op &conv, const ShareGeometry &g) {
 }
 
 // ---- weights and halos straight into LDS (conv3x3_mfma_dl.hip) -------------------------------------------------------
-// The streaming configurations of 8 waves on a plain source of whole steps of channels.  A strided layer's taps fall into phases (see the
+// One plain source of whole steps of channels.  A strided layer's taps fall into phases (see the
 // kernel); where they have fewer than four taps on average a step is shorter than its barrier and its loads are worth, and the
 // kernel that takes all taps at once stays.
 struct StreamedLdsGeometry {
@@ -388,7 +392,7 @@ struct StreamedLdsGeometry {
 };
 
 bool chooseStreamedLds(const ConvConfig &cfg, const Op &conv, unsigned pattern, unsigned CA, unsigned CB, const DeviceInfo &dev, StreamedLdsGeometry &g) {
-  if (cfg.resident || cfg.fold || cfg.mf != 32 || cfg.waves != 8 || cfg.rpw != 2 || (cfg.ck != 16 && cfg.ck != 32)) return false;
+  if (!cfg.intoLds) return false;
   const unsigned R = conv.R, S = conv.S, sy = conv.strideY, sx = conv.strideX;
   if ((pattern & ~(PAT_ACT | PAT_POOL)) || CB || sy > 2 || sx > 2 || R < sy || S < sx || R * S < 4 * sy * sx) return false;
   if (CA % cfg.ck || conv.K % 8) return false;
@@ -587,10 +591,15 @@ public:
           if (!v.valid || v.pitch % 8 || v.channelOffset % 8) continue;
         }
       }
-      if (m.blocked()) {
+      if (cfg.share || cfg.intoLds) {
         ShareGeometry sg;
         StreamedLdsGeometry lg;
-        if (!offeredBlocked(cfg) && !sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg) && !streamsIntoLds(cfg, conv, model, m, CA, CB, opt.deviceInfo, lg)) continue;
+        if (cfg.waves * 64 > opt.deviceInfo.maxComputeWorkGroupInvocations) continue;
+        if (cfg.share ? sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg) : streamsIntoLds(cfg, conv, model, m, CA, CB, opt.deviceInfo, lg)) out.push_back(c);
+        continue;
+      }
+      if (m.blocked()) {
+        if (!offeredBlocked(cfg)) continue;
         // block-major sources are read through the per-step buffer resource: every LDS step must lie in one source
         if (!m.inputFormats.empty() && m.inputFormats[0] && CB && CA % stepChannels(cfg, cpad)) continue;
       }
@@ -600,32 +609,28 @@ public:
       if ((cfg.waves + cfg.pw) * 64 > opt.deviceInfo.maxComputeWorkGroupInvocations) continue;
       ConvGeometry g;
       g.R = conv.R; g.S = conv.S; g.SY = conv.strideY; g.SX = conv.strideX;
-      ShareGeometry sg;
-      StreamedLdsGeometry lg;
-      if (!sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg) && !streamsIntoLds(cfg, conv, model, m, CA, CB, opt.deviceInfo, lg) && !chooseKT(cfg, CA, CB, conv.K, opt.deviceInfo, g)) continue;
+      if (!chooseKT(cfg, CA, CB, conv.K, opt.deviceInfo, g)) continue;
       out.push_back(c);
     }
-    bool forcedFold = false; // a forced upsample-folding configuration leaves matches without an upsample to nobody: not an error
-    for (unsigned c = 0; c < kNumConvConfigs; ++c) forcedFold |= kConvConfigs[c].fold && forced == kConvConfigs[c].name;
-    if (out.empty() && !forced.empty() && !m.blocked() && !(forcedFold && !(m.pattern & PAT_UPSAMPLE)))
+    bool forcedUpsampled = false; // a forced configuration for upsampled sources leaves matches without an upsample to nobody: not an error
+    for (unsigned c = 0; c < kNumConvConfigs; ++c) forcedUpsampled |= (kConvConfigs[c].fold || kConvConfigs[c].share) && forced == kConvConfigs[c].name;
+    if (out.empty() && !forced.empty() && !m.blocked() && !(forcedUpsampled && !(m.pattern & PAT_UPSAMPLE)))
       fail(Status::Unsupported, "conv configuration '" + forced + "' is not valid for this layer");
     return out;
   }
 
+  // whether every pixel of a result inside a concat starts on a 16-byte boundary
+  static bool wholeVectors(const Model &model, const Match &m) {
+    if (!m.outputVariant) return true;
+    const ConcatView v = concatViewOf(model, m.output);
+    return v.valid && v.pitch % 8 == 0 && v.channelOffset % 8 == 0;
+  }
   static bool sharesProducts(const ConvConfig &cfg, const Op &conv, const Model &model, const Match &m, unsigned CA, unsigned CB, const DeviceInfo &dev, ShareGeometry &g) {
-    if (m.outputVariant) { // whole 16-byte stores
-      const ConcatView v = concatViewOf(model, m.output);
-      if (!v.valid || v.pitch % 8 || v.channelOffset % 8) return false;
-    }
     if (m.blocked() && !m.inputFormats.empty() && m.inputFormats[0] && CB && (CA % 16 || CB % 8)) return false;
-    return chooseShare(cfg, conv, m.pattern, CA, CB, dev, g);
+    return wholeVectors(model, m) && chooseShare(cfg, conv, m.pattern, CA, CB, dev, g);
   }
   static bool streamsIntoLds(const ConvConfig &cfg, const Op &conv, const Model &model, const Match &m, unsigned CA, unsigned CB, const DeviceInfo &dev, StreamedLdsGeometry &g) {
-    if (m.outputVariant) { // whole 16-byte stores
-      const ConcatView v = concatViewOf(model, m.output);
-      if (!v.valid || v.pitch % 8 || v.channelOffset % 8) return false;
-    }
-    return chooseStreamedLds(cfg, conv, m.pattern, CA, CB, dev, g);
+    return wholeVectors(model, m) && chooseStreamedLds(cfg, conv, m.pattern, CA, CB, dev, g);
   }
 
   size_t parameterMemorySize(const Model &model, const Match &m) const override {
@@ -646,7 +651,9 @@ public:
     FoldGeometry fg{};
     ShareGeometry sg{};
     StreamedLdsGeometry lg{};
-    const bool share = sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg), intoLds = !share && streamsIntoLds(cfg, conv, model, m, CA, CB, opt.deviceInfo, lg);
+    const bool share = cfg.share, intoLds = cfg.intoLds;
+    if ((share && !sharesProducts(cfg, conv, model, m, CA, CB, opt.deviceInfo, sg)) || (intoLds && !streamsIntoLds(cfg, conv, model, m, CA, CB, opt.deviceInfo, lg)))
+      fail(Status::Internal, "conv config rejected at implement time");
     if (intoLds) {
       g.CA = CA; g.CB = 0; g.C = g.CPAD = CA; g.K = conv.K; g.KOUTP = lg.KOUTP; g.KT = lg.KT; g.slots = lg.slots;
     } else if (share) {

@@ -16,6 +16,8 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(16, 32, 1, 1, False), (16, 8, 2, 3, True), (32, 64, 16, 32, False), (32, 48, 33, 65, True), (64, 64, 31, 31, False), (64, 96, 34, 66, True), (96, 128, 17, 97, False),
           (128, 160, 20, 40, True), (112, 112, 65, 33, False), (192, 192, 15, 70, False), (256, 64, 9, 130, False), (64, 64, 300, 420, False), (32, 96, 270, 510, True)]
 
+CONFIGS = ["l8k32", "l8k16"]  # 32 and 16 channels per step
+
 
 def blocked(x):
     H, W, C = x.shape
@@ -27,11 +29,10 @@ def planar(y):
     return y.transpose(1, 2, 0, 3).reshape(H, W, g * 8)
 
 
-def is_this_kernel(d):
-    return d["workgroup_count"][1:] == [1, 1] and "SLOTS=" in d["debug_info"] and "WAVES=8" in d["debug_info"] and "UPA=0" in d["debug_info"]
+SOURCE = "conv3x3_mfma_dl.hip"
 
 
-@pytest.mark.parametrize("config", ["w8r2k32", "w8r2k16"])
+@pytest.mark.parametrize("config", CONFIGS)
 @pytest.mark.parametrize("C,K,H,W,pooled", SHAPES)
 def test_streamed_into_lds_equals_the_definition(oracle, config, C, K, H, W, pooled):
     rng = np.random.default_rng(C + K + H)
@@ -44,23 +45,18 @@ def test_streamed_into_lds_equals_the_definition(oracle, config, C, K, H, W, poo
     x = rng.integers(-2, 3, (H, W, C)).astype(np.float16)
     want = oracle.run_graph(m.to_ops({"H": H, "W": W}), {"x": x}, "fp32")[t.name]
     assert np.abs(want).max(initial=0) < 1024  # (a leaky slope of 1/2 leaves at most one bit below 1)
-    ran = 0
     for blocked_in in (False, True):
         for blocked_out in (False, True):
             layouts = dict(input_layout=dx.Layout.CHWC8 if blocked_in else dx.Layout.HWC, output_layout=dx.Layout.CHWC8 if blocked_out else dx.Layout.HWC)
-            try:
-                blob = dx.compile_model(m, conv_config=config, assume={"H": H, "W": W}, **layouts)
-            except dx.DenoxHipError as e:
-                assert e.status == 5
+            if C % int(config[-2:]):  # whole steps of channels only
+                with pytest.raises(dx.DenoxHipError) as e:
+                    dx.compile_model(m, conv_config=config, assume={"H": H, "W": W}, **layouts)
+                assert e.value.status == 5
                 continue
-            if not any(is_this_kernel(d) for d in dx.describe(blob, H=H, W=W)["dispatches"]):
-                continue
+            blob = dx.compile_model(m, conv_config=config, assume={"H": H, "W": W}, **layouts)
+            assert [d["src_path"] for d in dx.describe(blob, H=H, W=W)["dispatches"]] == [SOURCE]
             got = dx.Module.load(blob).instance(H=H, W=W).infer(blocked(x) if blocked_in else x)[0]
             assert_bits_equal(planar(got) if blocked_out else got, want.astype(np.float16), f"{config} {layouts}")
-            ran += 1
-    if not ran:
-        assert C % int(config[-2:])  # whole steps only
-        pytest.skip("not this kernel: no whole steps of channels")
 
 
 # filter, stride, padding (y, x), C, K, H, W: phases of unequal taps, padding past the image, extents that leave a phase a row or column short
@@ -68,7 +64,7 @@ STRIDED = [((5, 5), (2, 2), (2, 2), 32, 64, 45, 131), ((5, 5), (1, 1), (2, 2), 1
            ((3, 7), (1, 2), (5, 2), 32, 96, 18, 140), ((2, 2), (1, 1), (0, 0), 48, 128, 33, 33), ((5, 5), (2, 2), (0, 4), 64, 48, 5, 40)]
 
 
-@pytest.mark.parametrize("config", ["w8r2k32", "w8r2k16"])
+@pytest.mark.parametrize("config", CONFIGS)
 @pytest.mark.parametrize("filt,stride,pad,C,K,H,W", STRIDED)
 def test_strides_and_filters(oracle, config, filt, stride, pad, C, K, H, W):
     rng = np.random.default_rng(sum(filt) + C + K)
@@ -80,14 +76,13 @@ def test_strides_and_filters(oracle, config, filt, stride, pad, C, K, H, W):
     assert np.abs(want).max(initial=0) < 2048
     for blocked_in in (False, True):
         layout = dx.Layout.CHWC8 if blocked_in else dx.Layout.HWC
-        try:
-            blob = dx.compile_model(m, conv_config=config, assume={"H": H, "W": W}, input_layout=layout)
-        except dx.DenoxHipError as e:
-            assert e.status == 5 and C % int(config[-2:])
-            pytest.skip("not this kernel: no whole steps of channels")
-        if not any(is_this_kernel(d) for d in dx.describe(blob, H=H, W=W)["dispatches"]):
-            assert C % int(config[-2:])
-            pytest.skip("not this kernel: no whole steps of channels")
+        if C % int(config[-2:]):  # whole steps of channels only
+            with pytest.raises(dx.DenoxHipError) as e:
+                dx.compile_model(m, conv_config=config, assume={"H": H, "W": W}, input_layout=layout)
+            assert e.value.status == 5
+            continue
+        blob = dx.compile_model(m, conv_config=config, assume={"H": H, "W": W}, input_layout=layout)
+        assert [d["src_path"] for d in dx.describe(blob, H=H, W=W)["dispatches"]] == [SOURCE]
         assert_bits_equal(dx.Module.load(blob).instance(H=H, W=W).infer(blocked(x) if blocked_in else x)[0], want.astype(np.float16), f"{config} {layout}")
 
 
@@ -102,7 +97,7 @@ def test_result_inside_a_concat(oracle):
     m.output(t, "out")
     v = rng.integers(-2, 3, (H, W, 32)).astype(np.float16)
     want = oracle.run_graph(m.to_ops({"H": H, "W": W}), {"x": v}, "fp32")[t.name]
-    for config in ("w8r2k32", "w8r2k16"):
+    for config in CONFIGS:
         blob = dx.compile_model(m, conv_config=config, assume={"H": H, "W": W})
-        assert sum(is_this_kernel(d) for d in dx.describe(blob, H=H, W=W)["dispatches"]) == 2
+        assert [d["src_path"] for d in dx.describe(blob, H=H, W=W)["dispatches"]] == [SOURCE] * 2
         assert_bits_equal(dx.Module.load(blob).instance(H=H, W=W).infer(v)[0], want.astype(np.float16), config)

@@ -140,8 +140,10 @@ def test_every_conv_configuration_has_a_live_parity_case():
     every configuration compiles for at least one shape of the test that covers it -- none is tested by skips alone."""
     import test_gpu_conv_pair as tp
     import test_gpu_layers as tl
+    import test_gpu_streamed_lds as ts
+    import test_gpu_upshare as tu
     from util import he_weights, small_bias
-    listed = set(tl.ALL_CONFIGS) | set(tl.FOLD_CONFIGS) | set(tl.STRIDED_ONLY_CONFIGS) | set(tp.PAIR_CONFIGS)
+    listed = set(tl.ALL_CONFIGS) | set(tl.FOLD_CONFIGS) | set(tl.STRIDED_ONLY_CONFIGS) | set(tp.PAIR_CONFIGS) | set(ts.CONFIGS) | set(tu.CONFIGS)
     assert listed == set(dx.conv_config_names()), listed ^ set(dx.conv_config_names())
     rng = np.random.default_rng(0)
 
@@ -168,6 +170,8 @@ def test_every_conv_configuration_has_a_live_parity_case():
 
     dead = [c for c in tl.ALL_CONFIGS if not any(compiles(plain(C, K), c) for C, K, _, _ in tl.EVERY_CONFIG_SHAPES)]
     dead += [c for c in tl.FOLD_CONFIGS if not any(compiles(folded(CA, CB, K), c) for CA, CB, K, _, _, _ in tl.FOLD_SHAPES)]
+    dead += [c for c in ts.CONFIGS if not any(compiles(plain(C, K), c) for C, K, _, _, _ in ts.SHAPES)]
+    dead += [c for c in tu.CONFIGS if not all(compiles(folded(CA, CB, K), c) for CA, CB, K, _, _, _ in tu.BOTH)]
     dead += [c for c in tl.STRIDED_ONLY_CONFIGS if not any(compiles(plain(24, 40, stride, pad, R, S), c) for R, S, pad, stride in tl.GEOMETRY_CASES)]
     for c in tp.PAIR_CONFIGS:
         hit = False
@@ -177,6 +181,28 @@ def test_every_conv_configuration_has_a_live_parity_case():
         if not hit:
             dead.append(c)
     assert not dead, dead
+
+
+def test_a_configuration_name_stands_for_one_kernel():
+    """Timing tables, forced configurations and the table of estimates go by name: the streaming configurations of 8 waves stay the
+    register-streamed kernel on the layers that the kernels loading straight into LDS take as well, and those have names of their own."""
+    from util import he_weights
+    rng = np.random.default_rng(0)
+
+    def sources(config, upsampled, R=3, stride=1):
+        m = dx.Model()
+        x = m.upsample(m.input("x", m.sym("W") // 2, m.sym("H") // 2, 32)) if upsampled else m.input("x", "W", "H", 32)
+        m.output(m.relu(m.conv2d(x, he_weights(rng, 64, 32, R, R), np.zeros(64, np.float16), stride=(stride, stride), padding=(R // 2, R // 2))))
+        blob = dx.compile_model(m, conv_config=config, assume={"H": 64, "W": 64})
+        return [d["src_path"] for d in dx.describe(blob, H=64, W=64)["dispatches"] if "conv" in d["name"]]
+
+    for config in ("w8r2k32", "w8r2k16", "w8r1k16"):
+        assert sources(config, True) == sources(config, False) == ["conv3x3_mfma.hip"], config
+    assert sources("w8r2k16", False, 5, 2) == sources("w8r1k16", False, 5, 2) == ["conv3x3_mfma.hip"]
+    for config in ("e8r2", "e8r1"):
+        assert sources(config, True) == ["conv3x3_upshare.hip"], config
+    for config in ("l8k32", "l8k16"):
+        assert sources(config, False) == sources(config, False, 5, 2) == ["conv3x3_mfma_dl.hip"], config
 
 
 def test_missing_kernel_is_reported():
