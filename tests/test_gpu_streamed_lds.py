@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 import denox_amd as dx
-from util import assert_bits_equal
+from util import assert_bits_equal, integer_conv_on_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -84,6 +84,46 @@ def test_strides_and_filters(oracle, config, filt, stride, pad, C, K, H, W):
         blob = dx.compile_model(m, conv_config=config, assume={"H": H, "W": W}, input_layout=layout)
         assert [d["src_path"] for d in dx.describe(blob, H=H, W=W)["dispatches"]] == [SOURCE]
         assert_bits_equal(dx.Module.load(blob).instance(H=H, W=W).infer(blocked(x) if blocked_in else x)[0], want.astype(np.float16), f"{config} {layout}")
+
+
+# filter, stride, padding, C, K, H, W, pooled, layouts of source and result: two and more units for every workgroup (256 of them), with results kept for
+# the next unit's steps (one step, several, several phases) and stored at once (128 channels), several slices, a pooled result
+MANY_UNITS = [
+    ("l8k32", (3, 3), (1, 1), (1, 1), 64, 64, 544, 960, False, False, False), ("l8k32", (3, 3), (1, 1), (1, 1), 32, 32, 600, 1000, False, False, True),
+    ("l8k32", (3, 3), (1, 1), (1, 1), 96, 128, 545, 963, True, True, True), ("l8k16", (3, 3), (1, 1), (1, 1), 64, 64, 1088, 960, False, True, True),
+    ("l8k16", (3, 3), (1, 1), (1, 1), 48, 96, 700, 1000, True, False, False), ("l8k16", (3, 3), (1, 1), (1, 1), 128, 160, 270, 480, False, True, False),
+    ("l8k32", (5, 5), (2, 2), (2, 2), 32, 64, 1080, 1920, False, False, False), ("l8k16", (5, 5), (2, 2), (2, 2), 48, 128, 1080, 1920, False, True, True),
+    ("l8k32", (4, 4), (2, 2), (1, 1), 64, 96, 1001, 1441, False, True, False), ("l8k16", (7, 3), (2, 1), (3, 0), 16, 64, 1203, 901, False, False, True),
+    ("l8k16", (7, 7), (1, 1), (3, 3), 32, 64, 270, 520, False, False, False),
+]
+
+
+@pytest.mark.parametrize("config,filt,stride,pad,C,K,H,W,pooled,blocked_in,blocked_out", MANY_UNITS)
+def test_many_units_per_workgroup(config, filt, stride, pad, C, K, H, W, pooled, blocked_in, blocked_out):
+    """What only a second unit of work reaches: halo offsets moved from the last phase of one unit to the first of the next, stores of a
+    finished tile during the next one's steps, the parity of the two LDS buffers.  Twice: the same bits."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(C + H)
+    w, b = rng.choice([-1, 0, 0, 0, 1], (K, C) + filt).astype(np.float16), rng.integers(-3, 4, K).astype(np.float16)
+    m = dx.Model()
+    t = m.relu(m.conv2d(m.input("x", "W", "H", C), w, b, stride=stride, padding=pad))
+    m.output(m.pool(t) if pooled else t, "out")
+    blob = dx.compile_model(m, conv_config=config, assume={"H": H, "W": W}, input_layout=dx.Layout.CHWC8 if blocked_in else dx.Layout.HWC,
+                            output_layout=dx.Layout.CHWC8 if blocked_out else dx.Layout.HWC)
+    d, = dx.describe(blob, H=H, W=W)["dispatches"]
+    info = dict(kv.split("=") for kv in d["debug_info"].split(" | ")[1].split())
+    x = rng.integers(-2, 3, (H, W, C)).astype(np.float16)
+    want = torch.relu(integer_conv_on_gpu(x, w, b, stride, pad))
+    oh, ow = want.shape[:2]
+    assert d["src_path"] == SOURCE and -(-ow // 32) * -(-oh // (8 * int(info["RPW"]))) * (-(-K // 32) * 32 // int(info["KT"])) >= 2 * d["workgroup_count"][0]
+    assert float(want.max()) < 2048
+    if pooled:
+        want = want[:oh // 2 * 2, :ow // 2 * 2].reshape(oh // 2, 2, ow // 2, 2, K).amax((1, 3))
+    want = want.half().cpu().numpy()
+    inst = dx.Module.load(blob).instance(H=H, W=W)
+    for _ in range(2):
+        got = inst.infer(blocked(x) if blocked_in else x)[0]
+        assert_bits_equal(planar(got) if blocked_out else got, want, config)
 
 
 def test_result_inside_a_concat(oracle):

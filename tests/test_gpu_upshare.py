@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 import denox_amd as dx
-from util import assert_bits_equal
+from util import assert_bits_equal, integer_conv_on_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -71,6 +71,43 @@ def test_shared_products_equal_the_definition(oracle, config, CA, CB, K, H, W, p
             xs = [feeds[k] for k in ("lo", "x") if k in feeds]
             got = dx.Module.load(blob).instance(H=H, W=W).infer(*[blocked(x) if blocked_in else x for x in xs])[0]
             assert_bits_equal(planar(got) if blocked_out else got, want.astype(np.float16), f"{config} {layouts}")
+
+
+# CA, CB, K, H, W, padded, layouts of sources and result: two and more units for every workgroup (256 of them), among them units inside the image one
+# after the other, the last ones of an XCD, a result above 192 MiB (stored past the cache) and units of several slices
+MANY_UNITS = [
+    ("e8r2", 64, 9, 64, 1088, 1920, True, False, False), ("e8r2", 64, 16, 64, 1088, 1920, False, True, True), ("e8r2", 48, 16, 64, 500, 1000, False, True, False),
+    ("e8r2", 64, 0, 64, 500, 1002, False, False, True), ("e8r2", 128, 9, 128, 300, 960, True, False, False), ("e8r2", 32, 24, 64, 542, 960, False, False, True),
+    ("e8r1", 64, 9, 64, 542, 960, True, False, False), ("e8r1", 96, 32, 64, 400, 1000, False, True, True), ("e8r1", 112, 48, 96, 400, 480, False, False, True),
+]
+
+
+@pytest.mark.parametrize("config,CA,CB,K,H,W,padded,blocked_in,blocked_out", MANY_UNITS)
+def test_many_units_per_workgroup(config, CA, CB, K, H, W, padded, blocked_in, blocked_out):
+    """What only a second unit of work reaches: halo offsets moved from one unit to the next, its first step loaded while the last one's result
+    is on its way out, the parity of the two LDS buffers.  Twice: the same bits."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(CA + H)
+    m, t, feeds = layer(CA, CB, K, H, W, padded, rng)
+    blob = dx.compile_model(m, conv_config=config, assume={"H": H, "W": W}, input_layout=dx.Layout.CHWC8 if blocked_in else dx.Layout.HWC,
+                            output_layout=dx.Layout.CHWC8 if blocked_out else dx.Layout.HWC)
+    d, = dx.describe(blob, H=H, W=W)["dispatches"]
+    info = dict(kv.split("=") for kv in d["debug_info"].split(" | ")[1].split())
+    rows = 2 * (8 // (int(info["KT"]) // 32)) * int(info["RPW"])
+    assert d["src_path"] == "conv3x3_upshare.hip" and -(-W // 62) * -(-(H + 1) // rows) * (-(-K // 32) * 32 // int(info["KT"])) >= 2 * d["workgroup_count"][0]
+    x = np.zeros((H, W, CA + CB), np.float16)
+    x[:, :, :CA] = feeds["lo"].repeat(2, 0).repeat(2, 1)
+    if CB:
+        x[:, :, CA:] = np.pad(feeds["x"], ((1, 2), (2, 3), (0, 0)), "edge") if padded else feeds["x"]
+    conv, = [op for op in m.to_ops({"H": H, "W": W}) if "weight" in op]
+    want = torch.relu(integer_conv_on_gpu(x, conv["weight"], conv["bias"]))
+    assert float(want.max()) < 2048
+    want = want.half().cpu().numpy()
+    inst = dx.Module.load(blob).instance(H=H, W=W)
+    xs = [feeds[k] for k in ("lo", "x") if k in feeds]
+    for _ in range(2):
+        got = inst.infer(*[blocked(v) if blocked_in else v for v in xs])[0]
+        assert_bits_equal(planar(got) if blocked_out else got, want, config)
 
 
 @pytest.mark.parametrize("config", CONFIGS)

@@ -64,3 +64,21 @@ def fill_lds_with_nans():
         m.output(m.conv2d(m.input("x", "W", "H", 64), np.full((64, 64, 3, 3), nan, np.float16), np.full(64, nan, np.float16)))
         _poison = (dx.Module.compile(m, conv_config="s8r2k16").instance(H=256, W=512), np.full((256, 512, 64), nan, np.float16))
     _poison[0].infer(_poison[1])
+
+
+def integer_conv_on_gpu(x, w, b, stride=(1, 1), pad=(1, 1)):
+    """The convolution of an H x W x C image of small integers with K x C x R x S weights, one product of matrices per tap in binary32 on the
+    GPU: exact while every partial sum stays below 2^24, whatever order the library adds in.  For images too large for the oracle."""
+    import torch
+    x, w = torch.as_tensor(x, dtype=torch.float32, device="cuda"), torch.as_tensor(w, dtype=torch.float32, device="cuda")
+    H, W, C = x.shape
+    K, _, R, S = w.shape
+    padded = torch.zeros((H + 2 * pad[0], W + 2 * pad[1], C), device="cuda")
+    padded[pad[0]:pad[0] + H, pad[1]:pad[1] + W] = x
+    oh, ow = (H + 2 * pad[0] - R) // stride[0] + 1, (W + 2 * pad[1] - S) // stride[1] + 1
+    out = torch.as_tensor(b, dtype=torch.float32, device="cuda").repeat(oh * ow, 1)
+    for r in range(R):
+        for s in range(S):
+            tap = padded[r:r + (oh - 1) * stride[0] + 1:stride[0], s:s + (ow - 1) * stride[1] + 1:stride[1]]
+            out += tap.reshape(oh * ow, C).contiguous() @ w[:, :, r, s].t().contiguous()
+    return out.reshape(oh, ow, K)
