@@ -407,11 +407,13 @@ def measure(args, workload: str, steps: int, warmup: int, brief: bool):
             roofline["non_conv_frac_of_hbm"] = non_conv["frac_of_hbm"]
             roofline["non_conv_source"] = "unfused second schedule (the timed schedule has no bandwidth-only dispatch)"
 
+    # (the library launches lists of up to four dispatches one by one, and any list under DENOX_HIP_NO_GRAPH)
+    launched = "in one hipGraph" if mod.runtime_model.dispatch_count > 4 and "DENOX_HIP_NO_GRAPH" not in os.environ else "as plain launches"
     line = {
         "metric": "oidn_unet_fp16_hwc_1080p_throughput" if workload == "oidn_1080p" else f"{workload}_throughput", "value": H * W / (ms * 1e-3) * 1e-6, "unit": "Mpix/s",
         "n_gpus": 1, "steps": steps, "warmup": warmup, "ms_per_step": ms, "higher_is_better": True, "scaling": "weak",
         "vs_baseline": None, "dtype": "f16", "data": "synthetic",
-        "config": {"workload": f"{description}; {mod.runtime_model.dispatch_count} dispatches {'in one hipGraph' if mod.runtime_model.dispatch_count > 4 else 'as plain launches'}", "device_bytes": inst.device_bytes,
+        "config": {"workload": f"{description}; {mod.runtime_model.dispatch_count} dispatches {launched}", "device_bytes": inst.device_bytes,
                    "schedule": "min-cost over measured dispatch latencies" if db is not None else "min-cost over roofline estimates",
                    "tuning_seconds": round(tune_s, 2), "host_pointer_path_ms_per_frame": round(host_ms, 3), "host_pointer_pipelined_ms_per_frame": round(pipelined_ms, 3),
                    "two_frames_in_flight_ms_per_frame": round(two_ms, 4) if two_ms else None,
