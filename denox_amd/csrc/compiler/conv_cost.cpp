@@ -69,10 +69,12 @@ double cdiv(double a, double b) { return std::ceil(a / b); }
 // Kernels that share the products of an upsampled source (conv3x3_upshare.hip), one form for all of its configurations: a workgroup's units of
 // work one after the other -- the matrix instructions of the two waves of a SIMD at 2 GHz, 0.5 us per step (its barrier, the first
 // fragments behind it, loads that arrive late), the result's way out -- against the launch's memory traffic.  Fitted to 614 launches
-// of 12 layers (32 to 224 upsampled, 0 to 128 other channels, 16 to 224 outputs) at 96 x 64 to 1920 x 1088 in all layouts: measured over
-// estimated 0.89 - 1.16 for nine of ten, median 1.00.
-// (Its long straight-line code starts from cold instruction caches in a frame, which launches back to back do not show: 64 + 9 -> 64 at
-// 256 x 192 takes 12.6 us inside the U-Net, 11.0 without this.)
+// of 12 layers (32 to 224 upsampled, 0 to 128 other channels, 16 to 224 outputs) at 96 x 64 to 1920 x 1088 in all layouts, back to back: measured
+// over estimated, without the start, 0.89 - 1.16 for nine of ten, median 1.00.
+// The start is what a frame adds to a launch that the same kernel did not precede (64 + 9 -> 64 at 256 x 192: 12.6 us inside the U-Net, 11.0
+// back to back).  Whole frames of 37 networks and extents (the U-Net and twice its width at 96 x 96 to 1920 x 1080, the small U-Net), schedules by
+// estimates with starts of 0 to 2.2: 1.2 to 2.0 choose the same but for two frames (1 % either way), without one the frames at 512 x 512
+// and 640 x 360 are 2 % slower, with 2.2 the one at 1280 x 720.
 constexpr double kShareStartUs = 1.6;
 double share_cost_us(const ConvCost &c, double ow, double oh, double bytes, unsigned xcds) {
   const double cap = cdiv(c.CA, 16) * 16, cbp = cdiv(c.CB, 16) * 16, rows = c.waves / (c.KT / 32) * c.rpw, slices = cdiv(cdiv(c.K, 32) * 32, c.KT);
@@ -87,6 +89,10 @@ double share_cost_us(const ConvCost &c, double ow, double oh, double bytes, unsi
 // pixel-major source's lines more than once.  Fitted to 1632 launches of 15 layers (16 to 256 channels, with and without a pool) at
 // 96 x 64 to 1920 x 1088 in all layouts: measured over estimated 0.88 - 1.14 for nine of ten, median 1.00.  (5 x 5 with stride 2, 32 and 64 -> 64 channels at
 // 480 x 270 to 1920 x 1080: 0.92 - 1.27; the price of short pieces is four times as high there, every pixel lies in a phase of its own.)
+// The figures are back to back and without the start, which is fitted as above: with none the small U-Net takes the kernel for 16 -> 32 channels
+// and is slower than without it (760 x 448: 44.5 us a frame against 43.3, 960 x 540: 49.8 and 48.8), with 0.5 it does not, and seven frames
+// of the U-Nets gain 0.1 - 2 % (one loses 0.7); 0.3 leaves half of that, 0.8 and more lose in three.
+constexpr double kStreamedLdsStartUs = 0.5;
 double streamed_lds_cost_us(const ConvCost &c, double ow, double oh, double bytesRead, double bytesWritten, unsigned xcds) {
   const double kb = c.KT / 32, rows = 8.0 * c.rpw, slices = cdiv(cdiv(c.K, 32) * 32, c.KT), groups = c.CA / 16.0;
   const double rounds = cdiv(cdiv(cdiv(ow, 32) * cdiv(oh, rows) * slices, xcds), c.slots * slices);
@@ -97,7 +103,7 @@ double streamed_lds_cost_us(const ConvCost &c, double ow, double oh, double byte
   const double stored = bytesWritten / std::max(1.0, 2 * ow * oh * c.K), tileKB = rows * 32 * c.KT * 2 / 1024 * stored; // (a pooled tile is a quarter)
   const double unit = std::sqrt(matrix * matrix + lds * lds + loads * loads) + 0.0371 * phases * c.CA / c.ck + (c.ck == 16 && !c.blockedIn ? (phases > 1 ? 0.0144 : 0.0036) * haloKB : 0) + (c.blockedOut ? 0 : 0.0141 * tileKB);
   const double memory = (bytesRead + bytesWritten) / 5.712e6;
-  return kLaunchUs + factorOf(c.config) * std::pow(std::pow(rounds * unit, 1.2) + std::pow(memory, 1.2), 1 / 1.2);
+  return kLaunchUs + factorOf(c.config) * (kStreamedLdsStartUs + std::pow(std::pow(rounds * unit, 1.2) + std::pow(memory, 1.2), 1 / 1.2));
 }
 
 } // namespace

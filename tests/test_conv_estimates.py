@@ -73,6 +73,17 @@ def test_estimates_per_configuration_whatever_is_fused():
     assert len(forced) == 12 and inner(forced) <= 1.02 * inner(default)
 
 
+@pytest.mark.parametrize("net,H,W,layout,taken", [
+    ("tiny_unet", 448, 760, "HWC", []), ("tiny_unet", 540, 960, "HWC", []), ("tiny_unet", 532, 1680, "CHW", []), ("tiny_unet", 720, 1280, "HWC", []),  # 16 -> 32 channels
+    ("oidn_unet", 187, 251, "HWC", []), ("oidn_unet", 512, 512, "HWC", ["e8r1"]), ("oidn_unet", 1080, 1920, "HWC", ["e8r1", "e8r2", "l8k16", "l8k32"])])
+def test_kernels_that_load_into_lds_are_taken_where_they_pay(net, H, W, layout, taken):
+    """A launch starts colder inside a frame than behind itself, which the estimates are fitted to.  Measured frames with and without these
+    kernels: the small U-Net is up to 3 % slower with them, the U-Net 1 % slower at 187 x 251 and faster at the larger extents."""
+    lay = dx.Layout[layout]
+    dx.compile_model(networks.build(net)[0], assume={"H": H, "W": W}, input_layout=lay, output_layout=lay)
+    assert sorted({c for c in configs() if c[0] in "el"}) == taken
+
+
 @pytest.mark.parametrize("config", ["x4r2k16", "x8r2k16", "v4r2k64", "y4r2k32", "d4r2k64"])
 @pytest.mark.parametrize("H,W", [(16, 30), (64, 64), (300, 61), (1080, 1920)])
 def test_forced_pair_is_taken_on_any_extent(config, H, W):
