@@ -579,9 +579,9 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
 #pragma unroll
     for (int r = 0; r < OUT_ROWS; ++r) finish_row(g, r, out_acc(r, 0), out_acc(r, 1));
 #endif
+    STEP_WAIT(NSTORES); // the next unit's first step has landed (before the end too: no wave leaves loads into LDS behind); the stores may still be on their way
     if (!more)
       break;
-    STEP_WAIT(NSTORES); // the next unit's first step has landed; the stores may still be on their way
     DNX_SYNC();
     buf ^= 1;
     unit = next;
