@@ -29,20 +29,16 @@
 // 128: 78, so those suit block-major sources (121 and 65).
 //
 // Launch: persistent, NXCD * NKT * SLOTS workgroups; a unit of work is (tile, slice of KT output channels), each XCD has a contiguous band.
-#include "conv_common.h"
+#include "conv_into_lds.h"
 
 #ifndef KERNEL_NAME
 #define KERNEL_NAME conv3x3_mfma_dl
-#endif
-#ifndef NXCD
-#define NXCD 8
 #endif
 static_assert(CB == 0 && !UPA && !PADA && !CROP && MF == 32 && PW == 0 && SY <= 2 && SX <= 2, "one plain source, strides up to 2");
 static_assert(KR >= SY && KS >= SX, "a tap in every phase");
 static_assert(CA % CK == 0 && (CK == 16 || CK == 32 || CK == 64), "whole steps of a power of two of vectors");
 static_assert(KOUT % 8 == 0 && OPITCH % 8 == 0 && OVEC, "two 16-byte stores per pixel and block: the wait for a step's loads counts them");
 
-#define NKT (KOUTP / KT)
 // phase a of n taps with padding p and stride s: taps r = PH_FIRST, PH_FIRST + s, ...; the first one's offset d = (r - p - a) / s
 #define PH_FIRST(a, p, s) ((((a) + (p)) % (s)))
 #define PH_TAPS(a, n, p, s) (((n) - PH_FIRST(a, p, s) + (s) - 1) / (s))
@@ -82,10 +78,9 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
 
   const int tilesX = ((int)CONV_OUT_W(pc) + TW - 1) / TW, tilesY = ((int)CONV_OUT_H(pc) + TH - 1) / TH;
   const int units = tilesX * tilesY * NKT;
-  const int perXcd = (units + NXCD - 1) / NXCD;
-  const int first = (int)(DNX_BID_X % NXCD) * perXcd;
-  const int last = first + perXcd < units ? first + perXcd : units;
-  int unit = first + (int)(DNX_BID_X / NXCD);
+  const UnitBand band = unit_band(units);
+  const int last = band.last;
+  int unit = band.unit;
   if (unit >= last)
     return; // uniform for the workgroup
   const bool rev = (pc.FLAGS & 1u) != 0;
@@ -105,12 +100,7 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
   for (int i = tid; i < KOUTP; i += NT) sBias[i] = (float)BIAS[i];
 #endif
 
-  // What follows from the lane's number alone is derived again where it is needed rather than kept in registers.
-  auto fresh_lane = [&]() {
-    int l = lane;
-    __asm__ volatile("" : "+v"(l));
-    return l;
-  };
+  auto fresh_lane = [&]() { return fresh_lane_of(lane); };
   // Byte offsets of this lane's halo vectors in the source at channel 0, for one unit and phase; NO_LOAD outside the image (reads as
   // zero).  From one to the next they move by the same amount where both halos lie inside the image.
   unsigned hoff[NVH];
@@ -156,16 +146,8 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_void_t *)(sBuf + buf * BUF_SLOTS + f * 64), 16, fresh_lane() * 16, (kt * (NTAPS * KB * (CA / 16)) + first_frag(ph, k) + f) * 1024, 0, 0);
     }
   };
-#define STEP_WAIT(n) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
 
   Acc acc;
-  // Holds a step's matrix instructions in front of its barrier (they touch no memory: the compiler may collect several steps' worth behind it).
-  auto pin = [&]() {
-#pragma unroll
-    for (int b = 0; b < KB; ++b)
-#pragma unroll
-      for (int j = 0; j < RPW; ++j) __asm__ volatile("" : "+v"(acc.v[b][j]));
-  };
   auto step = [&](int buf, const int ph, auto load) { // load(i): item i of the loads for the next step
     typedef __attribute__((address_space(3))) const char lds_char_t;
     typedef __attribute__((address_space(3))) const half8 *lds_frag;
@@ -214,7 +196,10 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
         for (int j = 0; j < RPW; ++j) acc.v[b][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[u % WR][b], px[gr & 1][j + r], acc.v[b][j], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
-    pin();
+#pragma unroll
+    for (int b = 0; b < KB; ++b)
+#pragma unroll
+      for (int j = 0; j < RPW; ++j) pin(acc.v[b][j]);
   };
 
   int buf = 0;

@@ -29,19 +29,15 @@
 //
 // Launch: persistent, NXCD * NKT * SLOTS workgroups; a unit of work is (tile, slice of KT output channels), each XCD has a contiguous band.
 // Definitions: as conv_common.h (UPA = 1), plus CKA and SLOTS.
-#include "conv_common.h"
+#include "conv_into_lds.h"
 
 #ifndef KERNEL_NAME
 #define KERNEL_NAME conv3x3_upshare
-#endif
-#ifndef NXCD
-#define NXCD 8
 #endif
 static_assert(UPA == 1 && MF == 32 && !POOL && !CROP && !PADA && KR == 3 && KS == 3 && PY == 1 && PX == 1 && SY == 1 && SX == 1 && PW == 0, "upsampled source A, plain 3 x 3");
 static_assert(CA % 8 == 0 && (CB == 0 || CB >= 8), "whole vectors of A; B with at least one");
 static_assert(KOUT % 8 == 0 && OPITCH % 8 == 0 && OVEC, "two 16-byte stores per accumulator: the wait for a step's loads counts them");
 
-#define NKT (KOUTP / KT)
 #define RG (WAVES / KB)
 static_assert(KOUTP % KT == 0 && WAVES % KB == 0, "whole slices and row groups");
 #define CAP ((CA + 15) / 16 * 16)
@@ -114,10 +110,9 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
   const int WL = (int)(pc.IN_W >> 1), HL = (int)(pc.IN_H >> 1);
   const int tilesX = (WL + 30) / 31, tilesY = (2 * HL + OUT_ROWS * RG) / (OUT_ROWS * RG); // the first output row of the first tile is row -1
   const int units = HL > 0 ? tilesX * tilesY * NKT : 0;
-  const int perXcd = (units + NXCD - 1) / NXCD;
-  const int first = (int)(DNX_BID_X % NXCD) * perXcd;
-  const int last = first + perXcd < units ? first + perXcd : units;
-  int unit = first + (int)(DNX_BID_X / NXCD);
+  const UnitBand band = unit_band(units);
+  const int last = band.last;
+  int unit = band.unit;
   if (unit >= last)
     return; // uniform for the workgroup
   const bool rev = (pc.FLAGS & 1u) != 0;
@@ -138,13 +133,7 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
 #endif
 
   // ---- loads of a step into a buffer ----
-  // What follows from the lane's number alone is derived again where it is needed: kept from unit to unit (the compiler moves it out of
-  // the loop), slots, rows and columns of all vectors take 30 registers that the accumulators need.
-  auto fresh_lane = [&]() {
-    int l = lane;
-    __asm__ volatile("" : "+v"(l));
-    return l;
-  };
+  auto fresh_lane = [&]() { return fresh_lane_of(lane); };
   // A step's loads are items, a wave's share of one load instruction per 64 slots each, which the matrix loops issue one by one between their
   // instructions: a memory instruction waits for room in the memory pipeline, and all of a step's in front of its matrix work left
   // the matrix cores idle for that time.  No branch: a wave without an item left repeats the last one (the same bytes to the same place).
@@ -292,8 +281,6 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
 #endif
   };
 #endif
-  // every load into LDS of this wave has arrived; `n`: memory instructions issued since (they complete in issue order)
-#define STEP_WAIT(n) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
 
   // ---- matrix work ----
   float16v mm[RPW + 1], me[RPW + 1], em[RPW], ee[RPW];
@@ -358,9 +345,6 @@ extern "C" __global__ DNX_LAUNCH_BOUNDS(NT) void KERNEL_NAME(
     }
   };
 
-  // Holds a step's matrix instructions in front of its barrier: they touch no memory, and in a block without branches the compiler
-  // otherwise collects several steps' worth behind it, their operands in scratch memory meanwhile.
-  auto pin = [](float16v &v) { __asm__ volatile("" : "+v"(v)); };
   auto pin_a = [&]() {
 #pragma unroll
     for (int t = 0; t <= RPW; ++t) {
