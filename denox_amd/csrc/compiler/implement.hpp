@@ -189,7 +189,6 @@ public:
   virtual std::vector<Match> matchAll(const Model &model, const CompileOptions &opt) const = 0;
   // configuration ids valid for a match
   virtual std::vector<unsigned> acceptMatch(const Model &model, const Match &m, const CompileOptions &opt) const = 0;
-  virtual size_t parameterMemorySize(const Model &, const Match &) const { return 0; }
   virtual float speedup(unsigned /*config*/) const { return 1.0f; }
   virtual void implement(OpImpl &impl, const Model &model, const Match &m, unsigned config, SymGraph &sym, const CompileOptions &opt) const = 0;
 };

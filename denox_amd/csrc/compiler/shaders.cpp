@@ -38,10 +38,10 @@ std::string fmtFloat(float v) {
 }
 
 // ------------------------------------------------------------------ conv
-// Two kernel sources share one configuration table: conv3x3_mfma.hip streams the
+// Six kernel sources share one configuration table: conv3x3_mfma.hip streams the
 // weight slice of every reduction step through LDS (any layer size), conv3x3_mfma_ws.hip
-// keeps the whole slice resident and runs persistently (layers whose weights fit LDS).
-// waves: computing waves; pw: extra staging-only waves (wave specialisation, resident kernel only)
+// keeps the whole slice resident and runs persistently (layers whose weights fit LDS); fold, share and intoLds
+// below name the other four.
 // waves: computing waves; rpw: image rows per wave; ck: input channels per LDS step (0 = all, 1 = half);
 // resident: weights stay in LDS (persistent launch); pw: extra staging-only waves; maxKT: cap on output channels
 // per workgroup (0 = none); mf: matrix shape 32 (32x32x16) or 16 (16x16x32); xb: 16-pixel blocks per row (mf 16).
@@ -633,12 +633,6 @@ public:
     return wholeVectors(model, m) && chooseStreamedLds(cfg, conv, m.pattern, CA, CB, dev, g);
   }
 
-  size_t parameterMemorySize(const Model &model, const Match &m) const override {
-    const Op &conv = opOf(model, m, OpKind::Conv);
-    const unsigned C = conv.C, cpad = (C + 31) / 32 * 32, kp = (conv.K + 31) / 32 * 32; // upper bound over configurations
-    return static_cast<size_t>(kp) * conv.R * conv.S * cpad * 2 + static_cast<size_t>(kp) * 2;
-  }
-
   void implement(OpImpl &impl, const Model &model, const Match &m, unsigned config, SymGraph &sym, const CompileOptions &opt) const override {
     const ConvConfig &cfg = kConvConfigs[config];
     const Op &conv = opOf(model, m, OpKind::Conv);
@@ -957,12 +951,6 @@ public:
       out.push_back(c);
     }
     return out;
-  }
-
-  size_t parameterMemorySize(const Model &model, const Match &m) const override {
-    const auto [first, second] = convsOf(model, m);
-    return static_cast<size_t>(9 * 32) * ((first->C + 15) / 16 * 16 + 32) * 2 + 4 * 32;
-    (void)second;
   }
 
   void implement(OpImpl &impl, const Model &model, const Match &m, unsigned config, SymGraph &sym, const CompileOptions &opt) const override {
