@@ -96,7 +96,7 @@ static double selection_cost(const SuperGraphEdge &e, double cost, bool measured
     const bool forced = opt.forceConvConfig == d.convCost.config;
     // The upsample-folding kernels multiply sums of weights that are rounded to binary16 once more (the 1920 x 1080 U-Net's output is 1.34e-3
     // from binary64 with them, 1.22e-3 without): callers take that on with a timing table or by name, an estimate does not
-    // decide it for them, although it costs them time (592 us; 517 with folded kernels).
+    // decide it for them, although it costs them a little time (500 us; 492 with a table that takes folded kernels).
     if ((k == ConvKernel::Fold || k == ConvKernel::FoldStaged) && !forced) cost += unmeasuredFoldMs;
     // A forced conv -> conv configuration is taken wherever it exists: single convolutions keep their choice beside it (a forced
     // single one is the only one offered), and on extents that do not suit it two of them may be estimated faster.

@@ -1,7 +1,8 @@
 // Why an estimate per configuration: a bytes-and-FLOP bound is the same for every configuration of a layer, so a schedule
 // without a timing table used one configuration (the first of the table) for every layer.  A frame of the 1920 x 1080 U-Net took
-// 690 us so, 592 with these estimates and 578 with a measured table (none of them with folded weights); at 251 x 187 185, 96 and 95; with
-// doubled widths at 1917 x 1077 2530, 2037 and 2000.
+// 690 us so, 592 with estimates and 578 with a measured table (none of them with folded weights); at 251 x 187 185, 96 and 95; with
+// doubled widths at 1917 x 1077 2530, 2037 and 2000.  With the kernels that load straight into LDS, estimates and table: 496 and 510, 96 and 94,
+// 1390 and 1375 (denox_amd/conv_estimates.py).
 //
 // The form is the kernels' own: what the busiest compute unit does -- matrix instructions, halo staging and its memory round
 // trips, weight slices, stores -- against what the whole launch moves through memory; the parts that overlap combine as the root of
@@ -10,8 +11,8 @@
 // candidate of the U-Net at eight extents from 180 x 108 to 3840 x 2160 and at two widths, of the small U-Net, and of 16 single
 // convolutions (1 x 1 to 5 x 5, stride 1 and 2, 3 to 256 channels) at five extents.  denox_amd/conv_estimates.py measures how far
 // they are from a GPU, per configuration, and what a changed or new kernel's entry in kFactor should be.  On layers that are not among
-// those of the fit the measured time is 1.08 times the estimate in the median, 0.99 - 1.19 for half of the candidates; the schedules picked are
-// 1 - 7 percent slower than measured ones.  A timing table, where there is one, still decides.
+// those of the fit the measured time is 1.07 times the estimate in the median, 0.99 - 1.18 for half of the candidates; the schedules picked take
+// 0.97 - 1.07 times as long as measured ones.  A timing table, where there is one, still decides.
 #include "conv_cost.hpp"
 #include <algorithm>
 #include <cmath>
