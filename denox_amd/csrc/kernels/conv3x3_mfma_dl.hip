@@ -1,4 +1,5 @@
-// conv3x3_mfma_dl.hip -- convolution of one plain source with weights and halos streamed straight into LDS.
+// conv3x3_mfma_dl.hip -- convolution of one plain source with weights and halos streamed straight into LDS (any filter with a tap in
+// every phase, as the other kernels whose name says 3x3).
 //
 // The streaming kernel (conv3x3_mfma.hip) loads a step's weights and halo into registers, writes them to LDS and lets every wave wait at
 // two barriers per step.  Here both go from memory into one of two LDS buffers (buffer_load ... lds) while the other is
@@ -16,14 +17,14 @@
 // 1920 x 1088: 257 us, 215 with neither loads nor stores, 800 MB of memory traffic are 156).  Tiles of 32 rows (RPW = 4, two blocks) halve the
 // LDS reads per matrix instruction of tiles of 16, which need steps of 16 channels to fit; those fetch a pixel-major source's lines
 // twice or more, so the large tiles pay on block-major sources (128 -> 64 257 us, pixel-major 313 and with 32-channel steps 277).
-// Microseconds a launch, the best of the other kernels before, block-major or pixel-major source: 96 -> 96 at 960 x 544 95 and 74,
-// 192 -> 192 at 480 x 272 86 and 70, 64 -> 96 pooled at 960 x 544 64 and 50, 128 -> 128 at 960 x 544 151 and 123, 128 -> 64 at 1920 x 1088 310 and 257.
+// (These are back to back.)  Microseconds a launch inside frames of the U-Nets by estimates, the other kernels before: 96 -> 96 at 480 x 272 27 and 23,
+// 192 -> 192 there 79 and 68, 64 -> 96 pooled at 960 x 544 62 and 51, 128 -> 128 there 159 and 126, 128 -> 64 at 1920 x 1088 330 and 236.
 //
 // Strides.  Tap r of output row y reads input row y SY + r - PY = (y + d) SY + a: the taps fall into SY phases a, each of which is a
 // convolution of stride 1 over every SY-th row with consecutive offsets d (columns alike).  A step is one phase and CK channels: its
 // halo is staged as an image of its own, so a strided layer's matrix loop is that of a plain one -- consecutive lanes read consecutive
 // slots, a pixel fragment serves all of its rows -- where the other kernels read every SY-th pixel of one large halo.  5 x 5, stride 2:
-// phases of 9, 6, 6 and 4 taps.  Microseconds, resident weights and one large halo before: 32 -> 64 at 1920 x 1080, pixel-major, 86 to 93
+// phases of 9, 6, 6 and 4 taps.  Microseconds a launch, back to back, resident weights and one large halo before: 32 -> 64 at 1920 x 1080, pixel-major, 86 to 93
 // and 65 to 76 (dense signed values in buffers that take turns: 91 and 81; a card at its power limit: 93 both), first pass on new buffers
 // 126 and 105; 64 -> 64 at 960 x 544 (weights that do not stay in LDS): 38.  Of a 16-channel step each phase fetches 32 bytes of every
 // 128: 78, so those suit block-major sources (121 and 65).

@@ -23,9 +23,10 @@
 // bank groups.  One barrier per step.  A source whose channels are not whole vectors goes through registers.
 //
 // What bounds it: the LDS-fed matrix rate and, beside it, loads and stores that overlap it only in part.  64 + 9 -> 64 channels at
-// 1920 x 1088: 71 us with neither, 82 with stores, 90 with loads, 105 - 112 with both (memory alone: 371 MB, 73).  Microseconds a launch, the
-// best of the other exact kernels before: that layer 173 and 108, 96 + 32 -> 64 at 960 x 544 70 and 45, 112 + 48 -> 96 at 480 x 272 39 and
-// 25, 128 + 9 -> 128 at 1920 x 1088 618 and 262.  Four waves to a workgroup (one per SIMD) are slower on every layer measured.
+// 1920 x 1088: 71 us with neither, 82 with stores, 90 with loads, 105 - 112 with both (memory alone: 371 MB, 73).  Microseconds a launch inside
+// frames of the U-Nets by estimates, the other exact kernels before: that layer 160 and 109, 96 + 32 -> 64 at 960 x 544 80 and 50, 112 + 48 -> 96 at 480 x 272
+// 39 and 35, 192 + 64 -> 128 at 960 x 544 259 and 143, 128 + 9 -> 128 at 1920 x 1088 619 and 273.  Back to back, caches warm, small
+// images take less: 112 + 48 -> 96 25, 96 + 32 -> 64 45.  Four waves to a workgroup (one per SIMD) are slower on every layer measured.
 //
 // Launch: persistent, NXCD * NKT * SLOTS workgroups; a unit of work is (tile, slice of KT output channels), each XCD has a contiguous band.
 // Definitions: as conv_common.h (UPA = 1), plus CKA and SLOTS.
